@@ -408,12 +408,45 @@ __global__ void k_to(int n, const double *__restrict__ a, T *__restrict__ b) {
 // sweep from 4.7 to 4.1 TB/s).
 constexpr bool kStreamLevel = false;
 
-// sum_j anb_ij x'_j over the slots of row i, spread over LPR consecutive
-// lanes and combined with shuffles; x' = x + alpha*xc[parent] when PRO
-template <int LPR, class T, bool PRO>
+// The prolongation of a level's correction into the next finer level: the
+// kernel that forms a coarse cell's value adds alpha times it to the cell's
+// members (x[mem[q]], q in [mptr[p], mptr[p+1])).  Every finer cell belongs to
+// one coarse cell, so no two threads touch one value, and the sum is that of
+// a pass of its own (k_prolong) without that pass's launch (3.4 us, 28 of them
+// in the channel's F-cycle), and without the parent lookup of every neighbour
+// that forming it in the finer level's first sweep took (finest level of 128^3
+// hexahedra: 28.8 us instead of 16.9).  Not on the large levels in sliced
+// ELL, whose lanes would each walk a list of their own: 342k cells with 2.0M
+// members took 35 us, the plain sweep and k_prolong take 13 and 8.
+template <class T> struct Scatter {
+  const int *mptr, *mem; // members of the level's cells in the next finer level
+  T *x;                  // the finer level's iterate
+  T alpha;
+};
+
+// members lane, lane + step, ... of cell p, loads of a batch first
+template <class T> __device__ __forceinline__ void scatter_cell(const Scatter<T> &sc, int p, T v, int lane, int step) {
+  const int q1 = sc.mptr[p + 1];
+  const T add = sc.alpha * v;
+  constexpr int B = 4;
+  for (int q = sc.mptr[p] + lane; q < q1; q += B * step) {
+    int id[B];
+    T xv[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) id[u] = sc.mem[min(q + u * step, q1 - 1)];
+#pragma unroll
+    for (int u = 0; u < B; ++u) xv[u] = sc.x[id[u]];
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (q + u * step < q1) sc.x[id[u]] = xv[u] + add;
+  }
+}
+
+// sum_j anb_ij x_j over the slots of row i, spread over LPR consecutive
+// lanes and combined with shuffles
+template <int LPR, class T>
 __device__ __forceinline__ T row_offdiag(int i, int lane, int n, int w, EllNbr nbr,
-                                         const T *__restrict__ anb, const T *x, const int *__restrict__ parent,
-                                         const T *__restrict__ xc, T alpha) {
+                                         const T *__restrict__ anb, const T *x) {
   T s = T(0);
   if (LPR == 1) {
     // one lane per row: the row's slots in batches (loads first, then the
@@ -424,10 +457,8 @@ __device__ __forceinline__ T row_offdiag(int i, int lane, int n, int w, EllNbr n
       ell_batch<kEllBatch, kStreamLevel>(nbr, i, n, w, j0, k);
 #pragma unroll
       for (int u = 0; u < kEllBatch; ++u) {
-        const int kk = k[u] >= 0 ? k[u] : i;
         a[u] = ld_mat<kStreamLevel>(&anb[(size_t)min(j0 + u, w - 1) * n + i]);
-        xv[u] = x[kk];
-        if (PRO) xv[u] = xv[u] + alpha * xc[parent[kk]];
+        xv[u] = x[k[u] >= 0 ? k[u] : i];
       }
 #pragma unroll
       for (int u = 0; u < kEllBatch; ++u)
@@ -437,34 +468,26 @@ __device__ __forceinline__ T row_offdiag(int i, int lane, int n, int w, EllNbr n
   }
   for (int j = lane; j < w; j += LPR) {
     const int k = nbr.i32[(size_t)j * n + i];
-    if (k >= 0) {
-      T xk = x[k];
-      if (PRO) xk = xk + alpha * xc[parent[k]];
-      s += anb[(size_t)j * n + i] * xk;
-    }
+    if (k >= 0) s += anb[(size_t)j * n + i] * x[k];
   }
 #pragma unroll
   for (int off = LPR / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, LPR);
   return s;
 }
 
-// One damped-Jacobi sweep xn = x' + omega*(b - A x')/ac, x' = x (PRO false)
-// or x + alpha*xc[parent] (PRO true: the prolongation of the coarse
-// correction fused into the first post-smoothing sweep).  TO = double writes
-// the FP64 result of the cycle directly.
-template <int LPR, class T, class TO, bool PRO>
+// One damped-Jacobi sweep xn = x + omega*(b - A x)/ac of the finest level.
+// TO = double writes the FP64 result of the cycle directly.
+template <int LPR, class T, class TO>
 __global__ void __launch_bounds__(kBlock)
 k_sweep(int n, int w, EllNbr nbr, const T *__restrict__ ac, const T *__restrict__ anb,
-        const T *__restrict__ b, const T *x, const int *__restrict__ parent, const T *__restrict__ xc,
-        T alpha, T omega, TO *xn, const int *__restrict__ flags) {
+        const T *__restrict__ b, const T *x, T omega, TO *xn, const int *__restrict__ flags) {
   if (flags && flags[0]) return;
   const int t = xcd_block() * kBlock + threadIdx.x;
   const int i = t / LPR, lane = t % LPR;
   const bool ok = i < n;
-  const T s = row_offdiag<LPR, T, PRO>(ok ? i : 0, lane, ok ? n : 1, ok ? w : 0, nbr, anb, x, parent, xc, alpha);
+  const T s = row_offdiag<LPR, T>(ok ? i : 0, lane, ok ? n : 1, ok ? w : 0, nbr, anb, x);
   if (ok && lane == 0) {
-    T xi = x[i];
-    if (PRO) xi = xi + alpha * xc[parent[i]];
+    const T xi = x[i];
     xn[i] = (TO)(xi + omega * (b[i] - ac[i] * xi - s) / ac[i]);
   }
 }
@@ -478,45 +501,39 @@ k_resid(int n, int w, EllNbr nbr, const T *__restrict__ ac, const T *__restrict_
   const int t = xcd_block() * kBlock + threadIdx.x;
   const int i = t / LPR, lane = t % LPR;
   const bool ok = i < n;
-  const T s = row_offdiag<LPR, T, false>(ok ? i : 0, lane, ok ? n : 1, ok ? w : 0, nbr, anb, x, nullptr,
-                                         nullptr, T(0));
+  const T s = row_offdiag<LPR, T>(ok ? i : 0, lane, ok ? n : 1, ok ? w : 0, nbr, anb, x);
   if (ok && lane == 0) r[i] = b[i] - ac[i] * x[i] - s;
 }
 
 // ---- coarse levels in row-major CSR (no padding; a row's entries are
 // contiguous, so the LPR lanes of a row read one segment)
-template <int LPR, class T, bool PRO>
+template <int LPR, class T, class V>
 __device__ __forceinline__ T csr_offdiag(int i, int lane, const int *__restrict__ rp, const int *__restrict__ col,
-                                         const T *__restrict__ val, const T *x, const int *__restrict__ parent,
-                                         const T *__restrict__ xc, T alpha, bool ok) {
+                                         const V *__restrict__ val, const T *x, bool ok) {
   T s = T(0);
   if (ok)
-    for (int q = rp[i] + lane; q < rp[i + 1]; q += LPR) {
-      const int k = col[q];
-      T xk = x[k];
-      if (PRO) xk = xk + alpha * xc[parent[k]];
-      s += val[q] * xk;
-    }
+    for (int q = rp[i] + lane; q < rp[i + 1]; q += LPR) s += val[q] * x[col[q]];
 #pragma unroll
   for (int off = LPR / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, LPR);
   return s;
 }
 
-template <int LPR, class T, class TO, bool PRO>
+// SC: the level's last sweep, which also prolongates its result
+template <int LPR, class T, bool SC>
 __global__ void __launch_bounds__(kBlock)
 k_sweep_csr(int n, const int *__restrict__ rp, const int *__restrict__ col, const T *__restrict__ val,
-            const T *__restrict__ ac, const T *__restrict__ b, const T *x, const int *__restrict__ parent,
-            const T *__restrict__ xc, T alpha, T omega, TO *xn, const int *__restrict__ flags) {
+            const T *__restrict__ ac, const T *__restrict__ b, const T *x, T omega, T *xn, Scatter<T> sc,
+            const int *__restrict__ flags) {
   if (flags && flags[0]) return;
   const int t = xcd_block() * kBlock + threadIdx.x;
   const int i = t / LPR, lane = t % LPR;
   const bool ok = i < n;
-  const T s = csr_offdiag<LPR, T, PRO>(ok ? i : 0, lane, rp, col, val, x, parent, xc, alpha, ok);
-  if (ok && lane == 0) {
-    T xi = x[i];
-    if (PRO) xi = xi + alpha * xc[parent[i]];
-    xn[i] = (TO)(xi + omega * (b[i] - ac[i] * xi - s) / ac[i]);
-  }
+  const T s = csr_offdiag<LPR, T>(ok ? i : 0, lane, rp, col, val, x, ok);
+  if (!ok) return;
+  const T xi = x[i];
+  const T v = xi + omega * (b[i] - ac[i] * xi - s) / ac[i]; // the same on the row's lanes
+  if (lane == 0) xn[i] = v;
+  if (SC) scatter_cell<T>(sc, i, v, lane, LPR);
 }
 
 // ---- large coarse levels in sliced ELL: slices of 64 rows (one wavefront),
@@ -526,10 +543,9 @@ k_sweep_csr(int n, const int *__restrict__ rp, const int *__restrict__ col, cons
 // itself.  row[] maps a slot to its row (-1: past the end); rows are sorted by
 // length within windows of 256 rows so that a slice's rows have similar
 // lengths.  Each lane sums its row's entries in CSR order.
-template <class T, bool PRO>
+template <class T>
 __device__ __forceinline__ T sell_offdiag(int slot, int lane, const int *__restrict__ ptr, const int *__restrict__ col,
-                                          const T *__restrict__ val, const T *x, const int *__restrict__ parent,
-                                          const T *__restrict__ xc, T alpha) {
+                                          const T *__restrict__ val, const T *x) {
   const int sl = slot >> 6, q0 = ptr[sl] + lane, len = (ptr[sl + 1] - ptr[sl]) >> 6;
   constexpr int B = 4; // entries per batch: columns first, then values and gathers
   T s = T(0);
@@ -542,7 +558,6 @@ __device__ __forceinline__ T sell_offdiag(int slot, int lane, const int *__restr
     for (int u = 0; u < B; ++u) {
       v[u] = val[q0 + (min(k0 + u, len - 1) << 6)];
       xv[u] = x[c[u]];
-      if (PRO) xv[u] = xv[u] + alpha * xc[parent[c[u]]];
     }
 #pragma unroll
     for (int u = 0; u < B; ++u)
@@ -551,21 +566,19 @@ __device__ __forceinline__ T sell_offdiag(int slot, int lane, const int *__restr
   return s;
 }
 
-template <class T, class TO, bool PRO>
+template <class T>
 __global__ void __launch_bounds__(kBlock)
 k_sweep_sell(int nslots, const int *__restrict__ ptr, const int *__restrict__ row, const int *__restrict__ col,
-             const T *__restrict__ val, const T *__restrict__ ac, const T *__restrict__ b, const T *x,
-             const int *__restrict__ parent, const T *__restrict__ xc, T alpha, T omega, TO *xn,
+             const T *__restrict__ val, const T *__restrict__ ac, const T *__restrict__ b, const T *x, T omega, T *xn,
              const int *__restrict__ flags) {
   if (flags && flags[0]) return;
   const int t = xcd_block() * kBlock + threadIdx.x;
   if (t >= nslots) return;
   const int i = row[t];
   if (i < 0) return;
-  const T s = sell_offdiag<T, PRO>(t, t & 63, ptr, col, val, x, parent, xc, alpha);
-  T xi = x[i];
-  if (PRO) xi = xi + alpha * xc[parent[i]];
-  xn[i] = (TO)(xi + omega * (b[i] - ac[i] * xi - s) / ac[i]);
+  const T s = sell_offdiag<T>(t, t & 63, ptr, col, val, x);
+  const T xi = x[i];
+  xn[i] = xi + omega * (b[i] - ac[i] * xi - s) / ac[i];
 }
 
 // r = b - A x on a sliced-ELL level
@@ -579,7 +592,7 @@ k_resid_sell(int nslots, const int *__restrict__ ptr, const int *__restrict__ ro
   if (t >= nslots) return;
   const int i = row[t];
   if (i < 0) return;
-  const T s = sell_offdiag<T, false>(t, t & 63, ptr, col, val, x, nullptr, nullptr, T(0));
+  const T s = sell_offdiag<T>(t, t & 63, ptr, col, val, x);
   r[i] = b[i] - ac[i] * x[i] - s;
 }
 
@@ -608,7 +621,7 @@ k_resid_restrict_csr(int nc, const int *__restrict__ mptr, const int *__restrict
   T sum = T(0);
   for (int q = q0 + grp; q < q1; q += MPR) { // the same trip count on the LPR lanes of a group
     const int i = mem[q];
-    const T s = csr_offdiag<LPR, T, false>(i, lane, rp, col, val, x, nullptr, nullptr, T(0), true);
+    const T s = csr_offdiag<LPR, T>(i, lane, rp, col, val, x, true);
     sum = sum + (b[i] - ac[i] * x[i] - s);
   }
 #pragma unroll
@@ -761,160 +774,233 @@ __global__ void k_add2(int n, double *__restrict__ x, const double *__restrict__
 }
 
 // ------------------------------------------------------------ small levels
-// Every level from the first one below the tail threshold down to the
-// coarsest runs in ONE workgroup in one launch, with the levels' operators
-// held in LDS.  A byte image of the tail is kept in device memory: the static
-// part (CSR columns, row pointers, parents, aggregate members as uint16) is
-// written at setup, the coefficients (ac and the CSR values in the
-// hierarchy's precision) are packed after each Galerkin update, and the
-// coarsest level's FP64 inverse is written there too.  The kernel copies the
-// image into LDS with 16-byte loads, runs restriction, smoothing, the
-// coarsest solve and the prolongations between workgroup barriers, and
-// writes the top tail level's correction back to device memory.
-constexpr int kTailThreads = 1024;
-constexpr int kTailMaxLev = 8;
-constexpr int kTailDirectMax = 64; // coarsest levels up to this size are solved directly
+// The cycle below the first small level is one fixed linear map x = C b (it
+// starts every level from zero and never tests anything), so it is formed
+// once per operator as a dense matrix and applied as a matrix-vector product.
+// Column j is the cycle's answer to the j-th unit vector: k_dense_level forms
+// all columns of a level from the level's sparse operator and the dense map of
+// the level below it.  A product is bound by one round of loads (1190 cells in
+// FP32: 5.7 MB, spread over the chip) and takes 5 us
+// (1939 cells 7 us), where one workgroup
+// that walked the levels in LDS took 13-25 us per visit, 8 to 30 visits per
+// Krylov iteration; forming the maps takes 60-150 us per operator.
+constexpr int kDirectMax = 64;               // coarsest levels up to this size are solved directly
+constexpr size_t kDenseBytes = 16u << 20;    // largest map: 2048 cells in FP32, 1448 in FP64 (the L2s hold 32 MB)
+constexpr int kDenseThreads = 512;
+constexpr int kDenseRows = 8;                // rows of a product's workgroup
 
-struct TailLvl {
-  int n, nnz, lpr;
-  int o_ac, o_val, o_col, o_rp, o_par, o_mp, o_mem; // byte offsets of the image sections
-  int o_x, o_t, o_r, o_b;                           // byte offsets of the LDS-only vectors
-};
-struct TailDesc {
-  int nlev, img_bytes, lds_bytes, direct, o_g;
-  TailLvl L[kTailMaxLev];
-};
+inline int dense_max(size_t tsz) { return tsz == 4 ? 2048 : 1448; }
+static_assert((size_t)2048 * 2048 * 4 <= kDenseBytes && (size_t)1448 * 1448 * 8 <= kDenseBytes, "dense map size");
 
-// one pass over the rows of a tail level: out = b - A x (jac false) or
-// x + omega*(b - A x)/ac (jac true); lpr lanes per row, all threads take part
-template <class T>
-__device__ __forceinline__ void tail_pass(unsigned char *lds, const TailLvl &L, const T *x, T *out, T omega, bool jac) {
-  const T *ac = (const T *)(lds + L.o_ac), *val = (const T *)(lds + L.o_val), *b = (const T *)(lds + L.o_b);
-  const unsigned short *col = (const unsigned short *)(lds + L.o_col);
-  const unsigned short *rp = (const unsigned short *)(lds + L.o_rp);
-  const int lpr = L.lpr, lane = threadIdx.x % lpr, rows = blockDim.x / lpr;
-  for (int base = 0; base < L.n; base += rows) {
-    const int i = base + threadIdx.x / lpr;
-    T s = T(0);
-    if (i < L.n)
-      for (int q = rp[i] + lane; q < rp[i + 1]; q += lpr) s += val[q] * x[col[q]];
-    for (int off = lpr / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, lpr);
-    if (i < L.n && lane == 0) {
-      const T r = b[i] - ac[i] * x[i] - s;
-      out[i] = jac ? x[i] + omega * r / ac[i] : r;
-    }
-  }
+// A map is stored in strips of kDenseRows rows, each strip column by column,
+// so that a strip is one contiguous run of memory: entry (i, j) of an n x n map.
+__host__ __device__ __forceinline__ size_t dense_at(int i, int j, int n) {
+  return ((size_t)(i / kDenseRows) * n + j) * kDenseRows + i % kDenseRows;
 }
+// values of a map of n cells (the last strip is padded)
+inline size_t dense_size(int n) { return (size_t)((n + kDenseRows - 1) / kDenseRows) * kDenseRows * n; }
 
-// damped-Jacobi sweeps on a tail level; the result ends in x
-template <class T> __device__ __forceinline__ void tail_smooth(unsigned char *lds, const TailLvl &L, int sweeps, bool zero, T omega) {
-  T *x = (T *)(lds + L.o_x), *t = (T *)(lds + L.o_t);
-  const T *ac = (const T *)(lds + L.o_ac), *b = (const T *)(lds + L.o_b);
-  int sw = 0;
-  if (zero) {
-    for (int i = threadIdx.x; i < L.n; i += blockDim.x) x[i] = sweeps > 0 ? omega * b[i] / ac[i] : T(0);
-    __syncthreads();
-    sw = 1;
-  }
-  T *src = x, *dst = t;
-  for (; sw < sweeps; ++sw) {
-    tail_pass<T>(lds, L, src, dst, omega, true);
-    __syncthreads();
-    T *tmp = src;
-    src = dst;
-    dst = tmp;
-  }
-  if (src != x) {
-    for (int i = threadIdx.x; i < L.n; i += blockDim.x) x[i] = src[i];
-    __syncthreads();
-  }
-}
+// 16 bytes of T: the columns a workgroup of k_dense_level forms together, the
+// rows a lane of k_dense_apply loads at once
+template <class T> struct Vec16 {
+  static constexpr int K = 16 / sizeof(T);
+  typedef T V __attribute__((ext_vector_type(16 / sizeof(T))));
+};
 
-template <class T>
-__global__ void __launch_bounds__(kTailThreads)
-k_tail(const TailDesc *__restrict__ d, const unsigned char *__restrict__ img, const T *__restrict__ b_top,
-       T *__restrict__ x_top, int pre, int post, int coarse, T omega, T alpha, const int *__restrict__ flags) {
-  if (flags && flags[0]) return;
+// The map of a level, K columns per workgroup: `pre` damped-Jacobi sweeps from
+// zero on the unit vectors, the restricted residual through the map Cc of the
+// next level (nc cells), alpha times the result prolongated, `post` sweeps.
+// Cc null: the sweeps alone (a coarsest level too large for the direct solve).
+// The vectors live in LDS, K to a 16-byte element, and the level's rows come
+// from L2 once per pass for all K (the pass is bound by those reads: one
+// FP64 column a workgroup took 314 us for 1939 cells, 4 FP32 columns 100).  After one
+// sweep from zero the residual reaches only the aggregates next to the unit's
+// cell, so the coarse map is applied to the nonzero entries alone.
+template <class T, class TC>
+__global__ void __launch_bounds__(kDenseThreads)
+k_dense_level(int n, int w, const int *__restrict__ nbr, const T *__restrict__ anb,
+              const T *__restrict__ ac, const int *__restrict__ parent, int nc, const int *__restrict__ mptr,
+              const int *__restrict__ mem, const TC *__restrict__ Cc, int pre, int post, T omega, T alpha,
+              T *__restrict__ C) {
+  constexpr int K = Vec16<T>::K;
+  typedef typename Vec16<T>::V V;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int nlev = d->nlev;
-  {
-    const uint4 *src = (const uint4 *)img;
-    uint4 *dst = (uint4 *)lds;
-    const int nv = d->img_bytes / 16;
-    for (int i = threadIdx.x; i < nv; i += blockDim.x) dst[i] = src[i];
-    const TailLvl &L = d->L[0];
-    T *b = (T *)(lds + L.o_b);
-    for (int i = threadIdx.x; i < L.n; i += blockDim.x) b[i] = b_top[i];
+  V *x = (V *)lds, *y = x + n, *rc = y + n;
+  int *list = (int *)(rc + nc);
+  __shared__ int s_cnt;
+  const int j0 = blockIdx.x * K;
+  auto unit = [&](int i) {
+    V e;
+#pragma unroll
+    for (int k = 0; k < K; ++k) e[k] = i == j0 + k ? T(1) : T(0);
+    return e;
+  };
+  // y = x + omega (e - A x)/ac, or the residual e - A x; one row a lane, its
+  // slots in batches
+  auto pass = [&](bool jac) {
+    constexpr int B = 8;
+    for (int i = threadIdx.x; i < n; i += kDenseThreads) {
+      V sum = T(0);
+      for (int s0 = 0; s0 < w; s0 += B) {
+        int k[B];
+        T a[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+          const size_t at = (size_t)min(s0 + u, w - 1) * n + i;
+          k[u] = nbr[at];
+          a[u] = anb[at];
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+          if (s0 + u < w && k[u] >= 0) sum = sum + a[u] * x[k[u]];
+      }
+      const T a = ac[i];
+      const V r = unit(i) - a * x[i] - sum;
+      y[i] = jac ? x[i] + omega * r / a : r;
+    }
+    __syncthreads();
+    if (jac) {
+      V *t = x;
+      x = y;
+      y = t;
+    }
+  };
+  for (int i = threadIdx.x; i < n; i += kDenseThreads) {
+    V v = T(0);
+    if (pre > 0) v = omega * unit(i) / ac[i];
+    x[i] = v;
   }
   __syncthreads();
-  for (int l = 0; l + 1 < nlev; ++l) {
-    const TailLvl &L = d->L[l];
-    tail_smooth<T>(lds, L, pre, true, omega);
-    tail_pass<T>(lds, L, (const T *)(lds + L.o_x), (T *)(lds + L.o_r), omega, false);
-    __syncthreads();
-    const TailLvl &C = d->L[l + 1];
-    const T *r = (const T *)(lds + L.o_r);
-    T *bc = (T *)(lds + C.o_b);
-    const unsigned short *mp = (const unsigned short *)(lds + C.o_mp);
-    const unsigned short *mem = (const unsigned short *)(lds + C.o_mem);
-    for (int p = threadIdx.x; p < C.n; p += blockDim.x) {
-      T s = T(0);
-      for (int q = mp[p]; q < mp[p + 1]; ++q) s = s + r[mem[q]];
-      bc[p] = s;
+  for (int k = 1; k < pre; ++k) pass(true);
+  if (Cc) {
+    pass(false);
+    for (int p = threadIdx.x; p < nc; p += kDenseThreads) {
+      V s = T(0);
+      for (int q = mptr[p]; q < mptr[p + 1]; ++q) s = s + y[mem[q]];
+      rc[p] = s;
     }
     __syncthreads();
-  }
-  const TailLvl &Lc = d->L[nlev - 1];
-  if (d->direct) {
-    // coarsest level: x = G b with the FP64 (pseudo-)inverse G
-    const double *G = (const double *)(lds + d->o_g);
-    const T *b = (const T *)(lds + Lc.o_b);
-    T *x = (T *)(lds + Lc.o_x);
-    for (int i = threadIdx.x; i < Lc.n; i += blockDim.x) {
-      double s = 0.0;
-      for (int j = 0; j < Lc.n; ++j) s += G[(size_t)i * Lc.n + j] * (double)b[j];
-      x[i] = (T)s;
+    if (threadIdx.x < 64) { // the entries nonzero for any column, in order
+      int cnt = 0;
+      for (int p0 = 0; p0 < nc; p0 += 64) {
+        const int p = p0 + (int)threadIdx.x;
+        bool nz = false;
+        if (p < nc)
+#pragma unroll
+          for (int k = 0; k < K; ++k) nz = nz || rc[p][k] != T(0);
+        const unsigned long long m = __ballot(nz);
+        if (nz) list[cnt + __popcll(m & ((1ull << threadIdx.x) - 1ull))] = p;
+        cnt += __popcll(m);
+      }
+      if (threadIdx.x == 0) s_cnt = cnt;
     }
     __syncthreads();
-  } else {
-    tail_smooth<T>(lds, Lc, coarse, true, omega);
-  }
-  for (int l = nlev - 2; l >= 0; --l) {
-    const TailLvl &L = d->L[l];
-    T *x = (T *)(lds + L.o_x);
-    const T *xc = (const T *)(lds + d->L[l + 1].o_x);
-    const unsigned short *par = (const unsigned short *)(lds + L.o_par);
-    for (int i = threadIdx.x; i < L.n; i += blockDim.x) x[i] = x[i] + alpha * xc[par[i]];
+    const int cnt = s_cnt;
+    for (int p = threadIdx.x; p < nc; p += kDenseThreads) {
+      TC s[K];
+#pragma unroll
+      for (int k = 0; k < K; ++k) s[k] = TC(0);
+      for (int q = 0; q < cnt; ++q) {
+        const TC c = Cc[dense_at(p, list[q], nc)];
+        const V r = rc[list[q]];
+#pragma unroll
+        for (int k = 0; k < K; ++k) s[k] += c * (TC)r[k];
+      }
+      V o;
+#pragma unroll
+      for (int k = 0; k < K; ++k) o[k] = (T)s[k];
+      y[p] = o; // the residuals are summed: y is free
+    }
     __syncthreads();
-    tail_smooth<T>(lds, L, post, false, omega);
+    for (int i = threadIdx.x; i < n; i += kDenseThreads) x[i] = x[i] + alpha * y[parent[i]];
+    __syncthreads();
+    for (int k = 0; k < post; ++k) pass(true);
   }
-  const TailLvl &L0 = d->L[0];
-  const T *x0 = (const T *)(lds + L0.o_x);
-  for (int i = threadIdx.x; i < L0.n; i += blockDim.x) x_top[i] = x0[i];
+  // K columns of one row are K kDenseRows values: lanes run over a strip's
+  // rows first
+  const int values = (n + kDenseRows - 1) / kDenseRows * kDenseRows * K;
+  for (int t = threadIdx.x; t < values; t += kDenseThreads) {
+    const int i = t / (kDenseRows * K) * kDenseRows + t % kDenseRows, k = t / kDenseRows % K;
+    if (i < n && j0 + k < n) C[dense_at(i, j0 + k, n)] = x[i][k];
+  }
 }
 
-// coefficients of one tail level into its image sections (after Galerkin)
-template <class T>
-__global__ void k_tail_pack(int n, int nnz, const double *__restrict__ ac, const double *__restrict__ anb,
-                            const int *__restrict__ lin, T *__restrict__ img_ac, T *__restrict__ img_val) {
-  const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t < n) img_ac[t] = (T)ac[t];
-  if (t < nnz) img_val[t] = (T)anb[lin[t]];
+// x = C b (ACC: x += C b), the products and sums in FP64, and with SC the
+// prolongation of x.  A workgroup owns a strip of kDenseRows rows, whose
+// entries its threads load 16 bytes at a time in address order, all of a
+// thread's loads before the first product; the partial sums are combined in a
+// fixed order.
+template <class T, bool ACC, bool SC>
+__global__ void __launch_bounds__(kDenseThreads)
+k_dense_apply(int n, const T *__restrict__ C, const T *__restrict__ b, T *__restrict__ x,
+              const int *__restrict__ parent, Scatter<T> sc, const int *__restrict__ flags) {
+  constexpr int K = Vec16<T>::K, LPC = kDenseRows / K, W = kDenseThreads / 64, B = 8; // lanes per column
+  typedef typename Vec16<T>::V V;
+  __shared__ double part[W][kDenseRows];
+  __shared__ T xs[kDenseRows];
+  const int i0 = blockIdx.x * kDenseRows, cnt = n * LPC; // 16-byte elements of the strip
+  const V *strip = (const V *)(C + (size_t)i0 * n);
+  const int done = flags ? flags[0] : 0; // beside the other loads, tested before the stores
+  double acc[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) acc[k] = 0.0;
+  for (int e0 = threadIdx.x; e0 < cnt; e0 += B * kDenseThreads) {
+    V c[B];
+    T v[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int e = min(e0 + u * kDenseThreads, cnt - 1);
+      c[u] = strip[e];
+      v[u] = b[e / LPC];
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (e0 + u * kDenseThreads < cnt)
+#pragma unroll
+        for (int k = 0; k < K; ++k) acc[k] += (double)c[u][k] * (double)v[u];
+  }
+  if (done) return;
+  const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+  for (int off = LPC; off < 64; off <<= 1)
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] += __shfl_xor(acc[k], off, 64);
+  if (lane < LPC)
+#pragma unroll
+    for (int k = 0; k < K; ++k) part[wid][lane * K + k] = acc[k];
+  __syncthreads();
+  const int r = i0 + (int)threadIdx.x;
+  if (threadIdx.x < kDenseRows && r < n) {
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < W; ++k) s += part[k][threadIdx.x];
+    const T v = ACC ? (T)((double)x[r] + s) : (T)s;
+    x[r] = v;
+    if (SC) xs[threadIdx.x] = v;
+  }
+  if constexpr (SC) {
+    __syncthreads();
+    const int q1 = sc.mptr[min(i0 + kDenseRows, n)];
+    for (int q = sc.mptr[i0] + threadIdx.x; q < q1; q += kDenseThreads) {
+      const int f = sc.mem[q];
+      sc.x[f] = sc.x[f] + sc.alpha * xs[parent[f] - i0];
+    }
+  }
 }
 
 // FP64 inverse of the coarsest operator by Gauss-Jordan elimination without
 // pivoting (the coarse operators are diagonally dominant), one workgroup,
-// n <= kTailDirectMax.  A singular operator with zero row sums (the pure
+// n <= kDirectMax.  A singular operator with zero row sums (the pure
 // Neumann p' problem, null space = constants) is solved with its last
-// unknown pinned to zero: G is the inverse of the leading (n-1)x(n-1) block,
+// unknown pinned to zero: the result is the inverse of the leading (n-1)x(n-1) block,
 // bordered by zeros, a symmetric generalised inverse.  A zero or non-finite
-// pivot leaves G = 0 (no coarse correction) rather than garbage.
+// pivot leaves it 0 (no coarse correction) rather than garbage.
 constexpr int kInvThreads = 256;
 __global__ void __launch_bounds__(kInvThreads)
 k_coarse_inverse(int n, int w, const int *__restrict__ nbr, const double *__restrict__ ac,
-                 const double *__restrict__ anb, double *__restrict__ G) {
-  __shared__ double M[kTailDirectMax * kTailDirectMax];
-  __shared__ double rowk[kTailDirectMax], colk[kTailDirectMax];
+                 const double *__restrict__ anb, double *__restrict__ C) {
+  __shared__ double M[kDirectMax * kDirectMax];
+  __shared__ double rowk[kDirectMax], colk[kDirectMax];
   __shared__ int s_m, s_fail;
   const int nn = n * n;
   for (int e = threadIdx.x; e < nn; e += blockDim.x) {
@@ -923,21 +1009,23 @@ k_coarse_inverse(int n, int w, const int *__restrict__ nbr, const double *__rest
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    // off-diagonals in slot order; singularity test on the row sums
-    bool zero_rows = true;
-    for (int i = 0; i < n; ++i) {
-      double rs = ac[i];
-      for (int j = 0; j < w; ++j) {
-        const int k = nbr[(size_t)j * n + i];
-        if (k >= 0) {
-          M[i * n + k] += anb[(size_t)j * n + i];
-          rs += anb[(size_t)j * n + i];
-        }
-      }
-      if (!(fabs(rs) <= 1.0e-9 * fabs(ac[i]))) zero_rows = false;
-    }
-    s_m = zero_rows ? n - 1 : n;
+    s_m = n - 1;
     s_fail = 0;
+  }
+  __syncthreads();
+  // one row a thread, its off-diagonals in slot order (a level's neighbours
+  // are distinct); singularity test on the row sums
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    double rs = ac[i];
+    for (int j = 0; j < w; ++j) {
+      const int k = nbr[(size_t)j * n + i];
+      if (k >= 0) {
+        const double a = anb[(size_t)j * n + i];
+        M[i * n + k] += a;
+        rs += a;
+      }
+    }
+    if (!(fabs(rs) <= 1.0e-9 * fabs(ac[i]))) s_m = n; // every writer stores the same value
   }
   __syncthreads();
   const int m = s_m;
@@ -963,7 +1051,7 @@ k_coarse_inverse(int n, int w, const int *__restrict__ nbr, const double *__rest
   const bool fail = s_fail != 0;
   for (int e = threadIdx.x; e < nn; e += blockDim.x) {
     const int i = e / n, j = e % n;
-    G[e] = (!fail && i < m && j < m) ? M[i * n + j] : 0.0;
+    C[dense_at(i, j, n)] = (!fail && i < m && j < m) ? M[i * n + j] : 0.0;
   }
 }
 
@@ -984,7 +1072,6 @@ struct DLevel {
   DevBuf<int> color_cells;
   DevBuf<int> parent;            // 0-based parent in the next level
   DevBuf<int> mptr, mem;         // members of this level's aggregates (coarse)
-  std::vector<int> h_mptr, h_mem;
   DevBuf<int> gptr;
   DevBuf<int> gsrc;               // 32-bit: fine n + n w stays below 2^31
   int gne = 0;
@@ -994,6 +1081,10 @@ struct DLevel {
   DevBuf<int> csr_rp, csr_col, csr_pos;
   DevBuf<double> val64;
   DevBuf<float> val32;
+  // small levels: the dense map of the cycle from this level down, in the
+  // hierarchy's precision (the direct solve of a coarsest level always FP64)
+  DevBuf<double> dense64;
+  DevBuf<float> dense32;
   // large levels: sliced ELL instead (val64/val32 then hold the sliced
   // layout and csr_pos points into it)
   bool sell = false;
@@ -1046,14 +1137,13 @@ static void build_sell(int n, const std::vector<int> &rp, const std::vector<int>
   }
 }
 
-// The tail of one precision: its first level, descriptor and byte image.
-struct TailImage {
-  int ts = -1;                   // first tail level; == levels when there is no tail
-  TailDesc desc{};
-  DevBuf<unsigned char> img;
-  DevBuf<TailDesc> ddesc;
-  DevBuf<int> lin;               // CSR entry -> ELL linear index, all tail levels
-  std::vector<int> lin_off;      // per tail level
+// The levels whose cycle is held as a dense map (k_dense_level), for one
+// precision of the hierarchy.  ts: the first level of at most mg_tail_cells
+// cells (and whose map fits kDenseBytes), the bottom of the cycle pattern;
+// levels when there is none.  dl: the level the map is applied on, ts or the
+// level above it when that one's map fits as well.
+struct DenseTail {
+  int ts = -1, dl = -1;
 };
 
 struct Hierarchy {
@@ -1061,150 +1151,8 @@ struct Hierarchy {
   std::vector<DLevel> lev;
   int calls = 0;
   bool fp32 = false;
-  TailImage tail32, tail64;
+  DenseTail tail;
 };
-
-static size_t align16(size_t b) { return (b + 15) & ~(size_t)15; }
-
-static int lds_budget() {
-  static int budget = -1;
-  if (budget < 0) {
-    int dev = 0, v = 0;
-    budget = 64 * 1024;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 0)
-      budget = v;
-    budget = std::min(budget, 160 * 1024);
-    // the tail kernels ask for more than the default dynamic LDS window
-    if (hipFuncSetAttribute((const void *)k_tail<float>, hipFuncAttributeMaxDynamicSharedMemorySize, budget) !=
-            hipSuccess ||
-        hipFuncSetAttribute((const void *)k_tail<double>, hipFuncAttributeMaxDynamicSharedMemorySize, budget) !=
-            hipSuccess) {
-      (void)hipGetLastError();
-      budget = 64 * 1024;
-    }
-  }
-  return budget;
-}
-
-// lanes per row for a tail level: fewest dependent steps per sweep
-static int tail_lpr(int n, int nnz) {
-  int best = 1;
-  double best_cost = 1e30;
-  const double avg = n > 0 ? (double)nnz / n : 0.0;
-  for (int lpr = 1; lpr <= 16; lpr *= 2) {
-    const int rows = kTailThreads / lpr;
-    const double passes = std::ceil((double)n / rows);
-    int lg = 0;
-    while ((1 << lg) < lpr) ++lg;
-    const double cost = passes * (std::ceil(avg / lpr) + lg);
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = lpr;
-    }
-  }
-  return best;
-}
-
-// Lays out the tail of precision tsz (4 or 8 bytes) starting at the first
-// level at or below mg_tail_cells; moves the start down while the layout
-// does not fit the LDS budget, the level count or the uint16 index range.
-static void build_tail(fs_mesh *m, Hierarchy &H, TailImage &ti, size_t tsz) {
-  hipStream_t s = m->stream;
-  const int nl = (int)H.lev.size();
-  ti.ts = nl;
-  if (nl < 2) return;
-  int ts = nl;
-  for (int l = 1; l < nl; ++l)
-    if (H.lev[l].n <= m->mg_tail_cells) {
-      ts = l;
-      break;
-    }
-  const size_t budget = (size_t)lds_budget();
-  TailDesc d{};
-  for (; ts < nl; ++ts) {
-    const int nt = nl - ts;
-    if (nt > kTailMaxLev) continue;
-    d = TailDesc{};
-    d.nlev = nt;
-    size_t off = 0;
-    bool ok = true;
-    for (int q = 0; q < nt; ++q) {
-      const HostLevel &h = H.host[ts + q];
-      int nnz = 0;
-      for (int i = 0; i < h.n; ++i)
-        for (int j = 0; j < h.nnbr[i]; ++j)
-          if (h.nbr[(size_t)j * h.n + i] > 0) ++nnz;
-      if (h.n >= 65535 || nnz >= 65535 || (q > 0 && H.host[ts + q - 1].n >= 65535)) ok = false;
-      TailLvl &L = d.L[q];
-      L.n = h.n;
-      L.nnz = nnz;
-      L.lpr = tail_lpr(h.n, nnz);
-      L.o_ac = (int)off; off += align16(tsz * h.n);
-      L.o_val = (int)off; off += align16(tsz * std::max(nnz, 1));
-      L.o_col = (int)off; off += align16(2 * std::max(nnz, 1));
-      L.o_rp = (int)off; off += align16(2 * (h.n + 1));
-      L.o_par = (int)off; if (q + 1 < nt) off += align16(2 * h.n);
-      L.o_mp = (int)off; if (q > 0) off += align16(2 * (h.n + 1));
-      L.o_mem = (int)off; if (q > 0) off += align16(2 * H.host[ts + q - 1].n);
-    }
-    const int nc = d.L[nt - 1].n;
-    d.direct = nc <= kTailDirectMax ? 1 : 0;
-    d.o_g = (int)off;
-    if (d.direct) off += align16(sizeof(double) * nc * nc);
-    d.img_bytes = (int)off;
-    for (int q = 0; q < nt; ++q) {
-      TailLvl &L = d.L[q];
-      L.o_x = (int)off; off += align16(tsz * L.n);
-      L.o_t = (int)off; off += align16(tsz * L.n);
-      L.o_r = (int)off; off += align16(tsz * L.n);
-      L.o_b = (int)off; off += align16(tsz * L.n);
-    }
-    d.lds_bytes = (int)off;
-    if (ok && off <= budget) break;
-  }
-  ti.ts = ts;
-  if (ts >= nl) return;
-  // static sections of the image
-  std::vector<unsigned char> img(d.img_bytes, 0);
-  std::vector<int> lin;
-  ti.lin_off.assign(d.nlev, 0);
-  for (int q = 0; q < d.nlev; ++q) {
-    const HostLevel &h = H.host[ts + q];
-    const TailLvl &L = d.L[q];
-    unsigned short *col = (unsigned short *)(img.data() + L.o_col);
-    unsigned short *rp = (unsigned short *)(img.data() + L.o_rp);
-    ti.lin_off[q] = (int)lin.size();
-    int e = 0;
-    for (int i = 0; i < h.n; ++i) {
-      rp[i] = (unsigned short)e;
-      for (int j = 0; j < h.nnbr[i]; ++j) {
-        const int k = h.nbr[(size_t)j * h.n + i];
-        if (k > 0) {
-          col[e++] = (unsigned short)(k - 1);
-          lin.push_back(j * h.n + i);
-        }
-      }
-    }
-    rp[h.n] = (unsigned short)e;
-    if (q + 1 < d.nlev) {
-      unsigned short *par = (unsigned short *)(img.data() + L.o_par);
-      for (int i = 0; i < h.n; ++i) par[i] = (unsigned short)(h.parent[i] - 1);
-    }
-    if (q > 0) {
-      const DLevel &D = H.lev[ts + q];
-      unsigned short *mp = (unsigned short *)(img.data() + L.o_mp);
-      unsigned short *mem = (unsigned short *)(img.data() + L.o_mem);
-      for (int p = 0; p <= h.n; ++p) mp[p] = (unsigned short)D.h_mptr[p];
-      for (size_t t = 0; t < D.h_mem.size(); ++t) mem[t] = (unsigned short)D.h_mem[t];
-    }
-  }
-  if (lin.empty()) lin.push_back(0);
-  ti.desc = d;
-  ti.img.upload(img, s);
-  ti.ddesc.upload(&ti.desc, 1, s);
-  ti.lin.upload(lin, s);
-}
 
 static void build_hierarchy(fs_mesh *m, const double *ac, const double *anb) {
   auto H = std::make_shared<Hierarchy>();
@@ -1270,14 +1218,13 @@ static void build_hierarchy(fs_mesh *m, const double *ac, const double *anb) {
       D.gne = (int)gptrs[l].size() - 1;
       // members in increasing fine order
       const HostLevel &f = H->host[l - 1];
-      D.h_mptr.assign(h.n + 1, 0);
-      D.h_mem.assign(f.n, 0);
-      for (int i = 0; i < f.n; ++i) D.h_mptr[f.parent[i]]++;
-      for (int p = 0; p < h.n; ++p) D.h_mptr[p + 1] += D.h_mptr[p];
-      std::vector<int> fill(D.h_mptr.begin(), D.h_mptr.end() - 1);
-      for (int i = 0; i < f.n; ++i) D.h_mem[fill[f.parent[i] - 1]++] = i;
-      D.mptr.upload(D.h_mptr, s);
-      D.mem.upload(D.h_mem, s);
+      std::vector<int> mptr(h.n + 1, 0), mem(f.n, 0);
+      for (int i = 0; i < f.n; ++i) mptr[f.parent[i]]++;
+      for (int p = 0; p < h.n; ++p) mptr[p + 1] += mptr[p];
+      std::vector<int> fill(mptr.begin(), mptr.end() - 1);
+      for (int i = 0; i < f.n; ++i) mem[fill[f.parent[i] - 1]++] = i;
+      D.mptr.upload(mptr, s);
+      D.mem.upload(mem, s);
       std::vector<int> rp(h.n + 1, 0), col, pos((size_t)h.n * h.w, -1);
       for (int i = 0; i < h.n; ++i) {
         for (int j = 0; j < h.w; ++j) {
@@ -1333,13 +1280,79 @@ static void build_hierarchy(fs_mesh *m, const double *ac, const double *anb) {
     D.ac32.alloc(h.n);
     D.anb32.alloc((size_t)h.n * h.w);
   }
-  build_tail(m, *H, H->tail32, sizeof(float));
-  build_tail(m, *H, H->tail64, sizeof(double));
   FS_HIP_THROW(hipStreamSynchronize(s));
   m->amg = H;
 }
 
-void amg_prepare(fs_mesh *m, const double *ac, const double *anb) {
+// multicolour symmetric Gauss-Seidel only where it is cheap: few colours,
+// narrow rows
+static bool use_gs(const fs_mesh *m, const DLevel &D) {
+  return m->mg_smoother == 1 && (int)D.color_ptr.size() - 1 <= 4 && D.w <= 8;
+}
+
+// sweeps on the levels below the finest, and on a coarsest level too large
+// for the direct solve
+static int coarse_pre(const fs_mesh *m) { return m->mg_cpre >= 0 ? m->mg_cpre : m->mg_pre; }
+static int coarse_post(const fs_mesh *m) { return m->mg_cpost >= 0 ? m->mg_cpost : m->mg_post; }
+static int coarsest_sweeps(const fs_mesh *m) { return std::max(m->mg_coarse_sweeps, 1); }
+
+// The dense maps of the small levels, from the coarsest up to the one applied.
+static void build_dense(fs_mesh *m, Hierarchy &H, double alpha) {
+  hipStream_t s = m->stream;
+  const int nl = (int)H.lev.size(), most = dense_max(H.fp32 ? 4 : 8);
+  DenseTail &dt = H.tail;
+  dt.ts = nl;
+  for (int l = 1; l < nl; ++l)
+    if (H.lev[l].n <= std::min(m->mg_tail_cells, most)) {
+      dt.ts = l;
+      break;
+    }
+  dt.dl = dt.ts;
+  if (dt.ts >= nl) return;
+  if (dt.ts > 1) {
+    const DLevel &U = H.lev[dt.ts - 1];
+    if (U.n <= most && !U.sell && !use_gs(m, U)) dt.dl = dt.ts - 1;
+  }
+  const bool f32 = H.fp32;
+  for (int l = nl - 1; l >= dt.dl; --l) {
+    DLevel &D = H.lev[l];
+    const size_t size = dense_size(D.n);
+    const bool last = l == nl - 1, direct = last && D.n <= kDirectMax;
+    if (direct || !f32) D.dense64.alloc(size);
+    if (f32 && (!direct || l == dt.dl)) D.dense32.alloc(size);
+    if (direct) {
+      hipLaunchKernelGGL(k_coarse_inverse, dim3(1), dim3(kInvThreads), 0, s, D.n, D.w, D.nbr, D.ac64, D.anb64,
+                         D.dense64.p);
+      if (f32 && l == dt.dl)
+        hipLaunchKernelGGL(k_to<float>, dim3(gfor((int)size)), dim3(kBlock), 0, s, (int)size,
+                           (const double *)D.dense64.p, D.dense32.p);
+      continue;
+    }
+    DLevel *U = last ? nullptr : &H.lev[l + 1];
+    const bool below64 = !f32 || (!last && l + 1 == nl - 1 && U->n <= kDirectMax); // the type of the map below
+    const int nc = last ? 0 : U->n, pre = last ? coarsest_sweeps(m) : coarse_pre(m), post = last ? 0 : coarse_post(m);
+    const size_t lds = 16 * (2 * (size_t)D.n + nc) + sizeof(int) * (size_t)nc;
+    auto level = [&](auto kernel, const auto *anb, const auto *ac, const auto *Cc, auto *C) {
+      // the largest maps ask for more than the default dynamic LDS window
+      typedef std::decay_t<decltype(*C)> T;
+      if (lds > 64 * 1024)
+        FS_HIP_THROW(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      constexpr int K = Vec16<T>::K;
+      hipLaunchKernelGGL(kernel, dim3((D.n + K - 1) / K), dim3(kDenseThreads), (unsigned)lds, s, D.n, D.w, D.nbr,
+                         anb, ac, D.parent.p, nc, last ? nullptr : U->mptr.p, last ? nullptr : U->mem.p,
+                         Cc, pre, post, (T)m->mg_omega, (T)alpha, C);
+      FS_HIP_THROW(hipGetLastError()); // a refused launch (LDS request) must not pass silently
+    };
+    const double *c64 = last ? nullptr : U->dense64.p;
+    const float *c32 = last ? nullptr : U->dense32.p;
+    if (!f32) level(k_dense_level<double, double>, D.anb64, D.ac64, c64, D.dense64.p);
+    else if (below64)
+      level(k_dense_level<float, double>, (const float *)D.anb32.p, (const float *)D.ac32.p, c64, D.dense32.p);
+    else level(k_dense_level<float, float>, (const float *)D.anb32.p, (const float *)D.ac32.p, c32, D.dense32.p);
+  }
+}
+
+void amg_prepare(fs_mesh *m, const double *ac, const double *anb, double alpha) {
   const bool rebuild = !m->amg || (m->mg_reagg > 0 && m->ncalls_mg % m->mg_reagg == 0) ||
                        m->amg->lev.empty() || m->amg->lev[0].n != m->n;
   if (rebuild) build_hierarchy(m, ac, anb);
@@ -1362,30 +1375,7 @@ void amg_prepare(fs_mesh *m, const double *ac, const double *anb) {
                        H.fp32 ? C.ac32.p : nullptr, H.fp32 ? C.anb32.p : nullptr, C.csr_pos.p, C.val64.p,
                        H.fp32 ? C.val32.p : nullptr);
   }
-  // the tail of the precision in use: coefficients and the coarsest inverse
-  TailImage &ti = H.fp32 ? H.tail32 : H.tail64;
-  const int nl = (int)H.lev.size();
-  if (ti.ts < nl) {
-    const TailDesc &d = ti.desc;
-    for (int q = 0; q < d.nlev; ++q) {
-      DLevel &D = H.lev[ti.ts + q];
-      const TailLvl &L = d.L[q];
-      const int cnt = std::max(L.n, L.nnz);
-      unsigned char *base = ti.img.p;
-      if (H.fp32)
-        hipLaunchKernelGGL(k_tail_pack<float>, dim3(gfor(cnt)), dim3(kBlock), 0, s, L.n, L.nnz, D.ac64, D.anb64,
-                           ti.lin.p + ti.lin_off[q], (float *)(base + L.o_ac), (float *)(base + L.o_val));
-      else
-        hipLaunchKernelGGL(k_tail_pack<double>, dim3(gfor(cnt)), dim3(kBlock), 0, s, L.n, L.nnz, D.ac64,
-                           D.anb64, ti.lin.p + ti.lin_off[q], (double *)(base + L.o_ac),
-                           (double *)(base + L.o_val));
-    }
-    if (d.direct) {
-      DLevel &Dc = H.lev[nl - 1];
-      hipLaunchKernelGGL(k_coarse_inverse, dim3(1), dim3(kInvThreads), 0, s, Dc.n, Dc.w, Dc.nbr, Dc.ac64,
-                         Dc.anb64, (double *)(ti.img.p + d.o_g));
-    }
-  }
+  build_dense(m, H, alpha);
 }
 
 int amg_levels(fs_mesh *m) { return m->amg ? (int)m->amg->lev.size() : 1; }
@@ -1398,7 +1388,7 @@ template <class T> struct LV {
   static const T *ac(DLevel &d);
   static const T *anb(DLevel &d);
   static const T *val(DLevel &d);
-  static TailImage &tail(Hierarchy &h);
+  static const T *dense(DLevel &d);
 };
 template <> struct LV<double> {
   static double *x(DLevel &d) { return d.x64.p; }
@@ -1408,7 +1398,7 @@ template <> struct LV<double> {
   static const double *ac(DLevel &d) { return d.ac64; }
   static const double *anb(DLevel &d) { return d.anb64; }
   static const double *val(DLevel &d) { return d.val64.p; }
-  static TailImage &tail(Hierarchy &h) { return h.tail64; }
+  static const double *dense(DLevel &d) { return d.dense64.p; }
 };
 template <> struct LV<float> {
   static float *x(DLevel &d) { return d.x32.p; }
@@ -1418,7 +1408,7 @@ template <> struct LV<float> {
   static const float *ac(DLevel &d) { return d.ac32.p; }
   static const float *anb(DLevel &d) { return d.anb32.p; }
   static const float *val(DLevel &d) { return d.val32.p; }
-  static TailImage &tail(Hierarchy &h) { return h.tail32; }
+  static const float *dense(DLevel &d) { return d.dense32.p; }
 };
 
 // lanes per row of a coarse level's CSR kernels by its mean row length
@@ -1467,58 +1457,59 @@ static void launch_resid_restrict(fs_mesh *m, DLevel &D, DLevel &C, const T *b, 
   }
 }
 
-// one damped-Jacobi sweep on a grid-wide level, lanes per row by row width;
-// sweeps on the finest level go through the kernel clock (site
-// FS_CLOCK_FINE_SWEEP) with their algorithmic bytes: ac, b, x, the result, the
-// neighbour indices and the off-diagonal values, plus parent and the coarse
-// correction when the prolongation is fused in
-template <class T, class TO, bool PRO>
-static void launch_sweep(fs_mesh *m, DLevel &D, int level, const T *b, const T *x, const int *parent, const T *xc,
-                         int nc, T alpha, T om, TO *xn, const int *flags) {
+// one damped-Jacobi sweep on a coarse grid-wide level in CSR, lanes per row by
+// row width; with sc the prolongation of the result into the finer level
+template <class T, bool SC>
+static void launch_sweep_csr(fs_mesh *m, DLevel &D, const T *b, const T *x, T om, T *xn, Scatter<T> sc,
+                             const int *flags) {
+  hipStream_t s = m->stream;
+  const T *ac = LV<T>::ac(D), *val = LV<T>::val(D);
+  const int *rp = D.csr_rp.p, *col = D.csr_col.p;
+  switch (csr_lpr(D)) {
+  case 4:
+    hipLaunchKernelGGL((k_sweep_csr<4, T, SC>), dim3(gfor(D.n * 4)), dim3(kBlock), 0, s, D.n, rp, col, val, ac, b, x,
+                       om, xn, sc, flags);
+    break;
+  case 8:
+    hipLaunchKernelGGL((k_sweep_csr<8, T, SC>), dim3(gfor(D.n * 8)), dim3(kBlock), 0, s, D.n, rp, col, val, ac, b, x,
+                       om, xn, sc, flags);
+    break;
+  default:
+    hipLaunchKernelGGL((k_sweep_csr<16, T, SC>), dim3(gfor(D.n * 16)), dim3(kBlock), 0, s, D.n, rp, col, val, ac, b,
+                       x, om, xn, sc, flags);
+  }
+}
+
+// one damped-Jacobi sweep on the finest level, through the kernel clock (site
+// FS_CLOCK_FINE_SWEEP) with its algorithmic bytes: ac, b, x, the result, the
+// neighbour indices and the off-diagonal values
+template <class T, class TO>
+static void launch_sweep_fine(fs_mesh *m, DLevel &D, const T *b, const T *x, T om, TO *xn, const int *flags) {
   hipStream_t s = m->stream;
   const T *ac = LV<T>::ac(D), *anb = LV<T>::anb(D);
-  if (level > 0 && D.sell) {
-    hipLaunchKernelGGL((k_sweep_sell<T, TO, PRO>), dim3(gfor(D.sell_slots)), dim3(kBlock), 0, s, D.sell_slots,
-                       D.sell_ptr.p, D.sell_row.p, D.sell_col.p, LV<T>::val(D), ac, b, x, parent, xc, alpha, om, xn,
-                       flags);
-    return;
-  }
-  if (level > 0) {
-    const int *rp = D.csr_rp.p, *col = D.csr_col.p;
-    const T *val = LV<T>::val(D);
-    switch (csr_lpr(D)) {
-    case 4:
-      hipLaunchKernelGGL((k_sweep_csr<4, T, TO, PRO>), dim3(gfor(D.n * 4)), dim3(kBlock), 0, s, D.n, rp, col, val,
-                         ac, b, x, parent, xc, alpha, om, xn, flags);
-      break;
-    case 8:
-      hipLaunchKernelGGL((k_sweep_csr<8, T, TO, PRO>), dim3(gfor(D.n * 8)), dim3(kBlock), 0, s, D.n, rp, col, val,
-                         ac, b, x, parent, xc, alpha, om, xn, flags);
-      break;
-    default:
-      hipLaunchKernelGGL((k_sweep_csr<16, T, TO, PRO>), dim3(gfor(D.n * 16)), dim3(kBlock), 0, s, D.n, rp, col,
-                         val, ac, b, x, parent, xc, alpha, om, xn, flags);
-    }
-    return;
-  }
-  const int site = level == 0 ? FS_CLOCK_FINE_SWEEP : 0;
-  double bytes = 0.0;
-  if (site)
-    bytes = (double)D.n * (3.0 * sizeof(T) + sizeof(TO)) + (D.nbr16 ? 4.0 * ((D.w + 1) / 2) : 4.0 * D.w) * D.n +
-            (double)sizeof(T) * m->nnz + (PRO ? 4.0 * D.n + (double)sizeof(T) * nc : 0.0);
+  const double bytes = (double)D.n * (3.0 * sizeof(T) + sizeof(TO)) +
+                       (D.nbr16 ? 4.0 * ((D.w + 1) / 2) : 4.0 * D.w) * D.n + (double)sizeof(T) * m->nnz;
   const EllNbr nb(D.nbr, D.nbr16);
-  if (D.w <= 8)
-    timed_launch(m, site, bytes, k_sweep<1, T, TO, PRO>, dim3(gfor(D.n)), dim3(kBlock), 0, s, D.n, D.w, nb, ac, anb,
-                 b, x, parent, xc, alpha, om, xn, flags);
-  else if (D.w <= 16)
-    timed_launch(m, site, bytes, k_sweep<4, T, TO, PRO>, dim3(gfor(D.n * 4)), dim3(kBlock), 0, s, D.n, D.w, nb, ac,
-                 anb, b, x, parent, xc, alpha, om, xn, flags);
-  else if (D.w <= 32)
-    timed_launch(m, site, bytes, k_sweep<8, T, TO, PRO>, dim3(gfor(D.n * 8)), dim3(kBlock), 0, s, D.n, D.w, nb, ac,
-                 anb, b, x, parent, xc, alpha, om, xn, flags);
+  auto go = [&](auto kernel, int lpr) {
+    timed_launch(m, FS_CLOCK_FINE_SWEEP, bytes, kernel, dim3(gfor(D.n * lpr)), dim3(kBlock), 0, s, D.n, D.w, nb, ac, anb,
+                 b, x, om, xn, flags);
+  };
+  if (D.w <= 8) go(k_sweep<1, T, TO>, 1);
+  else if (D.w <= 16) go(k_sweep<4, T, TO>, 4);
+  else if (D.w <= 32) go(k_sweep<8, T, TO>, 8);
+  else go(k_sweep<16, T, TO>, 16);
+}
+
+// a sweep on any grid-wide level, nothing prolongated
+template <class T>
+static void launch_sweep(fs_mesh *m, DLevel &D, int level, const T *b, const T *x, T om, T *xn, const int *flags) {
+  if (level == 0)
+    launch_sweep_fine<T, T>(m, D, b, x, om, xn, flags);
+  else if (D.sell)
+    hipLaunchKernelGGL(k_sweep_sell<T>, dim3(gfor(D.sell_slots)), dim3(kBlock), 0, m->stream, D.sell_slots,
+                       D.sell_ptr.p, D.sell_row.p, D.sell_col.p, LV<T>::val(D), LV<T>::ac(D), b, x, om, xn, flags);
   else
-    timed_launch(m, site, bytes, k_sweep<16, T, TO, PRO>, dim3(gfor(D.n * 16)), dim3(kBlock), 0, s, D.n, D.w,
-                 D.nbr, ac, anb, b, x, parent, xc, alpha, om, xn, flags);
+    launch_sweep_csr<T, false>(m, D, b, x, om, xn, Scatter<T>{}, flags);
 }
 
 template <class T>
@@ -1542,12 +1533,6 @@ static void launch_resid(fs_mesh *m, DLevel &D, const T *b, const T *x, T *r, co
   else
     hipLaunchKernelGGL((k_resid<16, T>), dim3(gfor(D.n * 16)), dim3(kBlock), 0, s, D.n, D.w, nb, ac, anb, b, x, r,
                        flags);
-}
-
-// multicolour symmetric Gauss-Seidel only where it is cheap: few colours,
-// narrow rows
-static bool use_gs(const fs_mesh *m, const DLevel &D) {
-  return m->mg_smoother == 1 && (int)D.color_ptr.size() - 1 <= 4 && D.w <= 8;
 }
 
 template <class T>
@@ -1581,7 +1566,7 @@ static T *pre_smooth(fs_mesh *m, DLevel &D, int level, const T *b, int sweeps, T
     gs_sweeps<T>(m, D, b, cur, sweeps, flags); // x was zeroed by the caller
   } else {
     for (int k = 1; k < sweeps; ++k) {
-      launch_sweep<T, T, false>(m, D, level, b, cur, nullptr, nullptr, 0, T(0), om, oth, flags);
+      launch_sweep<T>(m, D, level, b, cur, om, oth, flags);
       std::swap(cur, oth);
     }
   }
@@ -1589,69 +1574,57 @@ static T *pre_smooth(fs_mesh *m, DLevel &D, int level, const T *b, int sweeps, T
   return cur;
 }
 
-// Prolongation of the coarse correction xc into x plus the post-smoothing
-// sweeps; the last operation writes dst (type TO), or a level buffer when dst
-// is null.  Returns the buffer holding the result when dst is null.
-template <class T, class TO>
-static T *post_smooth(fs_mesh *m, DLevel &D, int level, int nc, const T *b, T *x, T *other, const T *xc, int sweeps,
-                      T om, T al, TO *dst, const int *flags) {
+// Post-smoothing sweeps of a level whose iterate x already holds the coarse
+// correction.  Level 0 (out given) ends in out; a coarser level in a buffer,
+// which is returned, and with up given its result is prolongated into up (the
+// next finer level's iterate).
+template <class T>
+static T *post_smooth(fs_mesh *m, DLevel &D, int level, const T *b, T *x, T *other, int sweeps, T om, T al, DLevel *F,
+                      T *up, double *out, const int *flags) {
   hipStream_t s = m->stream;
-  if (use_gs(m, D)) {
-    hipLaunchKernelGGL((k_prolong<T, T>), dim3(gfor(D.n)), dim3(kBlock), 0, s, D.n, D.parent.p, xc, x, al, x,
-                       flags);
-    gs_sweeps<T>(m, D, b, x, sweeps, flags);
-    if (dst) hipLaunchKernelGGL((k_convert<T, TO>), dim3(gfor(D.n)), dim3(kBlock), 0, s, D.n, x, dst, flags);
-    return x;
-  }
-  if (sweeps == 0) {
-    if (dst) {
-      hipLaunchKernelGGL((k_prolong<T, TO>), dim3(gfor(D.n)), dim3(kBlock), 0, s, D.n, D.parent.p, xc, x, al, dst,
-                         flags);
-    } else {
-      hipLaunchKernelGGL((k_prolong<T, T>), dim3(gfor(D.n)), dim3(kBlock), 0, s, D.n, D.parent.p, xc, x, al, x,
-                         flags);
-    }
-    return x;
-  }
-  // the prolongation fused into the first sweep (each row adds the coarse
-  // value of itself and of its neighbours), or as a pass of its own first
-  // (FS_OPT_MG_FUSE_PROLONG 0: cheaper where the neighbours' parent lookups
-  // are scattered)
-  const bool fuse = m->mg_fuse_prolong != 0;
-  if (!fuse)
-    hipLaunchKernelGGL((k_prolong<T, T>), dim3(gfor(D.n)), dim3(kBlock), 0, s, D.n, D.parent.p, xc, x, al, x,
-                       flags);
+  const bool gs = use_gs(m, D);
   T *cur = x, *oth = other;
-  for (int k = 0; k < sweeps; ++k) {
-    const bool last = k + 1 == sweeps, pro = fuse && k == 0;
-    if (last && dst) {
-      if (pro) launch_sweep<T, TO, true>(m, D, level, b, cur, D.parent.p, xc, nc, al, om, dst, flags);
-      else launch_sweep<T, TO, false>(m, D, level, b, cur, nullptr, nullptr, 0, T(0), om, dst, flags);
-      return cur;
+  bool written = false; // the last sweep wrote out, or prolongated
+  if (gs) {
+    gs_sweeps<T>(m, D, b, x, sweeps, flags);
+  } else {
+    for (int k = 0; k < sweeps; ++k) {
+      const bool last = k + 1 == sweeps;
+      if (last && level == 0) {
+        launch_sweep_fine<T, double>(m, D, b, cur, om, out, flags);
+        return cur;
+      }
+      if (last && up && !D.sell) {
+        launch_sweep_csr<T, true>(m, D, b, cur, om, oth, Scatter<T>{D.mptr.p, D.mem.p, up, al}, flags);
+        written = true;
+      } else {
+        launch_sweep<T>(m, D, level, b, cur, om, oth, flags);
+      }
+      std::swap(cur, oth);
     }
-    if (pro) launch_sweep<T, T, true>(m, D, level, b, cur, D.parent.p, xc, nc, al, om, oth, flags);
-    else launch_sweep<T, T, false>(m, D, level, b, cur, nullptr, nullptr, 0, T(0), om, oth, flags);
-    std::swap(cur, oth);
   }
+  if (level == 0)
+    hipLaunchKernelGGL((k_convert<T, double>), dim3(gfor(D.n)), dim3(kBlock), 0, s, D.n, cur, out, flags);
+  else if (up && !written)
+    hipLaunchKernelGGL((k_prolong<T, T>), dim3(gfor(F->n)), dim3(kBlock), 0, s, F->n, F->parent.p, cur, up, al, up,
+                       flags);
   return cur;
 }
 
 // out = M^{-1} rhs: one V-cycle on the hierarchy held in precision T.  The
 // first sweep of each level is fused into the kernel that produces its
-// right-hand side, the prolongation into the first post-smoothing sweep, the
-// FP64 output into the last one; the levels from the tail's first level down
-// run in the one-workgroup tail kernel.  out must not alias rhs.
+// right-hand side, the prolongation into the kernel that finishes the coarser
+// level, the FP64 output into the last sweep; the levels from the tail's
+// applied level down are one dense product.  out must not alias rhs.
 template <class T>
 static void vcycle(fs_mesh *m, const double *rhs, double *out, double alpha, const int *flags) {
   Hierarchy &H = *m->amg;
   hipStream_t s = m->stream;
   const int L = (int)H.lev.size();
-  TailImage &ti = LV<T>::tail(H);
-  const int ts = std::min(ti.ts, L);
+  const int ts = H.tail.ts, dl = H.tail.dl;
   const T om = (T)m->mg_omega, al = (T)alpha;
   const int pre0 = m->mg_pre, post0 = m->mg_post;
-  const int cpre = m->mg_cpre >= 0 ? m->mg_cpre : pre0, cpost = m->mg_cpost >= 0 ? m->mg_cpost : post0;
-  const int coarse = std::max(m->mg_coarse_sweeps, 1);
+  const int cpre = coarse_pre(m), cpost = coarse_post(m), coarse = coarsest_sweeps(m);
   const bool fp64 = sizeof(T) == 8;
 
   DLevel &D0 = H.lev[0];
@@ -1667,13 +1640,14 @@ static void vcycle(fs_mesh *m, const double *rhs, double *out, double alpha, con
     return;
   }
   std::vector<T *> res(L, nullptr), oth(L, nullptr);
-  // levels above the bottom: grid-wide kernels
-  const int top = ts < L ? ts : L - 1;
+  const bool dense = dl < L;
+  const int bot = dense ? dl : L - 1;    // the level below the grid-wide ones
+  const int top = ts < L ? ts : L - 1;   // levels of the cycle pattern above its bottom
   // the restriction from level l into l + 1 also starts level l + 1: mode 0
-  // hands it to the tail kernel, 1 makes the first Jacobi sweep from zero,
+  // hands it to the dense product, 1 makes the first Jacobi sweep from zero,
   // 2 zeroes it (Gauss-Seidel)
   auto mode_from = [&](int l) {
-    if (l + 1 == ts) return 0;                                // the tail kernel takes over
+    if (dense && l + 1 == dl) return 0;                       // the dense product takes over
     if (l + 1 == L - 1) return 1;                             // grid-wide coarsest: `coarse` sweeps
     return (!use_gs(m, H.lev[l + 1]) && cpre > 0) ? 1 : 2;
   };
@@ -1688,72 +1662,90 @@ static void vcycle(fs_mesh *m, const double *rhs, double *out, double alpha, con
                          LV<T>::b(C), LV<T>::ac(C), LV<T>::x(C), om, mode, flags);
     }
   };
-  // the levels below the grid-wide ones
-  auto bottom = [&]() {
-    if (ts < L) {
-      DLevel &Dt = H.lev[ts];
-      hipLaunchKernelGGL(k_tail<T>, dim3(1), dim3(kTailThreads), ti.desc.lds_bytes, s, ti.ddesc.p, ti.img.p,
-                         LV<T>::b(Dt), LV<T>::x(Dt), cpre, cpost, coarse, om, al, flags);
-      FS_HIP_THROW(hipGetLastError()); // a refused launch (LDS request) must not pass silently
-      res[ts] = LV<T>::x(Dt);
+  auto dense_apply = [&](bool acc, bool up, const T *b) {
+    DLevel &D = H.lev[dl], &F = H.lev[dl - 1];
+    const Scatter<T> sc{D.mptr.p, D.mem.p, up ? res[dl - 1] : nullptr, al};
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((D.n + kDenseRows - 1) / kDenseRows), dim3(kDenseThreads), 0, s, D.n,
+                         LV<T>::dense(D), b, LV<T>::x(D), F.parent.p, sc, flags);
+    };
+    if (acc) {
+      if (up) go(k_dense_apply<T, true, true>);
+      else go(k_dense_apply<T, true, false>);
     } else {
-      DLevel &Dc = H.lev[L - 1];
-      // the restriction took the first of the coarse sweeps
-      T *o = nullptr;
-      res[L - 1] = pre_smooth<T>(m, Dc, L - 1, LV<T>::b(Dc), coarse, om, o, flags);
+      if (up) go(k_dense_apply<T, false, true>);
+      else go(k_dense_apply<T, false, false>);
     }
   };
-  // prolongation and post-smoothing from the bottom up to level stop (level
-  // 0 writes out)
+  // the bottom level from zero; up: its result is prolongated into the level
+  // above
+  auto bottom = [&](bool up) {
+    DLevel &D = H.lev[bot];
+    if (dense) {
+      dense_apply(false, up, LV<T>::b(D));
+      res[bot] = LV<T>::x(D);
+      return;
+    }
+    // the restriction took the first of the coarse sweeps
+    T *o = nullptr;
+    T *x = pre_smooth<T>(m, D, bot, LV<T>::b(D), coarse, om, o, flags);
+    if (up)
+      hipLaunchKernelGGL((k_prolong<T, T>), dim3(gfor(H.lev[bot - 1].n)), dim3(kBlock), 0, s, H.lev[bot - 1].n,
+                         H.lev[bot - 1].parent.p, x, res[bot - 1], al, res[bot - 1], flags);
+    res[bot] = x;
+  };
+  // post-smoothing from the bottom up to level stop (level 0 writes out);
+  // every level's result goes on into the next finer one, but for level stop's
   auto ascend = [&](int stop) {
-    for (int l = top - 1; l >= stop; --l) {
+    for (int l = bot - 1; l >= stop; --l) {
       DLevel &D = H.lev[l];
-      const T *b = l == 0 ? b0 : LV<T>::b(D);
-      const int npost = l == 0 ? post0 : cpost;
-      const int nc = H.lev[l + 1].n;
-      if (l == 0) {
-        post_smooth<T, double>(m, D, 0, nc, b, res[0], oth[0], res[1], npost, om, al, out, flags);
-      } else {
-        res[l] = post_smooth<T, T>(m, D, l, nc, b, res[l], oth[l], res[l + 1], npost, om, al, (T *)nullptr, flags);
-        oth[l] = res[l] == LV<T>::x(D) ? LV<T>::t(D) : LV<T>::x(D);
-      }
+      T *up = l > stop ? res[l - 1] : nullptr;
+      res[l] = post_smooth<T>(m, D, l, l == 0 ? b0 : LV<T>::b(D), res[l], oth[l], l == 0 ? post0 : cpost, om, al,
+                              l > 0 ? &H.lev[l - 1] : nullptr, up, out, flags);
+      if (l > 0) oth[l] = res[l] == LV<T>::x(D) ? LV<T>::t(D) : LV<T>::x(D);
     }
   };
   // a second coarse-grid correction of level l1 >= 1 (F and W cycles):
   // pre-sweeps from its current iterate, then a fresh descent (every coarser
-  // level from zero) to the bottom
-  auto redescend = [&](int l1) {
+  // level from zero) to the bottom.  On the dense level itself this is one
+  // more cycle from the iterate it has: x += C (b - A x).
+  auto redescend = [&](int l1, bool up) {
     DLevel &D = H.lev[l1];
     const T *b = LV<T>::b(D);
+    if (l1 == bot) {
+      launch_resid<T>(m, D, b, res[l1], LV<T>::r(D), flags);
+      dense_apply(true, up, LV<T>::r(D));
+      return;
+    }
     T *cur = res[l1], *o = oth[l1];
     if (use_gs(m, D)) {
       gs_sweeps<T>(m, D, b, cur, cpre, flags);
     } else {
       for (int k = 0; k < cpre; ++k) {
-        launch_sweep<T, T, false>(m, D, l1, b, cur, nullptr, nullptr, 0, T(0), om, o, flags);
+        launch_sweep<T>(m, D, l1, b, cur, om, o, flags);
         std::swap(cur, o);
       }
     }
     res[l1] = cur;
     oth[l1] = o;
     restrict_from(l1, b, cur);
-    for (int l = l1 + 1; l < top; ++l) {
+    for (int l = l1 + 1; l < bot; ++l) {
       DLevel &Dl = H.lev[l];
       res[l] = pre_smooth<T>(m, Dl, l, LV<T>::b(Dl), cpre, om, oth[l], flags);
       restrict_from(l, LV<T>::b(Dl), res[l]);
     }
-    bottom();
+    bottom(up);
   };
 
   // one Jacobi pre-sweep on the finest level: the entry and the residual of
   // that sweep in one kernel
-  const bool fuse0 = !use_gs(m, D0) && pre0 == 1 && top > 0;
+  const bool fuse0 = !use_gs(m, D0) && pre0 == 1 && bot > 0;
   if (!fuse0) {
     const bool gs = use_gs(m, D0);
     hipLaunchKernelGGL(k_enter<T>, dim3(gfor(D0.n)), dim3(kBlock), 0, s, D0.n, LV<T>::ac(D0), rhs,
                        fp64 ? nullptr : LV<T>::b(D0), LV<T>::x(D0), om, (!gs && pre0 > 0) ? 1 : 0, flags);
   }
-  for (int l = 0; l < top; ++l) {
+  for (int l = 0; l < bot; ++l) {
     DLevel &D = H.lev[l];
     const T *b = l == 0 ? b0 : LV<T>::b(D);
     const int npre = l == 0 ? pre0 : cpre;
@@ -1771,22 +1763,23 @@ static void vcycle(fs_mesh *m, const double *rhs, double *out, double alpha, con
     res[l] = pre_smooth<T>(m, D, l, b, npre, om, oth[l], flags);
     restrict_from(l, b, res[l]);
   }
-  bottom();
   // F and W cycles (FS_OPT_MG_CYCLE 1, 2) in the pattern of the reference's
   // fMultiGridCycle and wMultiGridCycle (MultiGridCycle.for:84-127, 162-220):
-  // back up to level l1 and down again, for l1 from the deepest grid-wide
-  // level up to level 1, and for W once more from level 2 down to the
+  // back up to level l1 and down again, for l1 from the deepest level above
+  // the tail up to level 1, and for W once more from level 2 down to the
   // deepest; the levels from the tail's first level down count as one
+  std::vector<int> again;
   if (m->mg_cycle >= 1)
-    for (int l1 = top - 1; l1 >= 1; --l1) {
-      ascend(l1);
-      redescend(l1);
-    }
+    for (int l1 = top - 1; l1 >= 1; --l1) again.push_back(l1);
   if (m->mg_cycle == 2)
-    for (int l1 = 2; l1 <= top - 1; ++l1) {
-      ascend(l1);
-      redescend(l1);
-    }
+    for (int l1 = 2; l1 <= top - 1; ++l1) again.push_back(l1);
+  // the bottom's result goes up unless the next correction is the bottom's own
+  auto goes_up = [&](size_t k) { return k >= again.size() || again[k] != bot; };
+  bottom(goes_up(0));
+  for (size_t k = 0; k < again.size(); ++k) {
+    if (again[k] != bot) ascend(again[k]);
+    redescend(again[k], goes_up(k + 1));
+  }
   ascend(0);
 }
 
@@ -1801,13 +1794,13 @@ void amg_apply(fs_mesh *m, const double *rhs, double *out, const int *flags, dou
 int amg_solve(fs_mesh *m, const double *ac, const double *anb, const double *bc, double *dphi,
               int solver, bool warm) {
   (void)solver;
-  amg_prepare(m, ac, anb);
+  // additive correction as in the reference unless asked otherwise
+  const double alpha = m->mg_alpha > 0.0 ? m->mg_alpha : 1.0;
+  amg_prepare(m, ac, anb, alpha);
   hipStream_t s = m->stream;
   const int n = m->n;
   double *r = m->wk.v[8], *c = m->wk.v[9];
   int *flags = m->wk.flags;
-  // additive correction as in the reference unless asked otherwise
-  const double alpha = m->mg_alpha > 0.0 ? m->mg_alpha : 1.0;
   // flags[2] holds itmax for the Krylov solvers; the multigrid loop is
   // bounded by MaxMultiGridCycles instead
   int itmax_cycles = m->mg_maxcycles;

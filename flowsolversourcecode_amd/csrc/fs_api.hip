@@ -211,7 +211,7 @@ int fs_set_option(fs_mesh *m, int key, double value) {
   case FS_OPT_MG_COARSE_PRESWEEP: m->mg_cpre = iv < -1 ? -1 : iv; break;
   case FS_OPT_MG_COARSE_POSTSWEEP: m->mg_cpost = iv < -1 ? -1 : iv; break;
   case FS_OPT_MG_SELL_ROWS: m->mg_sell_rows = iv < 0 ? 0 : iv; break;
-  case FS_OPT_MG_FUSE_PROLONG: m->mg_fuse_prolong = iv != 0; break;
+  case FS_OPT_MG_FUSE_PROLONG: break; // both forms take the same route now
   case FS_OPT_MG_CYCLE:
     if (iv < 0 || iv > 2) {
       set_error("fs_set_option: MG_CYCLE must be 0 (V), 1 (F) or 2 (W)");

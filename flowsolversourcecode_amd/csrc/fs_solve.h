@@ -60,7 +60,8 @@ int project_guess(fs_mesh *m, const double *ac, const double *anb, const double 
 // AMG (fs_amg.hip).  amg_prepare builds or refreshes the hierarchy for the
 // fine operator (ac, anb): aggregation on the first call and every
 // mg_reagg calls, device Galerkin operators otherwise.
-void amg_prepare(fs_mesh *m, const double *ac, const double *anb);
+// The coarse corrections of the cycles that follow are scaled by alpha.
+void amg_prepare(fs_mesh *m, const double *ac, const double *anb, double alpha);
 // out = one V-cycle applied to rhs (both FP64 device vectors, not aliased),
 // coarse corrections scaled by alpha.
 void amg_apply(fs_mesh *m, const double *rhs, double *out, const int *flags, double alpha);

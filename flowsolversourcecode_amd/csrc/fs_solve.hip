@@ -1455,8 +1455,8 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     // both r and rr (the transpose preconditioner is the cycle itself: exact
     // for symmetric operators such as p', an approximation otherwise)
     const bool pre = (lmg == FS_MG_PRECOND);
-    if (pre) amg_prepare(m, ac, anb);
     const double alpha = m->mg_alpha > 0.0 ? m->mg_alpha : 1.7;
+    if (pre) amg_prepare(m, ac, anb, alpha);
     const double *dc = pre ? nullptr : m->wk.dc;
     iters = run_batches(m, itmax, nf * 8 + solver, [&]() {
       if (pre) {
@@ -1500,8 +1500,8 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   } else if (solver == FS_BICGS) {
     // right-preconditioned BiCGSTAB; r=V0 r0=V1 p=V2 v=V3 s=V4 t=V5 phat=V6 shat=V7
     const bool pre = (lmg == FS_MG_PRECOND);
-    if (pre) amg_prepare(m, ac, anb);
     const double alpha = m->mg_alpha > 0.0 ? m->mg_alpha : 1.7;
+    if (pre) amg_prepare(m, ac, anb, alpha);
     // algorithmic bytes of y = A x with the (r0, y) partials: ac, the
     // neighbour words (4 per slot, or 4 per pair of slots), anb, x, y, r0
     const double ib = nb.d16 ? 4.0 * ((w + 1) / 2) : 4.0 * w;
@@ -1531,8 +1531,8 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   } else if (solver == FS_CG) {
     // preconditioned conjugate gradient; r=V0 z=V1 p=V2 q=V3
     const bool pre = (lmg == FS_MG_PRECOND);
-    if (pre) amg_prepare(m, ac, anb);
     const double alpha = m->mg_alpha > 0.0 ? m->mg_alpha : 1.7;
+    if (pre) amg_prepare(m, ac, anb, alpha);
     // y = A p with the (p, y) partials: ac, nbr, anb, p, y
     const double spmv_bytes = 8.0 * n + (nb.d16 ? 4.0 * ((w + 1) / 2) : 4.0 * w) * n + 8.0 * m->nnz + 16.0 * n;
     hipLaunchKernelGGL(k_resid_vec, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, V0, nullptr,
@@ -1558,8 +1558,8 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     // target, the basis is full or itmax is reached; the stop rule is checked on
     // the true L1 residual at every restart
     const bool pre = (lmg == FS_MG_PRECOND);
-    if (pre) amg_prepare(m, ac, anb);
     const double alpha = m->mg_alpha > 0.0 ? m->mg_alpha : 1.7;
+    if (pre) amg_prepare(m, ac, anb, alpha);
     const int gmm = std::max(1, std::min(64, m->gmres_m));
     if (sw.gm_m != gmm || sw.gm_V.n < (size_t)(gmm + 1) * n) {
       sw.gm_V.alloc((size_t)(gmm + 1) * n);

@@ -78,8 +78,11 @@ enum fs_option {
                                  of the previous solve of the same variable
                                  and solver (at most 4x this), later batches
                                  grow 2, 4, ... up to this                     */
-  FS_OPT_MG_TAIL_CELLS = 12,  /* levels with at most this many cells run in one
-                                 single-workgroup kernel [1024]                 */
+  FS_OPT_MG_TAIL_CELLS = 12,  /* from the first level with at most this many
+                                 cells down (at most 2048 cells in FP32, 1448
+                                 in FP64) the cycle is formed as one dense map
+                                 and counts as one level; 0 = no such level
+                                 [1024]                                        */
   FS_OPT_MG_COARSE_SWEEPS = 13,/* smoothing sweeps on a coarsest level too large
                                  for the direct FP64 solve (> 64 cells) [16]   */
   FS_OPT_MG_ALPHA = 14,       /* over-correction of the prolongated coarse
@@ -98,9 +101,11 @@ enum fs_option {
                                  its strongest negative coupling, 2 = two
                                  pairwise passes per level (aggregates of up to
                                  4 cells) -- no reference counterpart [0]      */
-  FS_OPT_MG_FUSE_PROLONG = 19, /* 1 = the prolongation of the coarse correction
-                                 fused into the first post-sweep of grid-wide
-                                 levels, 0 = a pass of its own before it [1]   */
+  FS_OPT_MG_FUSE_PROLONG = 19, /* accepted and without effect: the prolongation
+                                 of a coarse correction runs in the kernel that
+                                 finishes the coarse level, or as a pass of its
+                                 own, by the level's layout (the same values
+                                 either way) [1]                               */
   FS_OPT_WARM_PREVIOUS = 20   /* device SIMPLE case (fsamd_simple.h) without a
                                  warm-start network: 1 = start each p' solve
                                  from the previous iteration's p', scaled to
@@ -114,8 +119,8 @@ enum fs_option {
                                  (back up to level l and down again, for l from
                                  the deepest grid-wide level up to 1; W once
                                  more from 2 down), every coarser level of a
-                                 descent starting from zero; the one-workgroup
-                                 tail counts as one level [0]                  */
+                                 descent starting from zero; the levels of the
+                                 dense map count as one [0]                    */
 };
 
 /* Statistics of the last solve. */

@@ -1,0 +1,150 @@
+"""One multigrid cycle on the device against the same cycle in numpy.
+
+The cycle below the first small level is applied as a dense matrix the device
+forms from the level operators, and each level's correction is prolongated by
+the kernel that finishes the level.  Here one cycle (multigrid as the solver,
+one cycle allowed) is restated in numpy in FP64 from the exported hierarchy:
+damped Jacobi from zero, residuals summed over aggregates, alpha times the
+injected correction, the coarsest level smoothed or, as part of the tail and of
+at most 64 cells, solved directly (its last unknown pinned when every row sum is
+zero).
+
+Tolerances: an FP64 cycle is about 100 operations deep with terms of one
+size, 100 eps ~ 2e-14 of the largest entry times the growth of the coarsest
+solve (its condition, below 1e3 here): 1e-11.  FP32 likewise 100 * 6e-8 = 6e-6
+from the sweeps; the coarsest solve is FP64 on FP32 data: 1e-4.
+"""
+import numpy as np
+import pytest
+
+import systems
+
+fs = pytest.importorskip("flowsolversourcecode_amd")
+pytestmark = pytest.mark.gpu
+
+
+class Level:
+    def __init__(self, d):
+        import scipy.sparse as sp
+        n, w = d["n"], d["w"]
+        rows, cols, vals = [np.arange(n)], [np.arange(n)], [d["ac"]]
+        for j in range(w):
+            k = np.nonzero((d["nbr"][j] > 0) & (j < d["nnbr"]))[0]
+            rows.append(k)
+            cols.append(d["nbr"][j][k] - 1)
+            vals.append(d["anb"][j][k])
+        self.A = sp.csr_matrix((np.concatenate(vals), (np.concatenate(rows), np.concatenate(cols))), shape=(n, n))
+        self.n, self.ac, self.parent = n, d["ac"], d["parent"] - 1
+
+
+def coarsest(L, b, om, sweeps):
+    """sweeps < 0: the level belongs to the tail and is solved directly if small"""
+    if sweeps > 0 or L.n > 64:
+        sweeps = abs(sweeps)
+        return smooth(L, b, np.zeros(L.n), sweeps, om)
+    A = L.A.toarray()
+    m = L.n - 1 if np.all(np.abs(A.sum(1)) <= 1e-9 * np.abs(L.ac)) else L.n
+    x = np.zeros(L.n)
+    x[:m] = np.linalg.solve(A[:m, :m], b[:m])
+    return x
+
+
+def smooth(L, b, x, sweeps, om):
+    for _ in range(sweeps):
+        x = x + om * (b - L.A @ x) / L.ac
+    return x
+
+
+def cycle(levels, ts, b, pre, post, om, alpha, kind, csweeps):
+    """out = M b; kind 0 V, 1 F, 2 W, the levels from ts down counting as one."""
+    L = len(levels)
+    x, r = [None] * L, [None] * L
+    r[0] = b
+
+    def descend(l0, stop):
+        """from level l0's iterate down to stop, every coarser level from zero"""
+        for l in range(l0, stop):
+            res = r[l] - levels[l].A @ x[l]
+            r[l + 1] = np.bincount(levels[l].parent, res, levels[l + 1].n)
+            x[l + 1] = np.zeros(levels[l + 1].n)
+            if l + 1 < stop:
+                x[l + 1] = smooth(levels[l + 1], r[l + 1], x[l + 1], pre, om)
+
+    def bottom():
+        for l in range(ts, L - 1):
+            x[l] = smooth(levels[l], r[l], np.zeros(levels[l].n), pre, om)
+            r[l + 1] = np.bincount(levels[l].parent, r[l] - levels[l].A @ x[l], levels[l + 1].n)
+        x[L - 1] = coarsest(levels[L - 1], r[L - 1], om, csweeps)
+        ascend(L - 1, ts)
+
+    def ascend(frm, stop):
+        for l in range(frm - 1, stop - 1, -1):
+            x[l] = smooth(levels[l], r[l], x[l] + alpha * x[l + 1][levels[l].parent], post, om)
+
+    x[0] = smooth(levels[0], b, np.zeros(levels[0].n), pre, om)
+    descend(0, ts)
+    bottom()
+    again = []
+    if kind >= 1:
+        again += list(range(ts - 1, 0, -1))
+    if kind == 2:
+        again += list(range(2, ts))
+    for l1 in again:
+        ascend(ts, l1)
+        x[l1] = smooth(levels[l1], r[l1], x[l1], pre, om)
+        descend(l1, ts)
+        bottom()
+    ascend(ts, 0)
+    return x[0]
+
+
+def run(system, opts):
+    nbr, nnbr, ac, anb, bc = system
+    m = fs.Mesh(nbr, nnbr)
+    for k, v in opts.items():
+        m.set_option(k, v)
+    m.set_option("mg_maxcycles", 1)
+    _, _, dphi, _, _ = m.solve_equation("pressc", np.zeros(len(ac)), 1e-12, 1, "sor", 1, ac, anb, bc)
+    d = [m.amg_level(0)]
+    d += [m.amg_level(k) for k in range(1, d[0]["levels"])]
+    return dphi, [Level(x) for x in d]
+
+
+# cells: one or two small levels; the level above the tail small enough for a
+# dense map of its own (dl = ts - 1) or not; odd sizes off the 16-row tiles
+@pytest.mark.parametrize("shape", [(5, 4, 3), (13, 11, 9), (32, 24, 20), (41, 37, 1)])
+@pytest.mark.parametrize("opts", [
+    {}, {"mg_fp32": 1}, {"mg_presweep": 1, "mg_postsweep": 1}, {"mg_presweep": 1, "mg_postsweep": 2, "mg_fp32": 1},
+    {"mg_coarse_presweep": 0, "mg_coarse_postsweep": 2}, {"mg_coarse_presweep": 3, "mg_coarse_postsweep": 0},
+    {"mg_tail_cells": 100}, {"mg_tail_cells": 100, "mg_cycle": 1}, {"mg_tail_cells": 100, "mg_cycle": 2, "mg_fp32": 1},
+    {"mg_tail_cells": 5, "mg_cycle": 2}, {"mg_maxlevels": 2, "mg_coarse_sweeps": 3},
+    {"mg_maxlevels": 3, "mg_coarse_sweeps": 4, "mg_fp32": 1}, {"mg_alpha": 1.9, "mg_cycle": 1, "mg_sell_rows": 1},
+], ids=lambda o: ",".join(f"{k[3:]}={v}" for k, v in o.items()) or "default")
+@pytest.mark.parametrize("shift", [0.0, 0.05])
+def test_one_cycle_is_numpys(shape, opts, shift):
+    system = systems.pressure_like(*shape, 7, shift=shift)
+    dphi, levels = run(system, opts)
+    if len(levels) < 2:
+        pytest.skip("no coarse level")
+    most = 2048 if opts.get("mg_fp32") else 1448
+    ts = next((l for l in range(1, len(levels)) if levels[l].n <= min(opts.get("mg_tail_cells", 1024), most)), None)
+    cs = opts.get("mg_coarse_sweeps", 16)
+    want = full_cycle(levels, len(levels) - 1 if ts is None else ts, system[4], opts, cs if ts is None else -cs)
+    scale = np.abs(want).max()
+    np.testing.assert_allclose(dphi, want, rtol=0, atol=(1e-4 if opts.get("mg_fp32") else 1e-11) * scale)
+
+
+def full_cycle(levels, ts, bc, opts, cs):
+    """cycle() with the finest level's own sweep counts."""
+    p0, q0 = opts.get("mg_presweep", 2), opts.get("mg_postsweep", 2)
+    cp, cq = opts.get("mg_coarse_presweep", p0), opts.get("mg_coarse_postsweep", q0)
+    om, alpha = 0.8, opts.get("mg_alpha", 1.0)
+    if (p0, q0) == (cp, cq):
+        return cycle(levels, ts, bc, p0, q0, om, alpha, opts.get("mg_cycle", 0), cs)
+    assert not opts.get("mg_cycle", 0)
+    L0 = levels[0]
+    x = smooth(L0, bc, np.zeros(L0.n), p0, om)
+    r1 = np.bincount(L0.parent, bc - L0.A @ x, levels[1].n)
+    rest = levels[1:]
+    xc = coarsest(rest[0], r1, om, cs) if len(rest) == 1 else cycle(rest, max(ts - 1, 0), r1, cp, cq, om, alpha, 0, cs)
+    return smooth(L0, bc, x + alpha * xc[L0.parent], q0, om)
