@@ -107,12 +107,6 @@ struct fs_mesh {
   fs::DevBuf<int> d_nbr16;  // the same as int16 offsets k - i (0 = none), two
                             // slots per word, when every offset fits
   fs::DevBuf<int> d_mir;    // transpose map, linear anb index or -1
-  // exact natural-order D-ILU schedule (FactorizeUsingILU.for:29-75)
-  int ilu_nlevels = 0;
-  std::vector<int> ilu_level_ptr;
-  fs::DevBuf<int> d_ilu_cells;     // cells sorted by level
-  fs::DevBuf<int> d_ilu_ptr;       // [n+1] per-cell lower terms
-  fs::DevBuf<int> d_ilu_a, d_ilu_i, d_ilu_b; // anb(j,s) idx, i, anb(i,s') idx
   // face topology (optional)
   int nif = 0, nfaces_total = 0;
   std::vector<int> h_owner, h_neigh;

@@ -308,20 +308,140 @@ __global__ void k_pbcg_axpy(int n, double *__restrict__ dphi, double *__restrict
   rr[i] = rr[i] - ak * zz[i];
 }
 
-// Exact natural-order D-ILU diagonal, one dependency level per launch
-// (FactorizeUsingILU.for:23-75 in pull form): dc_j = 1/(ac_j - sum over the
-// lower couplings i of anb(j,i)*dc_i*anb(i,j)), terms in the reference's
-// push order.
-__global__ void k_ilu_level(int cnt, const int *__restrict__ cells, const int *__restrict__ ptr,
-                            const int *__restrict__ ta, const int *__restrict__ ti,
-                            const int *__restrict__ tb, const double *__restrict__ ac,
-                            const double *__restrict__ anb, double *__restrict__ dc) {
+// ---- level schedules of the natural-order triangular recurrences (the
+// D-ILU diagonal, ILU's forward and backward substitutions).  The cells are
+// sorted by dependency level, and everything a recurrence reads or writes is
+// kept in that order: position t has up to D terms, term e at [e n + t], each
+// naming the position it takes its value from.
+//
+// A level of a few hundred cells is far too short for a launch of its own
+// (3.1-3.5 us each, 183 levels for 86k tetrahedra, 138 for 101k hexahedra),
+// so a run of consecutive levels of at most kIluNarrow cells is worked by ONE
+// workgroup with a workgroup barrier between the levels: 1.06 us a level, 194
+// us a substitution of the tetrahedra instead of 600, 255 us for the
+// hexahedra's diagonal instead of 910.  What one CU
+// can fetch bounds it, hence the order: in cell order the values a level takes
+// lie on a line of memory each (1.7 us a level of 470 tetrahedra, 10 us a
+// level of 730 hexahedra with three gathered terms).  A wider level is left to
+// a launch over the chip: beyond about 2000 cells one CU's share of the cache
+// bandwidth costs more than the launch.
+//
+// steps: positions in order, each step at most a workgroup wide, twice the
+// position plus 1 where a level ends (the dependents start there).  A step's
+// own data do not depend on earlier levels and are loaded one step ahead,
+// behind the loads of the values that do.
+constexpr int kIluNarrow = 2048;
+constexpr int kIluThreads = 1024;
+constexpr int kIluTerms = 8; // most terms of a cell the runs carry in registers
+
+// out[q] = in[idx[q]] (a vector, or the terms' matrix entries, into an order)
+__global__ void k_gather(long long cnt, const int *__restrict__ idx, const double *__restrict__ in,
+                         double *__restrict__ out, const int *__restrict__ flags) {
+  if (flags && flags[F_DONE]) return;
+  const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
+  if (q < cnt) out[q] = in[idx[q]];
+}
+
+// x[cell[t]] += y[t]
+__global__ void k_scatter_add(int n, const int *__restrict__ cell, const double *__restrict__ y,
+                              double *__restrict__ x, const int *__restrict__ flags) {
+  if (flags && flags[F_DONE]) return;
   const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= cnt) return;
-  const int j = cells[t];
-  double d = ac[j];
-  for (int e = ptr[j]; e < ptr[j + 1]; ++e) d = d - anb[ta[e]] * dc[ti[e]] * anb[tb[e]];
-  dc[j] = 1.0 / d;
+  if (t >= n) return;
+  const int c = cell[t];
+  x[c] = x[c] + y[t];
+}
+
+// The recurrences, position t with right-hand side r, terms (a, b) and the
+// values y they take:
+//   DIAG   v = r - a y b - ...,  y_t = 1/v: dc_j = 1/(ac_j - sum of
+//          anb(j,i) dc_i anb(i,j)), terms in the reference's push order
+//          (FactorizeUsingILU.for:23-75 in pull form)
+//   FWD    v = r - a y - ...,    y_t = d v, and v kept: rc_j -= anb(j,i) (dc_i rc_i)
+//   BWD    v = r - a y - ...,    y_t = d v: rc_i -= anb(i,j) rc_j, rc_i = dc_i rc_i
+enum IluOp { ILU_DIAG = 0, ILU_FWD = 1, ILU_BWD = 2 };
+struct IluArgs {
+  int n;
+  const int *src;       // positions of the terms' values, -1: no term
+  const double *a, *b;  // the terms' matrix entries (b: DIAG only)
+  const double *r, *d;  // right-hand side, D-ILU diagonal (not DIAG)
+  double *y, *v;        // results; v: FWD only
+};
+
+template <int OP> __device__ __forceinline__ double ilu_term(double v, double a, double y, double b) {
+  if constexpr (OP == ILU_DIAG) return v - a * y * b;
+  else return v - a * y;
+}
+template <int OP> __device__ __forceinline__ void ilu_store(const IluArgs &A, int t, double v, double d) {
+  A.y[t] = OP == ILU_DIAG ? 1.0 / v : d * v;
+  if constexpr (OP == ILU_FWD) A.v[t] = v;
+}
+
+template <int OP, int D>
+__global__ void __launch_bounds__(kIluThreads)
+k_ilu_run(int ns, const int *__restrict__ steps, IluArgs A, const int *__restrict__ flags) {
+  if (flags && flags[F_DONE]) return;
+  const int *__restrict__ src = A.src;
+  const double *__restrict__ ta = A.a, *__restrict__ tb = A.b, *__restrict__ tr = A.r, *__restrict__ td = A.d;
+  const double *y = A.y;
+  struct Own { // one position's data: nothing earlier levels write
+    bool on;
+    int i[D];
+    double a[D], b[D], r, d;
+  };
+  auto fetch = [&](int p0, int p1, Own &o) {
+    const int t = p0 + (int)threadIdx.x;
+    o.on = t < p1;
+#pragma unroll
+    for (int e = 0; e < D; ++e) o.i[e] = -1;
+    if (!o.on) return;
+#pragma unroll
+    for (int e = 0; e < D; ++e) {
+      const size_t q = (size_t)e * A.n + t;
+      o.i[e] = src[q];
+      o.a[e] = ta[q];
+      if constexpr (OP == ILU_DIAG) o.b[e] = tb[q];
+    }
+    o.r = tr[t];
+    if constexpr (OP != ILU_DIAG) o.d = td[t];
+  };
+  Own cur, nxt;
+  int p0 = steps[0] >> 1, end = steps[1], next = ns > 1 ? steps[2] : end;
+  fetch(p0, end >> 1, cur);
+  for (int s = 0; s < ns; ++s) {
+    const int after = s + 3 <= ns ? steps[s + 3] : next;
+    double yv[D];
+#pragma unroll
+    for (int e = 0; e < D; ++e) yv[e] = cur.i[e] >= 0 ? y[cur.i[e]] : 0.0;
+    fetch(end >> 1, next >> 1, nxt);
+    if (cur.on) {
+      double v = cur.r;
+#pragma unroll
+      for (int e = 0; e < D; ++e)
+        if (cur.i[e] >= 0) v = ilu_term<OP>(v, cur.a[e], yv[e], cur.b[e]);
+      ilu_store<OP>(A, p0 + (int)threadIdx.x, v, cur.d);
+    }
+    if (end & 1) __syncthreads();
+    cur = nxt;
+    p0 = end >> 1;
+    end = next;
+    next = after;
+  }
+}
+
+// one wide level: positions p0 .. p1, nt terms
+template <int OP>
+__global__ void k_ilu_level(int p0, int p1, int nt, IluArgs A, const int *__restrict__ flags) {
+  if (flags && flags[F_DONE]) return;
+  const int t = p0 + blockIdx.x * kBlock + threadIdx.x;
+  if (t >= p1) return;
+  double v = A.r[t];
+  for (int e = 0; e < nt; ++e) {
+    const size_t q = (size_t)e * A.n + t;
+    const int i = A.src[q];
+    if (i >= 0) v = ilu_term<OP>(v, A.a[q], A.y[i], OP == ILU_DIAG ? A.b[q] : 0.0);
+  }
+  ilu_store<OP>(A, t, v, OP == ILU_DIAG ? 0.0 : A.d[t]);
 }
 
 // One colour of a multicolour Gauss-Seidel sweep: dphi_i = (bc_i - sum
@@ -447,47 +567,18 @@ __global__ void k_bicg_update(int n, double *__restrict__ x, double *__restrict_
 }
 
 // ---- the reference's ILU iteration (ILUMethod.for:4): rc = bc - A dphi with
-// the diagonal first, then level-scheduled forward and backward substitution
-// with the operation order of the sequential loops
+// the diagonal first, into the forward substitution's order (pos), then the
+// two level-scheduled substitutions with the operation order of the
+// sequential loops
 __global__ void k_ilu_resid(int n, int w, const int *__restrict__ nbr, const double *__restrict__ ac,
                             const double *__restrict__ anb, const double *__restrict__ bc,
-                            const double *__restrict__ dphi, double *__restrict__ rc, const int *__restrict__ flags) {
+                            const double *__restrict__ dphi, const int *__restrict__ pos, double *__restrict__ r,
+                            const int *__restrict__ flags) {
   if (flags[F_DONE]) return;
   const int i = xcd_block() * kBlock + threadIdx.x;
   if (i >= n) return;
-  rc[i] = ell_fold<kEllBatch>(i, n, w, nbr, anb, dphi, -ac[i] * dphi[i] + bc[i],
-                              [](double acc, double a, double xk) { return acc - a * xk; });
-}
-
-__global__ void k_ilu_fwd(int cnt, const int *__restrict__ cells, const int *__restrict__ ptr,
-                          const int *__restrict__ lin, const int *__restrict__ src, const double *__restrict__ anb,
-                          const double *__restrict__ dc, double *rc, const int *__restrict__ flags) {
-  if (flags[F_DONE]) return;
-  const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= cnt) return;
-  const int j = cells[t];
-  double v = rc[j];
-  for (int q = ptr[j]; q < ptr[j + 1]; ++q) {
-    const int i = src[q];
-    const double p1 = dc[i] * rc[i];
-    v = v - anb[lin[q]] * p1;
-  }
-  rc[j] = v;
-}
-
-__global__ void k_ilu_bwd(int cnt, const int *__restrict__ cells, const int *__restrict__ ptr,
-                          const int *__restrict__ lin, const int *__restrict__ src, const double *__restrict__ anb,
-                          const double *__restrict__ dc, double *rc, double *__restrict__ dphi,
-                          const int *__restrict__ flags) {
-  if (flags[F_DONE]) return;
-  const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= cnt) return;
-  const int i = cells[t];
-  double v = rc[i];
-  for (int q = ptr[i]; q < ptr[i + 1]; ++q) v = v - anb[lin[q]] * rc[src[q]];
-  const double p1 = dc[i] * v;
-  rc[i] = p1;
-  dphi[i] = dphi[i] + p1;
+  r[pos[i]] = ell_fold<kEllBatch>(i, n, w, nbr, anb, dphi, -ac[i] * dphi[i] + bc[i],
+                                  [](double acc, double a, double xk) { return acc - a * xk; });
 }
 
 // ---- restarted GMRES with right preconditioning (matrixSolverOMP.f90:48 is
@@ -887,13 +978,128 @@ static void precompute_transpose(fs_mesh *m, std::vector<int> &tlin, std::vector
   (void)w;
 }
 
-// Emulates the loops of FactorizeUsingILU.for:29-75 to list, per cell, the
-// terms of its D-ILU diagonal in the order the reference applies them, and
-// groups the cells into dependency levels.
-static void precompute_ilu(fs_mesh *m) {
+// The order of a level-scheduled recurrence and the pieces it is launched in:
+// runs of narrow levels (one workgroup each) and single wide levels.
+struct IluPiece {
+  int p0, p1;      // positions
+  int steps, at;   // a run's step count and where its steps start; steps 0: a wide level
+  int threads;     // of a run's workgroup
+};
+struct IluOrder {
+  int terms = 0;   // most terms of a cell
+  std::vector<IluPiece> pieces;
+  std::vector<int> h_cell, h_pos; // cell of a position, position of a cell
+  const int *cell = nullptr, *pos = nullptr, *steps = nullptr;
+};
+
+// Host integer arrays that go to the device together: one allocation, one
+// copy, one wait.
+struct IntPool {
+  std::vector<int> h;
+  std::vector<std::pair<const int **, size_t>> where;
+  DevBuf<int> d;
+  void put(const std::vector<int> &v, const int **out) {
+    where.push_back({out, h.size()});
+    h.insert(h.end(), v.begin(), v.end());
+  }
+  void upload(hipStream_t s) {
+    if (h.empty()) h.push_back(0);
+    d.upload(h, s);
+    FS_HIP_THROW(hipStreamSynchronize(s)); // h ends here
+    for (auto &w : where) *w.first = d.p + w.second;
+    std::vector<int>().swap(h);
+    where.clear();
+  }
+};
+
+// Sorts the cells by dependency level (src[ptr[i]..] are the cells that cell i
+// waits for; up: higher cells first) and cuts the levels into pieces.
+static void ilu_order(fs_mesh *m, const std::vector<int> &ptr, const std::vector<int> &src, bool up, IluOrder &O,
+                      IntPool &pool) {
+  const int n = m->n;
+  std::vector<int> level(n, 0), level_ptr, cells(n, 0);
+  int maxl = 0;
+  O.terms = 0;
+  for (int q = 0; q < n; ++q) {
+    const int i = up ? n - 1 - q : q; // dependencies are processed first
+    int l = 0;
+    for (int t = ptr[i]; t < ptr[i + 1]; ++t) l = std::max(l, level[src[t]] + 1);
+    level[i] = l;
+    maxl = std::max(maxl, l);
+    O.terms = std::max(O.terms, ptr[i + 1] - ptr[i]);
+  }
+  level_ptr.assign(maxl + 2, 0);
+  for (int i = 0; i < n; ++i) level_ptr[level[i] + 1]++;
+  for (int l = 0; l <= maxl; ++l) level_ptr[l + 1] += level_ptr[l];
+  std::vector<int> fill(level_ptr.begin(), level_ptr.end() - 1), steps;
+  for (int i = 0; i < n; ++i) cells[fill[level[i]]++] = i;
+  O.pieces.clear();
+  for (int l = 0; l <= maxl;) {
+    auto width = [&](int k) { return level_ptr[k + 1] - level_ptr[k]; };
+    IluPiece P{level_ptr[l], level_ptr[l + 1], 0, 0, 0};
+    if (width(l) > kIluNarrow || O.terms > kIluTerms) {
+      ++l;
+    } else {
+      int e = l, widest = 0;
+      for (; e <= maxl && width(e) <= kIluNarrow; ++e) widest = std::max(widest, width(e));
+      P.p1 = level_ptr[e];
+      P.threads = std::min(kIluThreads, (widest + 63) / 64 * 64);
+      P.at = (int)steps.size();
+      steps.push_back(2 * P.p0);
+      for (; l < e; ++l)
+        for (int p = level_ptr[l]; p < level_ptr[l + 1]; p += P.threads) {
+          const int q = std::min(p + P.threads, level_ptr[l + 1]);
+          steps.push_back(2 * q + (q == level_ptr[l + 1] ? 1 : 0));
+        }
+      P.steps = (int)steps.size() - P.at - 1;
+    }
+    O.pieces.push_back(P);
+  }
+  if (steps.empty()) steps.push_back(0);
+  O.h_pos.assign(n, 0);
+  for (int t = 0; t < n; ++t) O.h_pos[cells[t]] = t;
+  O.h_cell = std::move(cells);
+  pool.put(O.h_cell, &O.cell);
+  pool.put(O.h_pos, &O.pos);
+  pool.put(steps, &O.steps);
+}
+
+// terms a position of an order has room for: what its kernel (4, 6 or 8
+// terms, or any number a level at a time) reads
+static int ilu_width(const IluOrder &O) {
+  const int nt = std::max(O.terms, 1);
+  return nt <= 4 ? 4 : nt <= 6 ? 6 : std::max(nt, kIluTerms);
+}
+
+// list[ptr[cell of t] + e] at [e n + t], through map if given; absent terms
+// get `none`
+static void ilu_terms(fs_mesh *m, const IluOrder &O, const std::vector<int> &ptr, const std::vector<int> &list,
+                      const int *map, int none, IntPool &pool, const int **out) {
+  const int n = m->n;
+  std::vector<int> h((size_t)ilu_width(O) * n, none);
+  for (int t = 0; t < n; ++t) {
+    const int c = O.h_cell[t];
+    for (int q = ptr[c]; q < ptr[c + 1]; ++q) h[(size_t)(q - ptr[c]) * n + t] = map ? map[list[q]] : list[q];
+  }
+  pool.put(h, out);
+}
+
+// The schedule of the D-ILU diagonal: emulates the loops of
+// FactorizeUsingILU.for:29-75 to list, per cell, the terms of its diagonal in
+// the order the reference applies them.
+struct IluDiag {
+  bool ready = false;
+  IluOrder order;
+  const int *ta = nullptr, *ti = nullptr, *tb = nullptr; // the terms' anb entries and positions
+  double *a = nullptr, *b = nullptr, *r = nullptr, *y = nullptr; // those entries, ac and the result in the order
+  IntPool ints;
+  DevBuf<double> mem;
+};
+
+static void precompute_ilu(fs_mesh *m, IluDiag &F) {
   const int n = m->n, w = m->w;
   const size_t total = (size_t)n * w;
-  std::vector<std::vector<int>> ta(n), ti(n), tb(n);
+  std::vector<int> to, A0, I0, B0; // the terms as the loops reach them, and their cells
   for (int i1 = 1; i1 <= n; ++i1) {
     if (i1 == n - 1) continue; // FactorizeUsingILU.for:36
     const int i3 = m->h_nnbr[i1 - 1];
@@ -908,40 +1114,36 @@ static void precompute_ilu(fs_mesh *m) {
         i4 = lin < total ? m->h_nbr[lin] : 0;
       }
       if (i4 == i1) {
-        ta[j4 - 1].push_back((i2 - 1) * n + (j4 - 1));
-        ti[j4 - 1].push_back(i1 - 1);
-        tb[j4 - 1].push_back((j2 - 1) * n + (i1 - 1));
+        to.push_back(j4 - 1);
+        A0.push_back((i2 - 1) * n + (j4 - 1));
+        I0.push_back(i1 - 1);
+        B0.push_back((j2 - 1) * n + (i1 - 1));
       }
     }
   }
-  std::vector<int> level(n, 0), ptr(n + 1, 0), A, I, B;
-  int maxl = 0;
-  for (int j = 0; j < n; ++j) {
-    int l = 0;
-    for (int i : ti[j]) l = std::max(l, level[i] + 1);
-    level[j] = l;
-    maxl = std::max(maxl, l);
-    ptr[j + 1] = ptr[j] + (int)ta[j].size();
-    A.insert(A.end(), ta[j].begin(), ta[j].end());
-    I.insert(I.end(), ti[j].begin(), ti[j].end());
-    B.insert(B.end(), tb[j].begin(), tb[j].end());
+  // by cell, each cell's terms in the order reached
+  std::vector<int> ptr(n + 1, 0), A(to.size()), I(to.size()), B(to.size());
+  for (int j : to) ptr[j + 1]++;
+  for (int j = 0; j < n; ++j) ptr[j + 1] += ptr[j];
+  std::vector<int> at(ptr.begin(), ptr.end() - 1);
+  for (size_t q = 0; q < to.size(); ++q) {
+    const int k = at[to[q]]++;
+    A[k] = A0[q];
+    I[k] = I0[q];
+    B[k] = B0[q];
   }
-  m->ilu_nlevels = maxl + 1;
-  m->ilu_level_ptr.assign(maxl + 2, 0);
-  for (int j = 0; j < n; ++j) m->ilu_level_ptr[level[j] + 1]++;
-  for (int l = 0; l <= maxl; ++l) m->ilu_level_ptr[l + 1] += m->ilu_level_ptr[l];
-  std::vector<int> cells(n), fill(m->ilu_level_ptr.begin(), m->ilu_level_ptr.end() - 1);
-  for (int j = 0; j < n; ++j) cells[fill[level[j]]++] = j;
-  if (A.empty()) {
-    A.push_back(0);
-    I.push_back(0);
-    B.push_back(0);
-  }
-  m->d_ilu_cells.upload(cells, m->stream);
-  m->d_ilu_ptr.upload(ptr, m->stream);
-  m->d_ilu_a.upload(A, m->stream);
-  m->d_ilu_i.upload(I, m->stream);
-  m->d_ilu_b.upload(B, m->stream);
+  ilu_order(m, ptr, I, false, F.order, F.ints);
+  ilu_terms(m, F.order, ptr, A, nullptr, 0, F.ints, &F.ta);
+  ilu_terms(m, F.order, ptr, I, F.order.h_pos.data(), -1, F.ints, &F.ti);
+  ilu_terms(m, F.order, ptr, B, nullptr, 0, F.ints, &F.tb);
+  F.ints.upload(m->stream);
+  const size_t nt = (size_t)ilu_width(F.order) * n;
+  F.mem.alloc(2 * nt + 2 * (size_t)n);
+  F.a = F.mem.p;
+  F.b = F.a + nt;
+  F.r = F.b + nt;
+  F.y = F.r + n;
+  F.ready = true;
 }
 
 // Greedy colouring in cell order: each cell takes the smallest colour not
@@ -974,11 +1176,20 @@ void greedy_colors(int n, int w, const int *nbr0, std::vector<int> &ptr, std::ve
 // order, cells grouped in dependency levels.
 struct IluSweep {
   bool ready = false;
-  std::vector<int> fwd_level_ptr, bwd_level_ptr;
-  DevBuf<int> fwd_cells, fwd_ptr, fwd_lin, fwd_src, bwd_cells, bwd_ptr, bwd_lin, bwd_src;
+  struct Half {
+    IluOrder order;
+    const int *src = nullptr, *lin = nullptr; // the terms' positions and anb entries
+    const int *from_diag = nullptr;           // position in the diagonal's order
+    double *a = nullptr, *r = nullptr, *d = nullptr, *y = nullptr; // entries, right-hand side, diagonal, result
+  } fwd, bwd;
+  const int *fwd_of_bwd = nullptr;            // position in the forward order of each backward one
+  double *v = nullptr;                        // the forward result
+  IntPool ints;
+  DevBuf<double> mem;
 };
 
 struct SolveWork {
+  IluDiag diag;
   IluSweep ilu;
   int gm_m = 0;
   DevBuf<double> gm_V, gm_state, gm_part;
@@ -998,26 +1209,7 @@ static SolveWork &work(fs_mesh *m) {
 // anb(j, slot of i) * dc(i) * rc(i) for the lower neighbours i of j, i
 // increasing) and of the backward one (:97-138: rc(i) -= anb(i, j2) * rc(j)
 // for the upper neighbours j of i in slot order), with their levels.
-static void levels_of(int n, const std::vector<int> &ptr, const std::vector<int> &src, bool up,
-                      std::vector<int> &level_ptr, std::vector<int> &cells) {
-  std::vector<int> level(n, 0);
-  int maxl = 0;
-  for (int q = 0; q < n; ++q) {
-    const int i = up ? n - 1 - q : q; // dependencies are processed first
-    int l = 0;
-    for (int t = ptr[i]; t < ptr[i + 1]; ++t) l = std::max(l, level[src[t]] + 1);
-    level[i] = l;
-    maxl = std::max(maxl, l);
-  }
-  level_ptr.assign(maxl + 2, 0);
-  for (int i = 0; i < n; ++i) level_ptr[level[i] + 1]++;
-  for (int l = 0; l <= maxl; ++l) level_ptr[l + 1] += level_ptr[l];
-  cells.assign(n, 0);
-  std::vector<int> fill(level_ptr.begin(), level_ptr.end() - 1);
-  for (int i = 0; i < n; ++i) cells[fill[level[i]]++] = i;
-}
-
-static void precompute_ilu_sweep(fs_mesh *m, IluSweep &S) {
+static void precompute_ilu_sweep(fs_mesh *m, const IluDiag &diag, IluSweep &S) {
   const int n = m->n;
   const std::vector<int> &nb = m->h_nbr, &nn = m->h_nnbr;
   std::vector<std::vector<int>> flin(n), fsrc(n);
@@ -1054,19 +1246,32 @@ static void precompute_ilu_sweep(fs_mesh *m, IluSweep &S) {
       }
     bptr[i1] = (int)bl.size();
   }
-  std::vector<int> fcells, bcells;
-  levels_of(n, fptr, fs, false, S.fwd_level_ptr, fcells);
-  levels_of(n, bptr, bs, true, S.bwd_level_ptr, bcells);
-  for (auto *v : {&fl, &fs, &bl, &bs})
-    if (v->empty()) v->push_back(0);
-  S.fwd_cells.upload(fcells, m->stream);
-  S.fwd_ptr.upload(fptr, m->stream);
-  S.fwd_lin.upload(fl, m->stream);
-  S.fwd_src.upload(fs, m->stream);
-  S.bwd_cells.upload(bcells, m->stream);
-  S.bwd_ptr.upload(bptr, m->stream);
-  S.bwd_lin.upload(bl, m->stream);
-  S.bwd_src.upload(bs, m->stream);
+  auto half = [&](IluSweep::Half &H, const std::vector<int> &ptr, const std::vector<int> &lin,
+                  const std::vector<int> &src, bool up) {
+    ilu_order(m, ptr, src, up, H.order, S.ints);
+    ilu_terms(m, H.order, ptr, src, H.order.h_pos.data(), -1, S.ints, &H.src);
+    ilu_terms(m, H.order, ptr, lin, nullptr, 0, S.ints, &H.lin);
+    std::vector<int> from(n);
+    for (int t = 0; t < n; ++t) from[t] = diag.order.h_pos[H.order.h_cell[t]];
+    S.ints.put(from, &H.from_diag);
+  };
+  half(S.fwd, fptr, fl, fs, false);
+  half(S.bwd, bptr, bl, bs, true);
+  std::vector<int> fb(n);
+  for (int t = 0; t < n; ++t) fb[t] = S.fwd.order.h_pos[S.bwd.order.h_cell[t]];
+  S.ints.put(fb, &S.fwd_of_bwd);
+  S.ints.upload(m->stream);
+  const size_t nf = (size_t)ilu_width(S.fwd.order) * n, nb2 = (size_t)ilu_width(S.bwd.order) * n;
+  S.mem.alloc(nf + nb2 + 7 * (size_t)n);
+  double *at = S.mem.p;
+  for (IluSweep::Half *H : {&S.fwd, &S.bwd}) {
+    H->a = at;
+    H->r = H->a + (H == &S.fwd ? nf : nb2);
+    H->d = H->r + n;
+    H->y = H->d + n;
+    at = H->y + n;
+  }
+  S.v = at;
   S.ready = true;
 }
 
@@ -1077,7 +1282,9 @@ int mesh_prepare_solver(fs_mesh *m) {
   precompute_transpose(m, tlin, tsrc, sw->wt);
   sw->tlin.upload(tlin, m->stream);
   sw->tsrc.upload(tsrc, m->stream);
-  precompute_ilu(m);
+  // the solve without allocation may ask for the D-ILU diagonal; a larger
+  // mesh schedules it with its first PBCG or ILU solve
+  if (m->n <= FS_NOALLOC_MAX_CELLS) precompute_ilu(m, sw->diag);
   std::vector<int> nbr0((size_t)m->n * m->w);
   for (size_t t = 0; t < nbr0.size(); ++t) nbr0[t] = m->h_nbr_dev[t];
   std::vector<int> cells;
@@ -1193,15 +1400,63 @@ void mesh_release_solver(fs_mesh *m) {
   m->solve_work = nullptr;
 }
 
-// D-ILU diagonal on the device (exact reference order).
-static void ilu_factor(fs_mesh *m, const double *ac, const double *anb, double *dc) {
-  for (int l = 0; l < m->ilu_nlevels; ++l) {
-    const int b = m->ilu_level_ptr[l], e = m->ilu_level_ptr[l + 1];
-    if (e > b)
-      hipLaunchKernelGGL(k_ilu_level, dim3(grid_for(e - b)), dim3(kBlock), 0, m->stream, e - b,
-                         m->d_ilu_cells.p + b, m->d_ilu_ptr.p, m->d_ilu_a.p, m->d_ilu_i.p,
-                         m->d_ilu_b.p, ac, anb, dc);
+static void gather(fs_mesh *m, size_t cnt, const int *idx, const double *in, double *out, const int *flags = nullptr) {
+  if (cnt == 0) return;
+  hipLaunchKernelGGL(k_gather, dim3((unsigned)((cnt + kBlock - 1) / kBlock)), dim3(kBlock), 0, m->stream,
+                     (long long)cnt, idx, in, out, flags);
+}
+
+// a recurrence over its order
+template <int OP> static void ilu_pieces(fs_mesh *m, const IluOrder &O, const IluArgs &A, const int *flags) {
+  for (const IluPiece &P : O.pieces) {
+    if (P.steps == 0) {
+      hipLaunchKernelGGL(k_ilu_level<OP>, dim3(grid_for(P.p1 - P.p0)), dim3(kBlock), 0, m->stream, P.p0, P.p1, O.terms,
+                         A, flags);
+      continue;
+    }
+    auto run = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(1), dim3(P.threads), 0, m->stream, P.steps, O.steps + P.at, A,
+                         flags);
+    };
+    if (O.terms <= 4) run(k_ilu_run<OP, 4>);
+    else if (O.terms <= 6) run(k_ilu_run<OP, 6>);
+    else run(k_ilu_run<OP, kIluTerms>);
   }
+}
+
+// D-ILU diagonal on the device (exact reference order), in its schedule's
+// order in F.y and, with dc, in cell order
+static void ilu_factor(fs_mesh *m, const double *ac, const double *anb, double *dc) {
+  IluDiag &F = work(m).diag;
+  if (!F.ready) precompute_ilu(m, F);
+  const IluOrder &O = F.order;
+  const size_t n = m->n, nt = (size_t)O.terms * n;
+  gather(m, nt, F.ta, anb, F.a);
+  gather(m, nt, F.tb, anb, F.b);
+  gather(m, n, O.cell, ac, F.r);
+  ilu_pieces<ILU_DIAG>(m, O, IluArgs{m->n, F.ti, F.a, F.b, F.r, nullptr, F.y, nullptr}, nullptr);
+  if (dc) gather(m, n, O.pos, F.y, dc);
+}
+
+// the matrix and the diagonal in the orders of the two substitutions
+static void ilu_pack(fs_mesh *m, const double *anb) {
+  SolveWork &sw = work(m);
+  for (IluSweep::Half *H : {&sw.ilu.fwd, &sw.ilu.bwd}) {
+    gather(m, (size_t)H->order.terms * m->n, H->lin, anb, H->a);
+    gather(m, m->n, H->from_diag, sw.diag.y, H->d);
+  }
+}
+
+// one ILU iteration from the residual in the forward order (fwd.r):
+// dphi += U^-1 L^-1 r
+static void ilu_apply(fs_mesh *m, double *dphi, const int *flags) {
+  IluSweep &S = work(m).ilu;
+  IluSweep::Half &f = S.fwd, &b = S.bwd;
+  ilu_pieces<ILU_FWD>(m, f.order, IluArgs{m->n, f.src, f.a, nullptr, f.r, f.d, f.y, S.v}, flags);
+  gather(m, m->n, S.fwd_of_bwd, S.v, b.r, flags);
+  ilu_pieces<ILU_BWD>(m, b.order, IluArgs{m->n, b.src, b.a, nullptr, b.r, b.d, b.y, nullptr}, flags);
+  hipLaunchKernelGGL(k_scatter_add, dim3(grid_for(m->n)), dim3(kBlock), 0, m->stream, m->n, b.order.cell, b.y, dphi,
+                     flags);
 }
 
 static void host_flags(fs_mesh *m, int *fl) {
@@ -1613,24 +1868,14 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   } else if (solver == FS_ILU) {
     // the reference's ILU iteration: exact D-ILU diagonal, then per iteration
     // the residual and the two level-scheduled substitutions
-    if (!sw.ilu.ready) precompute_ilu_sweep(m, sw.ilu);
-    ilu_factor(m, ac, anb, m->wk.dc);
+    ilu_factor(m, ac, anb, nullptr);
+    if (!sw.ilu.ready) precompute_ilu_sweep(m, sw.diag, sw.ilu);
+    ilu_pack(m, anb);
     IluSweep &S = sw.ilu;
-    double *rcv = m->wk.v[0];
     iters = run_batches(m, itmax, nf * 8 + solver, [&]() {
-      hipLaunchKernelGGL(k_ilu_resid, dim3(ge), dim3(kBlock), 0, s, n, w, nbr, ac, anb, bc, dphi, rcv, flags);
-      for (size_t l = 0; l + 1 < S.fwd_level_ptr.size(); ++l) {
-        const int b0 = S.fwd_level_ptr[l], b1 = S.fwd_level_ptr[l + 1];
-        if (b1 > b0)
-          hipLaunchKernelGGL(k_ilu_fwd, dim3(grid_for(b1 - b0)), dim3(kBlock), 0, s, b1 - b0, S.fwd_cells.p + b0,
-                             S.fwd_ptr.p, S.fwd_lin.p, S.fwd_src.p, anb, m->wk.dc, rcv, flags);
-      }
-      for (size_t l = 0; l + 1 < S.bwd_level_ptr.size(); ++l) {
-        const int b0 = S.bwd_level_ptr[l], b1 = S.bwd_level_ptr[l + 1];
-        if (b1 > b0)
-          hipLaunchKernelGGL(k_ilu_bwd, dim3(grid_for(b1 - b0)), dim3(kBlock), 0, s, b1 - b0, S.bwd_cells.p + b0,
-                             S.bwd_ptr.p, S.bwd_lin.p, S.bwd_src.p, anb, m->wk.dc, rcv, dphi, flags);
-      }
+      hipLaunchKernelGGL(k_ilu_resid, dim3(ge), dim3(kBlock), 0, s, n, w, nbr, ac, anb, bc, dphi, S.fwd.order.pos,
+                         S.fwd.r, flags);
+      ilu_apply(m, dphi, flags);
       hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, flags);
       hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_CONV, gr, n, nf, part, scal, flags);
     });
