@@ -33,14 +33,23 @@ constexpr int kF = 8;      // input features (4 used, padded)
 constexpr int kIn = 2 * kH; // input width of a message-passing layer
 constexpr int kMaxLayers = 8;
 constexpr int kStatBlocks = 64;
-constexpr int kRowsFwd = 64;   // cells per block of the dense kernels
-constexpr int kChunkW = 256;   // cells per block of the weight-gradient kernel
+constexpr int kTile = 16;      // cells of a matrix-core tile
+constexpr int kTiles = 2;      // tiles a wavefront of the dense kernels works through
+constexpr int kRowsFwd = 4 * kTiles * kTile; // cells per block of the dense kernels
+constexpr int kStage = 64;     // cells the weight-gradient kernel stages at a time
+constexpr int kGradBlocks = 512; // most blocks (partial gradients) of the gradient kernels
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned char u8x4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 inline int cdiv(long long a, int b) { return (int)((a + b - 1) / b); }
+// cells per block of the gradient kernels: 256 fill the chip at 65536 cells;
+// above kGradBlocks blocks the partial gradients (33 KB each) would outgrow
+// the activations, so the blocks take more cells instead
+inline int grad_chunk(long long Bn) { return std::max(256, cdiv(cdiv(Bn, kGradBlocks), kStage) * kStage); }
 
 // float -> bfloat16 bits, round to nearest even (NaN kept quiet)
 __device__ __forceinline__ unsigned short f2bf(float f) {
@@ -90,13 +99,24 @@ __global__ void k_stats(int N, const int *__restrict__ ids, const T *__restrict_
   }
 }
 
-// scal[s] = {s_b, s_a, mean vol, mean x, mean xp}
+// sum over the 64 lanes of a wavefront in a fixed order, valid in lane 0
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  return v;
+}
+
+// scal[s] = {s_b, s_a, mean vol, mean x, mean xp}; one wavefront per sample,
+// nb <= 64 partials, one a lane
 __global__ void k_stats_fin(int N, int nb, const double *__restrict__ part, double *__restrict__ scal) {
-  const int s = blockIdx.x;
-  if (threadIdx.x != 0) return;
-  double a[kStats] = {0, 0, 0, 0, 0};
-  for (int k = 0; k < nb; ++k)
-    for (int q = 0; q < kStats; ++q) a[q] += part[((size_t)s * nb + k) * kStats + q];
+  static_assert(kStatBlocks <= 64, "one partial a lane");
+  const int s = blockIdx.x, k = threadIdx.x;
+  double a[kStats];
+#pragma unroll
+  for (int q = 0; q < kStats; ++q) a[q] = k < nb ? part[((size_t)s * nb + k) * kStats + q] : 0.0;
+#pragma unroll
+  for (int q = 0; q < kStats; ++q) a[q] = wave_sum(a[q]);
+  if (k != 0) return;
   scal[s * kStats + 0] = sqrt(a[0] / N) + 1e-300;
   for (int q = 1; q < kStats; ++q) scal[s * kStats + q] = a[q] / N;
 }
@@ -179,54 +199,67 @@ __global__ void k_agg(int N, int W, int Bn, const int *__restrict__ nbr0, const 
 }
 
 // z = [H M] W + b on the matrix cores; Hn = bf16(H + relu(z)); mask = z > 0.
-// Block: 4 waves, 64 cells; wave w: cells 16w..16w+15 x all 64 outputs
-// (4 tiles of 16x16), K = 128 in 4 steps of 32.
+// The product is formed transposed (rows: the 64 outputs, columns: 16 cells),
+// so that a lane holds four consecutive outputs of one cell and its state,
+// result and mask move 8, 8 and 4 bytes at a time; a wavefront keeps the
+// layer's weights in registers (64) for its kTiles tiles.  65536 cells:
+// 13.9 us (one cell column a lane, 2-byte accesses: 16.4 us).
 __global__ void __launch_bounds__(256)
 k_dense_fwd(int Bn, const unsigned short *__restrict__ H, const unsigned short *__restrict__ M,
             const unsigned short *__restrict__ wt, const float *__restrict__ bias, unsigned short *__restrict__ Hn,
             unsigned char *__restrict__ mask) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int r0 = blockIdx.x * kRowsFwd + wave * 16;
-  const int row = r0 + (lane & 15), kg = lane >> 4;
-  floatx4 acc[4];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, kg = lane >> 4;
+  bf16x8 wv[4][4];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) acc[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    bf16x8 a;
-    if (row < Bn) {
-      const unsigned short *src = ks < 2 ? H + (size_t)row * kH + ks * 32 + kg * 8
-                                         : M + (size_t)row * kH + (ks - 2) * 32 + kg * 8;
-      a = load_bf8(src);
-    } else {
-      a = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
-    }
+    for (int mt = 0; mt < 4; ++mt) wv[ks][mt] = load_bf8(wt + (size_t)(mt * 16 + (lane & 15)) * kIn + ks * 32 + kg * 8);
+  const int c0 = blockIdx.x * kRowsFwd + wave * kTiles * kTile + (lane & 15);
+  bf16x8 xv[kTiles][4];
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int col = nt * 16 + (lane & 15);
-      const bf16x8 bv = load_bf8(wt + (size_t)col * kIn + ks * 32 + kg * 8);
-      acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[nt], 0, 0, 0);
-    }
+  for (int t = 0; t < kTiles; ++t) {
+    const size_t row = (size_t)min(c0 + t * kTile, Bn - 1); // cells past the end repeat the last one
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      xv[t][ks] = load_bf8((ks < 2 ? H + row * kH + ks * 32 : M + row * kH + (ks - 2) * 32) + kg * 8);
   }
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const int col = nt * 16 + (lane & 15);
+  for (int t = 0; t < kTiles; ++t) {
+    const int c = c0 + t * kTile;
+    floatx4 acc[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int rr = r0 + kg * 4 + r;
-      if (rr >= Bn) continue;
-      const float z = acc[nt][r] + bias[col];
-      const size_t at = (size_t)rr * kH + col;
-      Hn[at] = f2bf(bf2f(H[at]) + fmaxf(z, 0.f));
-      mask[at] = z > 0.f;
+    for (int mt = 0; mt < 4; ++mt) acc[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt)
+        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[ks][mt], xv[t][ks], acc[mt], 0, 0, 0);
+    if (c >= Bn) continue;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      const int o = mt * 16 + kg * 4;
+      const size_t at = (size_t)c * kH + o;
+      const floatx4 bo = *reinterpret_cast<const floatx4 *>(bias + o);
+      const u16x4 h = *reinterpret_cast<const u16x4 *>(H + at);
+      u16x4 hn;
+      u8x4 mk;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float z = acc[mt][r] + bo[r];
+        hn[r] = f2bf(bf2f(h[r]) + fmaxf(z, 0.f));
+        mk[r] = z > 0.f;
+      }
+      *reinterpret_cast<u16x4 *>(Hn + at) = hn;
+      *reinterpret_cast<u8x4 *>(mask + at) = mk;
     }
   }
 }
 
 // y = H wd + bd per cell, partial sums of y per (sample, block)
 __global__ void k_decode(int N, int Bn, const unsigned short *__restrict__ H, const float *__restrict__ wdq,
-                         float bd, float *__restrict__ Y, double *__restrict__ part) {
+                         const float *__restrict__ bdp, float *__restrict__ Y, double *__restrict__ part) {
   const int s = blockIdx.y;
+  const float bd = *bdp;
   double acc = 0.0;
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < N; i += gridDim.x * kBlock) {
     const int c = s * N + i;
@@ -243,13 +276,11 @@ __global__ void k_decode(int N, int Bn, const unsigned short *__restrict__ H, co
   (void)Bn;
 }
 
-// ymean[s] from the partials
+// ymean[s] from the partials, one a lane
 __global__ void k_mean_fin(int N, int nb, const double *__restrict__ part, double *__restrict__ ymean) {
-  if (threadIdx.x != 0) return;
-  const int s = blockIdx.x;
-  double a = 0.0;
-  for (int k = 0; k < nb; ++k) a += part[(size_t)s * nb + k];
-  ymean[s] = a / N;
+  const int s = blockIdx.x, k = threadIdx.x;
+  const double a = wave_sum(k < nb ? part[(size_t)s * nb + k] : 0.0);
+  if (k == 0) ymean[s] = a / N;
 }
 
 // yc = y - mean; loss partials and dy = 2 (yc - t)/total (training), or the
@@ -279,151 +310,209 @@ __global__ void k_loss(int N, const double *__restrict__ ymean, const double *__
 }
 
 // ---------------------------------------------------------------- backward
-// dH[c][o] = dy[c] wd[o]
-__global__ void k_dec_bwd(int Bn, const float *__restrict__ DY, const float *__restrict__ wdq, float *__restrict__ dH) {
-  const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (t >= (long long)Bn * kH) return;
-  const int c = (int)(t >> 6), o = (int)(t & 63);
-  dH[t] = DY[c] * wdq[o];
+// four of a row's activation gradients and, with mask, the layer's dz =
+// bf16(mask ? dH : 0) formed from them
+__device__ __forceinline__ void store_dh(size_t at, floatx4 d, float *__restrict__ dH,
+                                         const unsigned char *__restrict__ mask, unsigned short *__restrict__ DZ) {
+  *reinterpret_cast<floatx4 *>(dH + at) = d;
+  if (!mask) return;
+  const u8x4 m = *reinterpret_cast<const u8x4 *>(mask + at);
+  u16x4 z;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) z[q] = f2bf(m[q] ? d[q] : 0.f);
+  *reinterpret_cast<u16x4 *>(DZ + at) = z;
 }
 
-// Per-block column sums: out[blk][o] = sum over the block's cells of
-// a[c] * V[c][o] (a = null: 1), V as BF16 (Vb) or FP32 (Vf); out[blk][64] =
-// sum of a[c] when a is given.  Block: 256 threads = 4 cell lanes x 64 columns.
-__global__ void k_colsum(int Bn, int chunk, const float *__restrict__ a, const unsigned short *__restrict__ Vb,
-                         const float *__restrict__ Vf, float *__restrict__ out) {
+// dH[c][o] = dy[c] wd[o], and dz of the last layer; thread per (cell, 4 outputs)
+__global__ void k_dec_bwd(int Bn, const float *__restrict__ DY, const float *__restrict__ wdq, float *__restrict__ dH,
+                          const unsigned char *__restrict__ mask, unsigned short *__restrict__ DZ) {
+  const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
+  const int c = (int)(t >> 4), o = (int)(t & 15) * 4;
+  if (c >= Bn) return;
+  const float dy = DY[c];
+  floatx4 d;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) d[q] = dy * wdq[o + q];
+  store_dh((size_t)c * kH + o, d, dH, mask, DZ);
+}
+
+// Decoder gradient: per-block sums out[blk][o] = sum of dy[c] H[c][o] over the
+// block's cells, out[blk][64] = sum of dy[c].  Block: 256 threads = 4 cell
+// lanes x 64 columns, the loads of 8 cells in flight.
+__global__ void k_dec_grad(int Bn, int chunk, const float *__restrict__ DY, const unsigned short *__restrict__ H,
+                           float *__restrict__ out) {
   const int o = threadIdx.x & 63, r = threadIdx.x >> 6;
   const int c0 = blockIdx.x * chunk, c1 = min(Bn, c0 + chunk);
   float s = 0.f, sa = 0.f;
-  for (int c = c0 + r; c < c1; c += 4) {
-    const float v = Vb ? bf2f(Vb[(size_t)c * kH + o]) : Vf[(size_t)c * kH + o];
-    const float w = a ? a[c] : 1.f;
-    s += w * v;
-    if (o == 0 && a) sa += w;
+  constexpr int B = 8;
+  for (int cb = c0 + r; cb < c1; cb += 4 * B) {
+    float dy[B], h[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int c = min(cb + 4 * u, c1 - 1);
+      dy[u] = DY[c];
+      h[u] = bf2f(H[(size_t)c * kH + o]);
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (cb + 4 * u < c1) {
+        s += dy[u] * h[u];
+        sa += dy[u];
+      }
   }
   __shared__ float red[4][kH + 1];
   red[r][o] = s;
   if (o == 0) red[r][kH] = sa;
   __syncthreads();
-  if (r == 0) {
-    out[(size_t)blockIdx.x * (kH + 1) + o] = red[0][o] + red[1][o] + red[2][o] + red[3][o];
-    if (o == 0) out[(size_t)blockIdx.x * (kH + 1) + kH] = red[0][kH] + red[1][kH] + red[2][kH] + red[3][kH];
-  }
+  for (int k = threadIdx.x; k <= kH; k += 256)
+    out[(size_t)blockIdx.x * (kH + 1) + k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
 }
 
-// dz = bf16(mask ? dH : 0)
-__global__ void k_relu_bwd(int Bn, const float *__restrict__ dH, const unsigned char *__restrict__ mask,
-                           unsigned short *__restrict__ DZ) {
-  const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (t >= (long long)Bn * kH) return;
-  DZ[t] = f2bf(mask[t] ? dH[t] : 0.f);
-}
-
-// D = dz W^T on the matrix cores: [Bn x 64] x [64 x 128] -> FP32 [Bn x 128].
-// Wave: 16 cells x 128 columns (8 tiles), K = 64 in 2 steps.
+// D = dz W^T on the matrix cores: [Bn x 64] x [64 x 128] -> FP32 [Bn x 128],
+// formed transposed like k_dense_fwd (16-byte stores; 65536 cells: 12.6 us,
+// 14.9 us with 4-byte stores and the weights loaded for every tile).
 __global__ void __launch_bounds__(256)
 k_dense_bwd_x(int Bn, const unsigned short *__restrict__ DZ, const unsigned short *__restrict__ wb,
               float *__restrict__ D) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int r0 = blockIdx.x * kRowsFwd + wave * 16;
-  const int row = r0 + (lane & 15), kg = lane >> 4;
-  floatx4 acc[8];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, kg = lane >> 4;
+  bf16x8 wv[2][8];
 #pragma unroll
-  for (int nt = 0; nt < 8; ++nt) acc[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const bf16x8 a = row < Bn ? load_bf8(DZ + (size_t)row * kH + ks * 32 + kg * 8)
-                              : __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
+    for (int mt = 0; mt < 8; ++mt) wv[ks][mt] = load_bf8(wb + (size_t)(mt * 16 + (lane & 15)) * kH + ks * 32 + kg * 8);
+  const int c0 = blockIdx.x * kRowsFwd + wave * kTiles * kTile + (lane & 15);
+  bf16x8 zv[kTiles][2];
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-      const int col = nt * 16 + (lane & 15); // input feature
-      const bf16x8 bv = load_bf8(wb + (size_t)col * kH + ks * 32 + kg * 8);
-      acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[nt], 0, 0, 0);
-    }
+  for (int t = 0; t < kTiles; ++t) {
+    const size_t row = (size_t)min(c0 + t * kTile, Bn - 1);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) zv[t][ks] = load_bf8(DZ + row * kH + ks * 32 + kg * 8);
   }
 #pragma unroll
-  for (int nt = 0; nt < 8; ++nt) {
-    const int col = nt * 16 + (lane & 15);
+  for (int t = 0; t < kTiles; ++t) {
+    const int c = c0 + t * kTile;
+    floatx4 acc[8];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int rr = r0 + kg * 4 + r;
-      if (rr < Bn) D[(size_t)rr * kIn + col] = acc[nt][r];
-    }
+    for (int mt = 0; mt < 8; ++mt) acc[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt)
+        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[ks][mt], zv[t][ks], acc[mt], 0, 0, 0);
+    if (c >= Bn) continue;
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt)
+      *reinterpret_cast<floatx4 *>(D + (size_t)c * kIn + mt * 16 + kg * 4) = acc[mt];
   }
 }
 
 // dH_prev[c] = dH[c] + D[c][0:64] + sum over neighbours k of c of
 // e_{k,c} D[k][64:128] (the transpose of the aggregation; e_{k,c} is the
-// weight of c in k's row, found through the mirror slot)
+// weight of c in k's row, found through the mirror slot), and dz of the layer
+// below (mask, DZ; none below the first)
 __global__ void k_agg_t(int N, int W, int Bn, const int *__restrict__ nbr0, const int *__restrict__ mir,
                         const float *__restrict__ E, const float *__restrict__ dH, const float *__restrict__ D,
-                        float *__restrict__ dHp) {
+                        float *__restrict__ dHp, const unsigned char *__restrict__ mask,
+                        unsigned short *__restrict__ DZ) {
   const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
-  const int c = (int)(t >> 3), g = (int)(t & 7);
+  const int c = (int)(t >> 4), g = (int)(t & 15) * 4;
   if (c >= Bn) return;
   const int s = c / N, i = c - s * N;
-  float acc[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) acc[q] = dH[(size_t)c * kH + g * 8 + q] + D[(size_t)c * kIn + g * 8 + q];
+  const floatx4 h = *reinterpret_cast<const floatx4 *>(dH + (size_t)c * kH + g);
+  floatx4 acc = h + *reinterpret_cast<const floatx4 *>(D + (size_t)c * kIn + g);
   for (int j = 0; j < W; ++j) {
     const int k = nbr0[(size_t)j * N + i];
     if (k < 0) continue;
     const int jm = mir[(size_t)j * N + i];
     const size_t ck = (size_t)s * N + k;
     const float e = E[(size_t)jm * Bn + ck];
-    const float *dk = D + ck * kIn + kH + g * 8;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) acc[q] += e * dk[q];
+    acc += e * *reinterpret_cast<const floatx4 *>(D + ck * kIn + kH + g);
   }
-#pragma unroll
-  for (int q = 0; q < 8; ++q) dHp[(size_t)c * kH + g * 8 + q] = acc[q];
+  store_dh((size_t)c * kH + g, acc, dHp, mask, DZ);
 }
 
-// Partial dW = [H M]^T dz over the block's cells on the matrix cores.  The
-// block stages 32 cells at a time transposed in LDS (feature-major, K =
-// cells contiguous); wave w owns the 2 x 4 output tiles of input features
-// 32w..32w+31.  out[blk][in][o], FP32.
-constexpr int kStageCells = 32;
-constexpr int kStageStride = kStageCells + 8; // bf16 elements per staged row
+// Partial dW = [H M]^T dz and db = column sums of dz over the block's cells,
+// out[blk] = {dW[in][o], db[o]}, FP32.  The matrix cores contract over cells,
+// so both operands are needed feature-major: the block stages kStage cells at
+// a time in LDS, each thread transposing one 8 cells x 8 features tile in
+// registers (16-byte loads and LDS stores; the next stage's loads are in
+// flight behind the products).  Wave w owns input features 32w..32w+31 (2 x 4
+// output tiles).  65536 cells: 9.4 us (2-byte staging of 32 cells: 53.6 us,
+// and another 20 us for the column sums).
+constexpr int kStageStride = kStage + 8; // bf16 elements per staged row: 16-byte rows, spread over the banks
+constexpr int kGradW = kIn * kH + kH;    // values of a layer's gradient (W, b)
+
 __global__ void __launch_bounds__(256)
-k_dense_bwd_w(int Bn, const unsigned short *__restrict__ H, const unsigned short *__restrict__ M,
+k_dense_bwd_w(int Bn, int chunk, const unsigned short *__restrict__ H, const unsigned short *__restrict__ M,
               const unsigned short *__restrict__ DZ, float *__restrict__ out) {
-  __shared__ __attribute__((aligned(16))) unsigned short xs[kIn * kStageStride];
-  __shared__ __attribute__((aligned(16))) unsigned short zs[kH * kStageStride];
+  __shared__ __attribute__((aligned(16))) unsigned short st[(kIn + kH) * kStageStride];
+  __shared__ float bred[4][kH];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, kg = lane >> 4;
-  const int c0 = blockIdx.x * kChunkW;
+  const int c0 = blockIdx.x * chunk, c1 = min(Bn, c0 + chunk);
+  // the thread's tile: cells 8 cg.., feature group fg of [H | M | dz]
+  const int cg = threadIdx.x & 7, fg = threadIdx.x >> 3;
+  const bool loads = fg < (kIn + kH) / 8;
+  const unsigned short *src = fg < 8 ? H + fg * 8 : fg < 16 ? M + (fg - 8) * 8 : DZ + (fg - 16) * 8;
+  uint4 w[8];
+  auto fetch = [&](int cs) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int c = cs + cg * 8 + r;
+      w[r] = uint4{0u, 0u, 0u, 0u};
+      if (loads && c < c1) w[r] = *reinterpret_cast<const uint4 *>(src + (size_t)c * kH);
+    }
+  };
   floatx4 acc[2][4];
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (int cs = c0; cs < c0 + kChunkW; cs += kStageCells) {
-    __syncthreads();
-    // stage: xs[f][cell] for f < 128, zs[o][cell]; zeros past Bn
-    for (int e = threadIdx.x; e < kStageCells * kIn; e += blockDim.x) {
-      const int cl = e / kIn, f = e - cl * kIn, c = cs + cl;
-      unsigned short v = 0;
-      if (c < Bn) v = f < kH ? H[(size_t)c * kH + f] : M[(size_t)c * kH + f - kH];
-      xs[f * kStageStride + cl] = v;
-    }
-    for (int e = threadIdx.x; e < kStageCells * kH; e += blockDim.x) {
-      const int cl = e / kH, o = e - cl * kH, c = cs + cl;
-      zs[o * kStageStride + cl] = c < Bn ? DZ[(size_t)c * kH + o] : (unsigned short)0;
-    }
-    __syncthreads();
+  float bs = 0.f;
+  fetch(c0);
+  for (int cs = c0; cs < c1; cs += kStage) {
+    __syncthreads(); // the last stage has been read
+    if (loads) {
+      auto word = [&](int r, int q) { return q == 0 ? w[r].x : q == 1 ? w[r].y : q == 2 ? w[r].z : w[r].w; };
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      const int f = wave * 32 + mt * 16 + (lane & 15);
-      const bf16x8 a = load_bf8(xs + f * kStageStride + kg * 8);
+      for (int q = 0; q < 4; ++q) {
+        unsigned lo[4], hi[4];
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const int o = nt * 16 + (lane & 15);
-        const bf16x8 bv = load_bf8(zs + o * kStageStride + kg * 8);
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[mt][nt], 0, 0, 0);
+        for (int k = 0; k < 4; ++k) {
+          const unsigned a = word(2 * k, q), b = word(2 * k + 1, q);
+          lo[k] = (a & 0xffffu) | (b << 16);
+          hi[k] = (a >> 16) | (b & 0xffff0000u);
+        }
+        unsigned short *dst = st + (size_t)(fg * 8 + 2 * q) * kStageStride + cg * 8;
+        *reinterpret_cast<uint4 *>(dst) = uint4{lo[0], lo[1], lo[2], lo[3]};
+        *reinterpret_cast<uint4 *>(dst + kStageStride) = uint4{hi[0], hi[1], hi[2], hi[3]};
       }
     }
+    __syncthreads();
+    if (cs + kStage < c1) fetch(cs + kStage);
+    const unsigned short *zs = st + (size_t)kIn * kStageStride;
+#pragma unroll
+    for (int ks = 0; ks < kStage / 32; ++ks) {
+      bf16x8 bv[4];
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) bv[nt] = load_bf8(zs + (nt * 16 + (lane & 15)) * kStageStride + ks * 32 + kg * 8);
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+        const bf16x8 a = load_bf8(st + (wave * 32 + mt * 16 + (lane & 15)) * kStageStride + ks * 32 + kg * 8);
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv[nt], acc[mt][nt], 0, 0, 0);
+      }
+    }
+    // column sums: lane o, a quarter of the stage's cells per wave
+#pragma unroll
+    for (int k = 0; k < kStage / 32; ++k) {
+      const u16x8 z = *reinterpret_cast<const u16x8 *>(zs + lane * kStageStride + wave * (kStage / 4) + k * 8);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) bs += bf2f(z[q]);
+    }
   }
-  float *dst = out + (size_t)blockIdx.x * kIn * kH;
+  bred[wave][lane] = bs;
+  __syncthreads();
+  float *dst = out + (size_t)blockIdx.x * kGradW;
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -435,6 +524,9 @@ k_dense_bwd_w(int Bn, const unsigned short *__restrict__ H, const unsigned short
         dst[f * kH + o] = acc[mt][nt][r];
       }
     }
+  if (threadIdx.x < kH)
+    dst[kIn * kH + threadIdx.x] =
+        bred[0][threadIdx.x] + bred[1][threadIdx.x] + bred[2][threadIdx.x] + bred[3][threadIdx.x];
 }
 
 // encoder gradient partials: out[blk][f][o] = sum X0[c][f] dz0[c][o] (f < 8),
@@ -443,14 +535,31 @@ __global__ void k_enc_bwd(int Bn, int chunk, const float *__restrict__ X0, const
                           const float *__restrict__ dH, float *__restrict__ out) {
   const int o = threadIdx.x & 63, r = threadIdx.x >> 6;
   const int c0 = blockIdx.x * chunk, c1 = min(Bn, c0 + chunk);
+  static_assert(kF == 8, "features in two 16-byte loads");
   float s[kF + 1];
 #pragma unroll
   for (int f = 0; f <= kF; ++f) s[f] = 0.f;
-  for (int c = c0 + r; c < c1; c += 4) {
-    const float dz = bf2f(H0[(size_t)c * kH + o]) > 0.f ? dH[(size_t)c * kH + o] : 0.f;
+  constexpr int B = 8; // cells in flight
+  for (int cb = c0 + r; cb < c1; cb += 4 * B) {
+    float dz[B];
+    floatx4 xa[B], xb[B];
 #pragma unroll
-    for (int f = 0; f < kF; ++f) s[f] += X0[(size_t)c * kF + f] * dz;
-    s[kF] += dz;
+    for (int u = 0; u < B; ++u) {
+      const size_t c = (size_t)min(cb + 4 * u, c1 - 1);
+      const float h = bf2f(H0[c * kH + o]), d = dH[c * kH + o];
+      dz[u] = h > 0.f && cb + 4 * u < c1 ? d : 0.f;
+      xa[u] = *reinterpret_cast<const floatx4 *>(X0 + c * kF);
+      xb[u] = *reinterpret_cast<const floatx4 *>(X0 + c * kF + 4);
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        s[f] += xa[u][f] * dz[u];
+        s[4 + f] += xb[u][f] * dz[u];
+      }
+      s[kF] += dz[u];
+    }
   }
   __shared__ float red[4][kF + 1][kH];
 #pragma unroll
@@ -461,23 +570,30 @@ __global__ void k_enc_bwd(int Bn, int chunk, const float *__restrict__ X0, const
       out[((size_t)blockIdx.x * (kF + 1) + f) * kH + o] = red[0][f][o] + red[1][f][o] + red[2][f][o] + red[3][f][o];
 }
 
-// dst[k] = sum over blocks b (in order) of part[b][k], k < K
+// dst[k] = sum over the nb blocks' partials part[b][k], k < K.  A block sums 32
+// columns with 8 row groups (rows g, g + 8, ... in order, 8 loads in flight),
+// the groups combined in order: 4-8 us for 256 x 8256 values (one thread a
+// column over all rows: 60 us, and as much for each bias).
 __global__ void k_reduce(int nb, int K, const float *__restrict__ part, float *__restrict__ dst) {
-  const int k = blockIdx.x * kBlock + threadIdx.x;
-  if (k >= K) return;
+  constexpr int C = 32, G = kBlock / C, B = 8;
+  const int kk = threadIdx.x % C, g = threadIdx.x / C, k = blockIdx.x * C + kk;
   float s = 0.f;
-  for (int b = 0; b < nb; ++b) s += part[(size_t)b * K + k];
-  dst[k] = s;
-}
-
-// the bias and wd gradients from k_colsum partials (nb blocks of 65)
-__global__ void k_reduce_cols(int nb, const float *__restrict__ part, float *__restrict__ dcol, float *__restrict__ dscalar) {
-  const int o = threadIdx.x;
-  if (o > kH) return;
-  float s = 0.f;
-  for (int b = 0; b < nb; ++b) s += part[(size_t)b * (kH + 1) + o];
-  if (o < kH) dcol[o] = s;
-  else if (dscalar) *dscalar = s;
+  for (int b0 = g; b0 < nb; b0 += G * B) {
+    float v[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) v[u] = k < K && b0 + u * G < nb ? part[(size_t)(b0 + u * G) * K + k] : 0.f;
+#pragma unroll
+    for (int u = 0; u < B; ++u) s += v[u];
+  }
+  __shared__ float red[G][C];
+  red[g][kk] = s;
+  __syncthreads();
+  if (g == 0 && k < K) {
+    float t = 0.f;
+#pragma unroll
+    for (int u = 0; u < G; ++u) t += red[u][kk];
+    dst[k] = t;
+  }
 }
 
 __global__ void k_adam(int n, float *__restrict__ th, const float *__restrict__ g, float *__restrict__ m,
@@ -560,8 +676,7 @@ static void mpnn_grow(fs_mpnn *n, int B) {
   for (auto &h : n->Hs) h.alloc(Bn * kH);
   for (auto &m : n->Ms) m.alloc(Bn * kH);
   for (auto &m : n->masks) m.alloc(Bn * kH);
-  const size_t nbw = cdiv(Bn, kChunkW);
-  n->gpart.alloc(std::max(nbw * kIn * kH, nbw * (kF + 1) * kH));
+  n->gpart.alloc((size_t)cdiv(Bn, grad_chunk(Bn)) * kGradW);
   n->bn_cap = Bn;
 }
 
@@ -574,7 +689,7 @@ static void quantize(fs_mpnn *n) {
 // number of stat blocks per sample.
 template <class T>
 static void mpnn_forward(fs_mpnn *n, int B, const T *b, const T *ac, const T *anb, const T *vol, const T *x,
-                         const T *xp, float bd) {
+                         const T *xp) {
   hipStream_t s = n->s;
   const int N = n->N, W = n->W;
   const int Bn = B * N;
@@ -593,70 +708,60 @@ static void mpnn_forward(fs_mpnn *n, int B, const T *b, const T *ac, const T *an
                        n->wt.p + (size_t)l * kIn * kH, n->theta.p + mpnn_offset_W(l) + kIn * kH, n->Hs[l + 1].p,
                        n->masks[l].p);
   }
-  hipLaunchKernelGGL(k_decode, dim3(nb, B), dim3(kBlock), 0, s, N, Bn, n->Hs[n->L].p, n->wdq.p, bd, n->Y.p,
-                     n->part.p);
+  hipLaunchKernelGGL(k_decode, dim3(nb, B), dim3(kBlock), 0, s, N, Bn, n->Hs[n->L].p, n->wdq.p,
+                     n->theta.p + n->P - 1, n->Y.p, n->part.p);
   hipLaunchKernelGGL(k_mean_fin, dim3(B), dim3(64), 0, s, N, nb, n->part.p, n->ymean.p);
 }
 
-static float host_bd(fs_mpnn *n) {
-  float bd = 0.f;
-  FS_HIP_THROW(hipMemcpyAsync(&bd, n->theta.p + n->P - 1, sizeof(float), hipMemcpyDeviceToHost, n->s));
-  FS_HIP_THROW(hipStreamSynchronize(n->s));
-  return bd;
-}
-
-// loss (and gradient into n->grad when want_grad)
-static double mpnn_loss_grad(fs_mpnn *n, const int *ids, int B, bool want_grad) {
+// The batch's loss partials and, with want_grad, the gradient into n->grad, on
+// the network's stream.
+static void mpnn_loss_grad(fs_mpnn *n, const int *ids, int B, bool want_grad) {
   hipStream_t s = n->s;
   for (int k = 0; k < B; ++k)
     if (ids[k] < 0 || ids[k] >= n->count) throw std::runtime_error("sample id out of range");
   mpnn_grow(n, B);
   FS_HIP_THROW(hipMemcpyAsync(n->ids.p, ids, sizeof(int) * B, hipMemcpyHostToDevice, s));
   const int N = n->N, Bn = B * N;
-  const float bd = host_bd(n);
-  mpnn_forward<float>(n, B, n->ds_b.p, n->ds_ac.p, n->ds_anb.p, n->ds_vol.p, n->ds_x.p, n->ds_xp.p, bd);
+  mpnn_forward<float>(n, B, n->ds_b.p, n->ds_ac.p, n->ds_anb.p, n->ds_vol.p, n->ds_x.p, n->ds_xp.p);
   const int nb = std::min(kStatBlocks, cdiv(N, kBlock));
   hipLaunchKernelGGL(k_loss, dim3(nb, B), dim3(kBlock), 0, s, N, n->ymean.p, n->scal.p, n->Y.p, n->Tg.p, n->DY.p,
                      1.0 / Bn, n->part.p, (double *)nullptr);
-  n->h_part.resize((size_t)B * nb);
-  FS_HIP_THROW(hipMemcpyAsync(n->h_part.data(), n->part.p, sizeof(double) * B * nb, hipMemcpyDeviceToHost, s));
-  if (want_grad) {
-    const int L = n->L;
-    float *g = n->grad.p;
-    // decoder
-    const int nbc = cdiv(Bn, kChunkW);
-    hipLaunchKernelGGL(k_colsum, dim3(nbc), dim3(256), 0, s, Bn, kChunkW, n->DY.p, n->Hs[L].p, (const float *)nullptr,
+  if (!want_grad) return;
+  const int L = n->L, chunk = grad_chunk(Bn), nbc = cdiv(Bn, chunk);
+  float *g = n->grad.p;
+  auto reduce = [&](int K, float *dst) {
+    hipLaunchKernelGGL(k_reduce, dim3(cdiv(K, 32)), dim3(kBlock), 0, s, nbc, K, n->gpart.p, dst);
+  };
+  // decoder (wd and bd are the last parameters)
+  hipLaunchKernelGGL(k_dec_grad, dim3(nbc), dim3(256), 0, s, Bn, chunk, n->DY.p, n->Hs[L].p, n->gpart.p);
+  reduce(kH + 1, g + mpnn_offset_W(L));
+  const unsigned quads = cdiv((long long)Bn * (kH / 4), kBlock);
+  hipLaunchKernelGGL(k_dec_bwd, dim3(quads), dim3(kBlock), 0, s, Bn, n->DY.p, n->wdq.p, n->dH.p, n->masks[L - 1].p,
+                     n->DZ.p);
+  float *dH = n->dH.p, *dH2 = n->dH2.p;
+  for (int l = L - 1; l >= 0; --l) {
+    hipLaunchKernelGGL(k_dense_bwd_w, dim3(nbc), dim3(256), 0, s, Bn, chunk, n->Hs[l].p, n->Ms[l].p, n->DZ.p,
                        n->gpart.p);
-    hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(128), 0, s, nbc, n->gpart.p, g + mpnn_offset_W(L),
-                       g + n->P - 1);
-    hipLaunchKernelGGL(k_dec_bwd, dim3(cdiv((long long)Bn * kH, kBlock)), dim3(kBlock), 0, s, Bn, n->DY.p, n->wdq.p,
-                       n->dH.p);
-    float *dH = n->dH.p, *dH2 = n->dH2.p;
-    for (int l = L - 1; l >= 0; --l) {
-      hipLaunchKernelGGL(k_relu_bwd, dim3(cdiv((long long)Bn * kH, kBlock)), dim3(kBlock), 0, s, Bn, dH,
-                         n->masks[l].p, n->DZ.p);
-      hipLaunchKernelGGL(k_colsum, dim3(nbc), dim3(256), 0, s, Bn, kChunkW, (const float *)nullptr, n->DZ.p,
-                         (const float *)nullptr, n->gpart.p);
-      hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(128), 0, s, nbc, n->gpart.p,
-                         g + mpnn_offset_W(l) + kIn * kH, (float *)nullptr);
-      hipLaunchKernelGGL(k_dense_bwd_w, dim3(nbc), dim3(256), 0, s, Bn, n->Hs[l].p, n->Ms[l].p, n->DZ.p,
-                         n->gpart.p);
-      hipLaunchKernelGGL(k_reduce, dim3(cdiv(kIn * kH, kBlock)), dim3(kBlock), 0, s, nbc, kIn * kH, n->gpart.p,
-                         g + mpnn_offset_W(l));
-      hipLaunchKernelGGL(k_dense_bwd_x, dim3(cdiv(Bn, kRowsFwd)), dim3(256), 0, s, Bn, n->DZ.p,
-                         n->wb.p + (size_t)l * kIn * kH, n->D.p);
-      hipLaunchKernelGGL(k_agg_t, dim3(cdiv((long long)Bn * 8, kBlock)), dim3(kBlock), 0, s, N, n->W, Bn, n->nbr0.p,
-                         n->mir.p, n->E.p, dH, n->D.p, dH2);
-      std::swap(dH, dH2);
-    }
-    hipLaunchKernelGGL(k_enc_bwd, dim3(nbc), dim3(256), 0, s, Bn, kChunkW, n->X0.p, n->Hs[0].p, dH, n->gpart.p);
-    hipLaunchKernelGGL(k_reduce, dim3(cdiv((kF + 1) * kH, kBlock)), dim3(kBlock), 0, s, nbc, (kF + 1) * kH,
-                       n->gpart.p, g);
+    reduce(kGradW, g + mpnn_offset_W(l));
+    hipLaunchKernelGGL(k_dense_bwd_x, dim3(cdiv(Bn, kRowsFwd)), dim3(256), 0, s, Bn, n->DZ.p,
+                       n->wb.p + (size_t)l * kIn * kH, n->D.p);
+    hipLaunchKernelGGL(k_agg_t, dim3(quads), dim3(kBlock), 0, s, N, n->W, Bn, n->nbr0.p, n->mir.p, n->E.p, dH, n->D.p,
+                       dH2, l > 0 ? n->masks[l - 1].p : nullptr, n->DZ.p);
+    std::swap(dH, dH2);
   }
-  FS_HIP_THROW(hipStreamSynchronize(s));
+  hipLaunchKernelGGL(k_enc_bwd, dim3(nbc), dim3(256), 0, s, Bn, chunk, n->X0.p, n->Hs[0].p, dH, n->gpart.p);
+  reduce((kF + 1) * kH, g);
+}
+
+// The loss of the batch just evaluated; waits for the stream.
+static double mpnn_loss(fs_mpnn *n, int B) {
+  const int nb = std::min(kStatBlocks, cdiv(n->N, kBlock));
+  n->h_part.resize((size_t)B * nb);
+  FS_HIP_THROW(hipMemcpyAsync(n->h_part.data(), n->part.p, sizeof(double) * B * nb, hipMemcpyDeviceToHost, n->s));
+  FS_HIP_THROW(hipStreamSynchronize(n->s));
   double loss = 0.0;
   for (double v : n->h_part) loss += v;
-  return loss / Bn;
+  return loss / ((double)B * n->N);
 }
 
 } // namespace fs
@@ -858,7 +963,8 @@ int fs_mpnn_loss_grad(fs_mpnn *n, const int *ids, int batch, double *loss, doubl
     set_error("fs_mpnn_loss_grad: invalid arguments");
     return -1;
   }
-  *loss = fs::mpnn_loss_grad(n, ids, batch, grad != nullptr);
+  fs::mpnn_loss_grad(n, ids, batch, grad != nullptr);
+  *loss = fs::mpnn_loss(n, batch);
   if (grad) {
     std::vector<float> h(n->P);
     FS_HIP(hipMemcpyAsync(h.data(), n->grad.p, sizeof(float) * n->P, hipMemcpyDeviceToHost, n->s));
@@ -875,14 +981,14 @@ int fs_mpnn_train_step(fs_mpnn *n, const int *ids, int batch, double lr, double 
     set_error("fs_mpnn_train_step: invalid arguments");
     return -1;
   }
-  const double l = fs::mpnn_loss_grad(n, ids, batch, true);
-  if (loss) *loss = l;
+  fs::mpnn_loss_grad(n, ids, batch, true);
   n->steps++;
   const float c1 = 1.f - std::pow(0.9f, (float)n->steps), c2 = 1.f - std::pow(0.999f, (float)n->steps);
   hipLaunchKernelGGL(fs::k_adam, dim3(fs::cdiv(n->P, fs::kBlock)), dim3(fs::kBlock), 0, n->s, n->P, n->theta.p,
                      n->grad.p, n->am.p, n->av.p, (float)lr, c1, c2);
   fs::quantize(n);
-  FS_HIP(hipStreamSynchronize(n->s));
+  const double l = fs::mpnn_loss(n, batch); // the step's only wait
+  if (loss) *loss = l;
   return 0;
   MPNN_GUARD_END
 }
@@ -923,8 +1029,7 @@ int mpnn_predict_device(fs_mpnn *n, hipStream_t stream, const double *b, const d
     mpnn_grow(n, 1);
     const int zero = 0;
     FS_HIP_THROW(hipMemcpyAsync(n->ids.p, &zero, sizeof(int), hipMemcpyHostToDevice, stream));
-    const float bd = host_bd(n);
-    mpnn_forward<double>(n, 1, b, ac, anb, vol, (const double *)nullptr, xp, bd);
+    mpnn_forward<double>(n, 1, b, ac, anb, vol, (const double *)nullptr, xp);
     const int nb = std::min(kStatBlocks, cdiv(n->N, kBlock));
     hipLaunchKernelGGL(k_loss, dim3(nb, 1), dim3(kBlock), 0, stream, n->N, n->ymean.p, n->scal.p, n->Y.p,
                        (const float *)nullptr, (float *)nullptr, 0.0, n->part.p, x);
