@@ -1352,10 +1352,13 @@ static void build_dense(fs_mesh *m, Hierarchy &H, double alpha) {
   }
 }
 
+bool amg_will_build(const fs_mesh *m) {
+  return !m->amg || (m->mg_reagg > 0 && m->ncalls_mg % m->mg_reagg == 0) || m->amg->lev.empty() ||
+         m->amg->lev[0].n != m->n;
+}
+
 void amg_prepare(fs_mesh *m, const double *ac, const double *anb, double alpha) {
-  const bool rebuild = !m->amg || (m->mg_reagg > 0 && m->ncalls_mg % m->mg_reagg == 0) ||
-                       m->amg->lev.empty() || m->amg->lev[0].n != m->n;
-  if (rebuild) build_hierarchy(m, ac, anb);
+  if (amg_will_build(m)) build_hierarchy(m, ac, anb);
   m->ncalls_mg++;
   Hierarchy &H = *m->amg;
   H.fp32 = m->mg_fp32 != 0;
@@ -1618,6 +1621,7 @@ static T *post_smooth(fs_mesh *m, DLevel &D, int level, const T *b, T *x, T *oth
 // applied level down are one dense product.  out must not alias rhs.
 template <class T>
 static void vcycle(fs_mesh *m, const double *rhs, double *out, double alpha, const int *flags) {
+  if (solve_done(m)) return; // its kernels would return at once
   Hierarchy &H = *m->amg;
   hipStream_t s = m->stream;
   const int L = (int)H.lev.size();
@@ -1775,8 +1779,10 @@ static void vcycle(fs_mesh *m, const double *rhs, double *out, double alpha, con
     for (int l1 = 2; l1 <= top - 1; ++l1) again.push_back(l1);
   // the bottom's result goes up unless the next correction is the bottom's own
   auto goes_up = [&](size_t k) { return k >= again.size() || again[k] != bot; };
+  if (solve_done(m)) return; // the rest would return at once
   bottom(goes_up(0));
   for (size_t k = 0; k < again.size(); ++k) {
+    if (solve_done(m)) return;
     if (again[k] != bot) ascend(again[k]);
     redescend(again[k], goes_up(k + 1));
   }
@@ -1791,8 +1797,8 @@ void amg_apply(fs_mesh *m, const double *rhs, double *out, const int *flags, dou
 // The reference's multigrid solve loop (AlgebraicMultiGridMainRoutine.for:
 // 371-416): cycles while the fine L1 residual exceeds rrf*ires and at most
 // MaxMultiGridCycles; each cycle corrects with one V-cycle of the residual.
-int amg_solve(fs_mesh *m, const double *ac, const double *anb, const double *bc, double *dphi,
-              int solver, bool warm) {
+void amg_solve(fs_mesh *m, const double *ac, const double *anb, const double *bc, double *dphi,
+               int solver, bool warm) {
   (void)solver;
   // additive correction as in the reference unless asked otherwise
   const double alpha = m->mg_alpha > 0.0 ? m->mg_alpha : 1.0;
@@ -1801,36 +1807,20 @@ int amg_solve(fs_mesh *m, const double *ac, const double *anb, const double *bc,
   const int n = m->n;
   double *r = m->wk.v[8], *c = m->wk.v[9];
   int *flags = m->wk.flags;
-  // flags[2] holds itmax for the Krylov solvers; the multigrid loop is
-  // bounded by MaxMultiGridCycles instead
-  int itmax_cycles = m->mg_maxcycles;
-  FS_HIP_THROW(hipMemcpyAsync(flags + 2, &itmax_cycles, sizeof(int), hipMemcpyHostToDevice, s));
   const int gr = std::min(kPartials, gfor(n));
   // the first cycle's right-hand side: bc (dphi = 0), or the residual of the
   // initial guess
   if (warm)
     hipLaunchKernelGGL(k_amg_res, dim3(gr), dim3(kBlock), 0, s, n, m->w, m->d_nbr.p, ac, anb, bc, dphi, r,
                        m->wk.partial, (const int *)flags);
-  else
-    FS_HIP_THROW(hipMemcpyAsync(r, bc, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-  int fl[4] = {0, 0, 0, 0};
-  FS_HIP_THROW(hipMemcpyAsync(fl, flags, sizeof(int) * 4, hipMemcpyDeviceToHost, s));
-  FS_HIP_THROW(hipStreamSynchronize(s));
-  int launched = 0;
-  while (!fl[0] && launched < itmax_cycles) {
-    const int batch = std::min(m->check_every, itmax_cycles - launched);
-    for (int b = 0; b < batch; ++b) {
-      amg_apply(m, r, c, flags, alpha);
-      hipLaunchKernelGGL(k_add2, dim3(gfor(n)), dim3(kBlock), 0, s, n, dphi, c, flags);
-      hipLaunchKernelGGL(k_amg_res, dim3(gr), dim3(kBlock), 0, s, n, m->w, m->d_nbr.p, ac, anb,
-                         bc, dphi, r, m->wk.partial, flags);
-      launch_fin_conv(m, gr);
-    }
-    launched += batch;
-    FS_HIP_THROW(hipMemcpyAsync(fl, flags, sizeof(int) * 4, hipMemcpyDeviceToHost, s));
-    FS_HIP_THROW(hipStreamSynchronize(s));
-  }
-  return fl[1];
+  const double *rhs = warm ? r : bc;
+  run_cycles(m, gr, m->mg_maxcycles, [&]() {
+    amg_apply(m, rhs, c, flags, alpha);
+    hipLaunchKernelGGL(k_add2, dim3(gfor(n)), dim3(kBlock), 0, s, n, dphi, c, flags);
+    hipLaunchKernelGGL(k_amg_res, dim3(gr), dim3(kBlock), 0, s, n, m->w, m->d_nbr.p, ac, anb,
+                       bc, dphi, r, m->wk.partial, flags);
+    rhs = r;
+  });
 }
 
 int amg_export(fs_mesh *m, int level, int *dims, int *parent, int *seed, int *nchild,

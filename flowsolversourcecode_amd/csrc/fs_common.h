@@ -76,6 +76,16 @@ template <class T> struct DevBuf {
 
 struct Hierarchy; // fs_amg.hip
 
+// What a solve tells the host without a copy or a synchronisation: pinned
+// host memory that the one-block finalise kernels write.  `word` is the
+// progress of the solve with the number in its upper half (post_word in
+// fs_solve.hip); scal and extra are complete when it carries the final bit.
+struct SolveBox {
+  unsigned long long word;
+  double scal[24];
+  double extra[16];
+};
+
 // Per-launch HIP-event timing of one kernel site of the solve loops: events
 // are recorded by the dispatch itself (hipExtLaunchKernelGGL), tagged with
 // the Krylov iteration that launched them, so launches after convergence
@@ -117,6 +127,8 @@ struct fs_mesh {
   fs::DevBuf<double> partial;  // kPartials * 5
   fs::DevBuf<double> scal;     // scalar slots
   fs::DevBuf<int> flags;       // [0] done, [1] iterations
+  fs::SolveBox *box = nullptr; // pinned; what the finalise kernels post to the host
+  unsigned seq = 0;            // the solve the posts belong to
   // The scratch the solve uses: the mesh's buffers above, or slices of the
   // library's static device array for the duration of a
   // fs_solve_equation_device_noalloc call.
@@ -139,7 +151,6 @@ struct fs_mesh {
   int mg_sell_rows = 100000;       // coarse levels at least this large use sliced ELL
   double mg_alpha = 0.0;           // over-correction (0: 1 as solver, 1.7 as preconditioner)
   int gmres_m = 30, check_every = 8;
-  int iter_pred[256] = {0}; // iterations of the last solve per (variable, solver)
   int ncalls_mg = 0;
   long long nnz = 0;                    // off-diagonal entries of the ELL pattern
   fs::KernelClock kclock;

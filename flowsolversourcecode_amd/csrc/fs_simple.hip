@@ -1259,12 +1259,12 @@ static int phase_momentum_solve(SimpleCase &C, int comp, fs_simple_stats *st) {
     // assembly copied into mx: solve for it, then bring it back
     mirror_options(C.mom_mesh, C.mesh);
     rc = solve_device(C.mom_mesh, comp + 1, C.mx.p, C.mrrf, C.mitmax, C.msolver, C.mlmg, C.ac.p, C.anb.p, C.bc.p,
-                      C.dphi.p, res4, &ss);
+                      C.dphi.p, res4, &ss, false, false);
     if (rc < 0) return rc;
     hipLaunchKernelGGL(k_unpermute, dim3(blocks(C.N)), dim3(kBlock), 0, C.s, C.N, C.mperm.p, C.mx.p, phi);
   } else {
     rc = solve_device(C.mesh, comp + 1, phi, C.mrrf, C.mitmax, C.msolver, C.mlmg, C.ac.p, C.anb.p, C.bc.p,
-                      C.dphi.p, res4, &ss);
+                      C.dphi.p, res4, &ss, false, false);
     if (rc < 0) return rc;
   }
   if (C.periodic()) { // UpdatePeriodic (SolveXMomentumEquation.for:299)
@@ -1372,7 +1372,7 @@ static int phase_pc_solve_correct(SimpleCase &C, fs_simple_stats *st) {
     FS_HIP(hipMemcpyAsync(C.dphi.p, C.pcprev.p, sizeof(double) * C.N, hipMemcpyDeviceToDevice, C.s));
   }
   const int rc = solve_device(C.mesh, 4, C.pc.p, C.prrf, C.pitmax, C.psolver, C.plmg, C.ac.p,
-                              C.anb.p, C.bc.p, C.dphi.p, res4, &ss, warm || prev);
+                              C.anb.p, C.bc.p, C.dphi.p, res4, &ss, warm || prev, false);
   if (rc < 0) return rc;
   if (C.sink) mpnn_capture(C.sink, C.s, C.bc.p, C.dphi.p, C.ac.p, C.anb.p, C.vol.p, C.pcprev.p);
   FS_HIP(hipMemcpyAsync(C.pcprev.p, C.dphi.p, sizeof(double) * C.N, hipMemcpyDeviceToDevice, C.s));
@@ -1470,7 +1470,7 @@ static int phase_sst_equation(SimpleCase &C, int var, fs_simple_stats *st) {
   double res4[4];
   const int rc = solve_device(C.mesh, var ? 10 : 8, var ? T.om.p : T.k.p, var ? T.wrrf : T.krrf,
                               var ? T.witmax : T.kitmax, var ? T.wsolver : T.ksolver, 0, C.ac.p, C.anb.p, C.bc.p,
-                              C.dphi.p, res4, &ss);
+                              C.dphi.p, res4, &ss, false, false);
   if (rc < 0) return rc;
   (var ? T.it_w : T.it_k) = ss.iterations;
   if (st) st->turbulence_iterations += ss.iterations;
@@ -1513,7 +1513,7 @@ static int wall_distance(SimpleCase &C, double tol, int maxouter, int *passes) {
     fs_solve_stats ss{};
     double res4[4];
     const int rc = solve_device(C.mesh, 5, phi.p, 1e-8, 500, FS_CG, FS_MG_PRECOND, C.ac.p, C.anb.p, C.bc.p,
-                                C.dphi.p, res4, &ss);
+                                C.dphi.p, res4, &ss, false, false);
     if (rc < 0) return rc;
     if (first < 0.0) first = ss.initial_l1;
     done = !(ss.initial_l1 > tol * first);

@@ -14,15 +14,18 @@
 // cell, every sum is formed in the reference's slot order, so a sweep,
 // residual or product of one cell is bitwise the reference's.
 //
-// Convergence never needs the host inside a batch: a one-block kernel
-// updates the device flags (done, iteration count), every iteration kernel
-// returns immediately once done is set, and the host reads the flags only
-// every check_every iterations.
+// Convergence never waits for the host: a one-block kernel updates the device
+// flags (done, iteration count), and every iteration kernel returns
+// immediately once done is set.  The same kernel posts the iteration count
+// and done to pinned host memory, and the host launches iterations only one
+// ahead of the last one posted.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstring>
+#include <functional>
 #include <mutex>
 #include <stdexcept>
 
@@ -45,6 +48,18 @@ enum Flag {
   F_NEEDPOS = 7, // set by the host when the solver divides by the diagonal
   F_NFLAGS = 8
 };
+static_assert(S_NSLOTS <= (int)(sizeof(SolveBox::scal) / sizeof(double)), "scalars of the box");
+
+// The progress word of SolveBox: bit 0 done, bit 1 final (the scalars are
+// there as well), bits 2-3 F_BAD, then the iteration count, and the solve's
+// number in the upper 32 bits, so that a word of an earlier solve is not
+// taken for this one's.
+constexpr unsigned long long kBoxDone = 1, kBoxFinal = 2;
+__device__ __forceinline__ void post_word(SolveBox *box, unsigned seq, const int *flags, unsigned long long final_bit) {
+  const unsigned long long w = ((unsigned long long)seq << 32) | ((unsigned long long)(flags[F_ITER] & 0xfffffff) << 4) |
+                               ((unsigned long long)flags[F_BAD] << 2) | final_bit | (flags[F_DONE] ? kBoxDone : 0);
+  __hip_atomic_store(&box->word, w, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // F_INNER: the GMRES cycle in progress has finished its Arnoldi steps;
 // F_GATE = F_DONE | F_INNER, the flag the cycle's kernels (and the V-cycle
 // they call) test
@@ -801,7 +816,19 @@ enum FinOp {
   FIN_CG_ALPHA,       // alpha = rz/(p,q)
   FIN_WARM,           // reject an initial guess whose L1 residual exceeds ires
   FIN_WARM_SCALE,     // gamma = (A x0, b)/(A x0, A x0)
-  FIN_CONV_BICG_RHO   // FIN_CONV, then (unless done) FIN_BICG_RHO of the next iteration
+  FIN_CONV_BICG_RHO,  // FIN_CONV, then (unless done) FIN_BICG_RHO of the next iteration
+  FIN_POST            // post the scalars and the final word
+};
+
+// what the initial finaliser sets up a solve with, and where it posts
+struct SolveStart {
+  double rrf;
+  int itmax, itmax0; // of the loop; itmax0 < 1: done before it starts
+  int needpos;       // the solver divides by the diagonal
+};
+struct Post {
+  SolveBox *box;
+  unsigned seq;
 };
 
 // one workgroup of kFinBlock threads combines up to kPartials partials
@@ -852,9 +879,10 @@ __device__ void bicg_rho(double a, double *__restrict__ scal, int *__restrict__ 
 }
 
 __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ part,
-                      double *__restrict__ scal, int *__restrict__ flags) {
-  if (op != FIN_INIT_NORMS && op != FIN_TRUE_RES && flags[F_DONE]) return;
-  const double a = reduce_partials(part, np);
+                      double *__restrict__ scal, int *__restrict__ flags, SolveStart st, Post to) {
+  const bool always = op == FIN_INIT_NORMS || op == FIN_TRUE_RES || op == FIN_POST;
+  if (!always && flags[F_DONE]) return;
+  const double a = op == FIN_POST ? 0.0 : reduce_partials(part, np);
   double b = 0.0, c = 0.0, d = 0.0, e = 0.0;
   if (op == FIN_INIT_NORMS) {
     b = reduce_partials_max(part + kPartials, np);
@@ -865,19 +893,25 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
     b = reduce_partials(part + kPartials, np);
   }
   if (threadIdx.x != 0) return;
+  bool counted = false; // an iteration ended
   switch (op) {
   case FIN_INIT_NORMS: {
+    for (int k = 0; k < S_NSLOTS; ++k) scal[k] = 0.0;
+    for (int k = 0; k < F_NFLAGS; ++k) flags[k] = 0;
+    scal[S_RRF] = st.rrf;
+    flags[F_ITMAX] = st.itmax;
+    flags[F_NEEDPOS] = st.needpos;
     scal[S_RES_ABS] = a;
     scal[S_RES_MAX] = b;
     scal[S_RES_RMS] = sqrt(c / n);
     scal[S_RES_SCALED] = (nf == 4) ? 0.0 : b / (d + 1.0e-15);
     scal[S_IRES] = a;
     scal[S_FRES] = a;
-    flags[F_ITER] = 0;
-    flags[F_DONE] = !(a > scal[S_RRF] * a && 0 < flags[F_ITMAX]);
+    flags[F_DONE] = !(a > st.rrf * a && 0 < st.itmax0);
     // refused input: nothing runs, the caller's arrays stay as they were
-    flags[F_BAD] = e >= 2.0 ? 2 : (e >= 1.0 && flags[F_NEEDPOS]) ? 1 : 0;
+    flags[F_BAD] = e >= 2.0 ? 2 : (e >= 1.0 && st.needpos) ? 1 : 0;
     if (flags[F_BAD]) flags[F_DONE] = 1;
+    counted = true;
     break;
   }
   case FIN_PBCG_BK: {
@@ -891,6 +925,7 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
     scal[S_AK] = scal[S_BKNUM] / (a + 1.0e-10);
     break;
   case FIN_CONV: {
+    counted = true;
     scal[S_FRES] = a;
     const int it = flags[F_ITER] + 1;
     flags[F_ITER] = it;
@@ -902,6 +937,7 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
     bicg_rho(a, scal, flags);
     break;
   case FIN_CONV_BICG_RHO: {
+    counted = true;
     scal[S_FRES] = a;
     const int it = flags[F_ITER] + 1;
     flags[F_ITER] = it;
@@ -920,6 +956,8 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
     break;
   case FIN_TRUE_RES:
     scal[S_FRES] = a;
+    break;
+  case FIN_POST:
     break;
   case FIN_CG_RHO: {
     if (flags[F_ITER] > 0) {
@@ -948,6 +986,12 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
       flags[F_DONE] = 1;
     }
     break;
+  }
+  if (op == FIN_POST) {
+    for (int k = 0; k < S_NSLOTS; ++k) to.box->scal[k] = scal[k];
+    post_word(to.box, to.seq, flags, kBoxFinal);
+  } else if (counted || (!always && flags[F_DONE])) {
+    post_word(to.box, to.seq, flags, 0);
   }
 }
 
@@ -1295,6 +1339,8 @@ int mesh_prepare_solver(fs_mesh *m) {
   m->partial.alloc(5 * kPartials);
   m->scal.alloc(S_NSLOTS);
   m->flags.alloc(F_NFLAGS);
+  FS_HIP_THROW(hipHostMalloc((void **)&m->box, sizeof(SolveBox), hipHostMallocDefault));
+  memset(m->box, 0, sizeof(SolveBox));
   for (int k = 0; k < 12; ++k) m->wk.v[k] = m->v[k].p;
   m->wk.dc = sw->dc.p;
   m->wk.partial = m->partial.p;
@@ -1398,6 +1444,8 @@ void mesh_release_solver(fs_mesh *m) {
   kernel_clock_release(m);
   delete reinterpret_cast<SolveWork *>(m->solve_work);
   m->solve_work = nullptr;
+  if (m->box) (void)hipHostFree(m->box);
+  m->box = nullptr;
 }
 
 static void gather(fs_mesh *m, size_t cnt, const int *idx, const double *in, double *out, const int *flags = nullptr) {
@@ -1459,44 +1507,79 @@ static void ilu_apply(fs_mesh *m, double *dphi, const int *flags) {
                      flags);
 }
 
+static void fin(fs_mesh *m, FinOp op, int np, int nf, SolveStart st = SolveStart{}) {
+  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, m->stream, (int)op, np, m->n, nf, m->wk.partial, m->wk.scal,
+                     m->wk.flags, st, Post{m->box, m->seq});
+}
+
 static void host_flags(fs_mesh *m, int *fl) {
   FS_HIP_THROW(hipMemcpyAsync(fl, m->wk.flags, sizeof(int) * F_NFLAGS, hipMemcpyDeviceToHost, m->stream));
   FS_HIP_THROW(hipStreamSynchronize(m->stream));
 }
 
-// Runs `body` in batches until the device sets done.  The first batch is the
-// iteration count of the previous solve of the same variable and solver (the
-// SIMPLE loop solves nearly the same system every outer iteration; at most
-// 4 check_every), later batches grow 2, 4, ... up to check_every; without a
-// previous solve every batch is check_every long.  Iterations launched past
-// convergence return at once, so the batch sizes only trade idle launches
-// against host checks.
-template <class F> static int run_batches(fs_mesh *m, int itmax, int key, F body) {
-  int fl[F_NFLAGS] = {0};
-  int launched = 0;
-  int &pred = m->iter_pred[key & 255];
-  int next = pred > 0 ? std::min(pred, 4 * m->check_every) : m->check_every, grow = 2;
-  m->kclock.solve_first = m->kclock.used;
-  while (!fl[F_DONE] && launched < itmax) {
-    const int batch = std::min(next, itmax - launched);
-    for (int b = 0; b < batch; ++b) {
-      m->kclock.cur_iter = launched + b;
-      body();
+// The progress of the solve in flight as posted so far (0: nothing yet).
+static unsigned long long box_word(const fs_mesh *m) {
+  const unsigned long long w = __atomic_load_n(&m->box->word, __ATOMIC_ACQUIRE);
+  return (unsigned)(w >> 32) == m->seq ? w : 0;
+}
+static int box_iterations(unsigned long long w) { return (int)(w >> 4 & 0xfffffff); }
+static int box_bad(unsigned long long w) { return (int)(w >> 2 & 3); }
+
+bool solve_done(const fs_mesh *m) { return box_word(m) & kBoxDone; }
+
+// Waits for a post that pred accepts.  Ends with the stream in any case: the
+// stream is asked now and then, and a stream that has failed, or has nothing
+// left to run that could post, raises an error.
+template <class P> static unsigned long long box_wait(fs_mesh *m, P pred) {
+  for (unsigned long long w;;) {
+    for (int k = 0; k < 2000; ++k) {
+      if (pred(w = box_word(m))) return w;
+#if defined(__x86_64__)
+      __builtin_ia32_pause();
+#endif
     }
-    launched += batch;
-    host_flags(m, fl);
-    next = pred > 0 ? std::min(grow, m->check_every) : m->check_every;
-    // stop doubling at check_every: an unbounded doubling overflows int
-    // after 31 batches
-    if (grow < m->check_every) grow *= 2;
+    const hipError_t e = hipStreamQuery(m->stream);
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();
+      continue;
+    }
+    FS_HIP_THROW(e);
+    if (pred(w = box_word(m))) return w;
+    throw std::runtime_error("the stream ended without the solve's post");
   }
-  pred = fl[F_ITER];
-  // launches of iterations past the converged one returned at once
+}
+
+unsigned long long box_wait_final(fs_mesh *m) {
+  return box_wait(m, [](unsigned long long w) { return (w & kBoxFinal) != 0; });
+}
+
+// Runs `body` until the device posts done, at most itmax times, two iterations
+// ahead of the last one posted (at most FS_OPT_CHECK_EVERY - 1), so that the
+// stream is never empty; the iterations launched past the last one run idle:
+// their kernels return at once, and bodies of many launches stop where they
+// see done posted.  One ahead leaves gaps where an iteration takes the host
+// as long as the device (24 launches of 3 us on 4096 cells).  Waiting for
+// copied flags after batches of the previous solve's iteration count cost a
+// synchronisation of about 20 us a batch and up to check_every idle iterations.
+template <class F> static void run_iterations(fs_mesh *m, int itmax, F body) {
+  const int ahead = std::min(2, m->check_every - 1);
+  m->kclock.solve_first = m->kclock.used;
+  for (int k = 0; k < itmax; ++k) {
+    const unsigned long long w = box_wait(m, [&](unsigned long long v) {
+      return (v & kBoxDone) || (v ? box_iterations(v) : -1) + ahead >= k;
+    });
+    if (w & kBoxDone) break;
+    m->kclock.cur_iter = k;
+    body();
+  }
+  m->kclock.cur_iter = -1;
+}
+
+// the clock's launches of iterations past the converged one returned at once
+static void clock_iterations(fs_mesh *m, int iters) {
   KernelClock &c = m->kclock;
   for (int u = c.solve_first; u < c.used; ++u)
-    if (c.iter[u] >= fl[F_ITER]) c.live[u] = 0;
-  c.cur_iter = -1;
-  return fl[F_ITER];
+    if (c.iter[u] >= iters) c.live[u] = 0;
 }
 
 // x0 *= (A x0, b)/(A x0, A x0): the scaling of an initial guess with the
@@ -1507,8 +1590,7 @@ static void scale_guess(fs_mesh *m, const double *ac, const double *anb, const d
   hipStream_t s = m->stream;
   hipLaunchKernelGGL(k_spmv_dot_ts, dim3(gr), dim3(kBlock), 0, s, n, m->w, EllNbr(m->d_nbr.p, m->d_nbr16.p), ac, anb, x,
                      v, bc, m->wk.partial, m->wk.flags);
-  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_WARM_SCALE, gr, n, 4, m->wk.partial, m->wk.scal,
-                     m->wk.flags);
+  fin(m, FIN_WARM_SCALE, gr, 4);
   hipLaunchKernelGGL(k_warm_scale, dim3(grid_for(n)), dim3(kBlock), 0, s, n, x, m->wk.scal, m->wk.flags);
 }
 
@@ -1556,15 +1638,17 @@ __global__ void __launch_bounds__(kBlock) k_proj_gram(int n, ProjVecs y, const d
   }
 }
 
-// out[u] = sum of row u of the partials, in a fixed order
-__global__ void __launch_bounds__(kBlock) k_proj_fin(int ns, int gp, const double *__restrict__ part,
-                                                     double *__restrict__ out) {
+// extra[u] of the box = sum of row u of the partials, in a fixed order
+__global__ void __launch_bounds__(kBlock) k_proj_fin(int ns, int gp, const double *__restrict__ part, Post to) {
   for (int u = 0; u < ns; ++u) {
     double t = 0.0;
     for (int j = threadIdx.x; j < gp; j += kBlock) t += part[(size_t)u * gp + j];
     t = block_sum<kBlock>(t);
-    if (threadIdx.x == 0) out[u] = t;
+    if (threadIdx.x == 0) to.box->extra[u] = t;
   }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&to.box->word, ((unsigned long long)to.seq << 32) | kBoxFinal, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void k_proj_comb(int n, int k, ProjVecs x, ProjCoef c, double *__restrict__ out) {
@@ -1589,17 +1673,18 @@ int project_guess(fs_mesh *m, const double *ac, const double *anb, const double 
                        m->wk.v[a]);
   }
   const int ns = k * (k + 1) / 2 + k;
-  double *part = m->wk.partial, *out = m->wk.partial + (size_t)ns * kProjGrid;
+  double *part = m->wk.partial;
   switch (k) {
   case 1: hipLaunchKernelGGL(k_proj_gram<1>, dim3(kProjGrid), dim3(kBlock), 0, s, n, yv, bc, part); break;
   case 2: hipLaunchKernelGGL(k_proj_gram<2>, dim3(kProjGrid), dim3(kBlock), 0, s, n, yv, bc, part); break;
   case 3: hipLaunchKernelGGL(k_proj_gram<3>, dim3(kProjGrid), dim3(kBlock), 0, s, n, yv, bc, part); break;
   default: hipLaunchKernelGGL(k_proj_gram<4>, dim3(kProjGrid), dim3(kBlock), 0, s, n, yv, bc, part); break;
   }
-  hipLaunchKernelGGL(k_proj_fin, dim3(1), dim3(kBlock), 0, s, ns, kProjGrid, part, out);
-  double g[kProjMax * (kProjMax + 1) / 2 + kProjMax];
-  FS_HIP_THROW(hipMemcpyAsync(g, out, sizeof(double) * ns, hipMemcpyDeviceToHost, s));
-  FS_HIP_THROW(hipStreamSynchronize(s));
+  ++m->seq; // a post of its own
+  hipLaunchKernelGGL(k_proj_fin, dim3(1), dim3(kBlock), 0, s, ns, kProjGrid, part, Post{m->box, m->seq});
+  static_assert(kProjMax * (kProjMax + 1) / 2 + kProjMax <= (int)(sizeof(SolveBox::extra) / sizeof(double)), "Gram sums");
+  box_wait_final(m);
+  const double *g = m->box->extra;
   double G[kProjMax][kProjMax] = {}, h[kProjMax] = {};
   for (int a = 0, u = 0; a < k; ++a) {
     for (int c = a; c < k; ++c) G[a][c] = G[c][a] = g[u++];
@@ -1643,7 +1728,7 @@ int project_guess(fs_mesh *m, const double *ac, const double *anb, const double 
 
 int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int solver, int lmg,
                  const double *ac, const double *anb, const double *bc, double *dphi, double *res4,
-                 fs_solve_stats *st, bool warm) {
+                 fs_solve_stats *st, bool warm, bool sync) {
   const int n = m->n, w = m->w;
   hipStream_t s = m->stream;
   auto t0 = std::chrono::steady_clock::now();
@@ -1654,35 +1739,30 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   const EllNbr nb(m->d_nbr.p, m->d_nbr16.p); // the row loops of the hot kernels
   SolveWork &sw = work(m);
 
-  double h_sc[S_NSLOTS] = {0};
-  h_sc[S_RRF] = rrf;
   if (solver < FS_SOR || solver > FS_CG || solver == FS_DIRECT) {
     set_error("unsupported solver code " + std::to_string(solver) +
               (solver == FS_DIRECT ? " ('direct' is the host's dense LU)" : ""));
     return -3;
   }
-  int h_fl[F_NFLAGS] = {0, 0, itmax, 0};
   // Gauss-Seidel, D-ILU (also PBCG's preconditioner) and every multigrid
   // smoother divide by the diagonal
-  h_fl[F_NEEDPOS] = (lmg != FS_MG_OFF || solver == FS_SOR || solver == FS_ILU || solver == FS_PBCG) ? 1 : 0;
-  FS_HIP(hipMemcpyAsync(scal, h_sc, sizeof(h_sc), hipMemcpyHostToDevice, s));
-  FS_HIP(hipMemcpyAsync(flags, h_fl, sizeof(h_fl), hipMemcpyHostToDevice, s));
+  SolveStart start{rrf, lmg == FS_MG_SOLVER ? m->mg_maxcycles : itmax, itmax, 0};
+  start.needpos = (lmg != FS_MG_OFF || solver == FS_SOR || solver == FS_ILU || solver == FS_PBCG) ? 1 : 0;
+  ++m->seq;
   hipLaunchKernelGGL(k_init_norms, dim3(gr), dim3(kBlock), 0, s, n, ac, bc, fit, part);
-  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_INIT_NORMS, gr, n, nf, part, scal, flags);
+  fin(m, FIN_INIT_NORMS, gr, nf, start);
   if (!warm) hipLaunchKernelGGL(k_zero_start, dim3(ge), dim3(kBlock), 0, s, n, dphi, (const int *)flags);
   auto refuse = [](int bad) {
     set_error(bad == 2 ? "a coefficient ac or source bc is not finite"
                        : "a diagonal coefficient ac <= 0, which this solver divides by");
     return bad == 2 ? -4 : -1;
   };
-  if (lmg != FS_MG_OFF) {
+  if (lmg != FS_MG_OFF && amg_will_build(m)) {
     // the hierarchy is built from the operator: refuse bad input before that
-    int fl0[F_NFLAGS];
-    host_flags(m, fl0);
-    if (fl0[F_BAD]) return refuse(fl0[F_BAD]);
+    const int bad = box_bad(box_wait(m, [](unsigned long long w) { return w != 0; }));
+    if (bad) return refuse(bad);
   }
 
-  int iters = 0;
   double *V0 = m->wk.v[0], *V1 = m->wk.v[1], *V2 = m->wk.v[2], *V3 = m->wk.v[3], *V4 = m->wk.v[4],
          *V5 = m->wk.v[5], *V6 = m->wk.v[6], *V7 = m->wk.v[7];
 
@@ -1694,12 +1774,12 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   if (warm) {
     scale_guess(m, ac, anb, bc, dphi, V3);
     hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, flags);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_WARM, gr, n, nf, part, scal, flags);
+    fin(m, FIN_WARM, gr, nf);
     hipLaunchKernelGGL(k_warm_fix, dim3(ge), dim3(kBlock), 0, s, n, dphi, (const int *)flags);
   }
 
   if (lmg == FS_MG_SOLVER) {
-    iters = amg_solve(m, ac, anb, bc, dphi, solver, warm);
+    amg_solve(m, ac, anb, bc, dphi, solver, warm);
   } else if (solver == FS_PBCG) {
     // r=V0 rr=V1 p=V2 pp=V3 z=V4 zz=V5 (PBCG1.F90:4)
     ilu_factor(m, ac, anb, m->wk.dc);
@@ -1713,20 +1793,20 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     const double alpha = m->mg_alpha > 0.0 ? m->mg_alpha : 1.7;
     if (pre) amg_prepare(m, ac, anb, alpha);
     const double *dc = pre ? nullptr : m->wk.dc;
-    iters = run_batches(m, itmax, nf * 8 + solver, [&]() {
+    run_iterations(m, itmax, [&]() {
       if (pre) {
         amg_apply(m, V0, V6, flags, alpha);
         amg_apply(m, V1, V7, flags, alpha);
       }
       hipLaunchKernelGGL(k_pbcg_bknum, dim3(gr), dim3(kBlock), 0, s, n, V0, V1, dc, V6, part, flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_PBCG_BK, gr, n, nf, part, scal, flags);
+      fin(m, FIN_PBCG_BK, gr, nf);
       hipLaunchKernelGGL(k_pbcg_p, dim3(ge), dim3(kBlock), 0, s, n, V0, V1, dc, V6, V7, V2, V3, scal, flags);
       hipLaunchKernelGGL(k_pbcg_ap, dim3(gr), dim3(kBlock), 0, s, n, w, sw.wt, nbr, sw.tlin.p,
                          sw.tsrc.p, ac, anb, V2, V3, V4, V5, part, flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_PBCG_AK, gr, n, nf, part, scal, flags);
+      fin(m, FIN_PBCG_AK, gr, nf);
       hipLaunchKernelGGL(k_pbcg_axpy, dim3(ge), dim3(kBlock), 0, s, n, dphi, V0, V1, V2, V4, V5, scal, flags);
       hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_CONV, gr, n, nf, part, scal, flags);
+      fin(m, FIN_CONV, gr, nf);
     });
   } else if (solver == FS_SOR) {
     // multicolour symmetric Gauss-Seidel: colours forward then backward.  A
@@ -1736,9 +1816,10 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     // forward pass after the first at colour 1 (the residual check between
     // iterations leaves x alone).
     bool first = true;
-    iters = run_batches(m, itmax, nf * 8 + solver, [&]() {
+    run_iterations(m, itmax, [&]() {
       const int nc = (int)sw.color_ptr.size() - 1;
       for (int c = first ? 0 : 1; c < nc; ++c) {
+        if (solve_done(m)) return; // the rest would return at once
         const int b = sw.color_ptr[c], e = sw.color_ptr[c + 1];
         hipLaunchKernelGGL(k_gs_color, dim3(grid_for(e - b)), dim3(kBlock), 0, s, e - b,
                            sw.color_cells.p + b, n, w, nb, ac, anb, bc, dphi, flags);
@@ -1750,7 +1831,7 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
       }
       first = false;
       hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_CONV, gr, n, nf, part, scal, flags);
+      fin(m, FIN_CONV, gr, nf);
     });
   } else if (solver == FS_BICGS) {
     // right-preconditioned BiCGSTAB; r=V0 r0=V1 p=V2 v=V3 s=V4 t=V5 phat=V6 shat=V7
@@ -1765,23 +1846,23 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     hipLaunchKernelGGL(k_zero, dim3(ge), dim3(kBlock), 0, s, n, V3);
     // rho of the first iteration; every later rho comes with the update
     hipLaunchKernelGGL(k_dot2, dim3(gr), dim3(kBlock), 0, s, n, V1, V0, nullptr, nullptr, part, flags);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_BICG_RHO, gr, n, nf, part, scal, flags);
-    iters = run_batches(m, itmax, nf * 8 + solver, [&]() {
+    fin(m, FIN_BICG_RHO, gr, nf);
+    run_iterations(m, itmax, [&]() {
       hipLaunchKernelGGL(k_bicg_p, dim3(ge), dim3(kBlock), 0, s, n, V0, V3, V2, scal, flags);
       if (pre) amg_apply(m, V2, V6, flags, alpha);
       const double *ph = pre ? V6 : V2;
       timed_launch(m, FS_CLOCK_SPMV, spmv_bytes, k_spmv_dot, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, ph,
                    V3, (const double *)V1, part, (const int *)flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_BICG_ALPHA, gr, n, nf, part, scal, flags);
+      fin(m, FIN_BICG_ALPHA, gr, nf);
+      if (solve_done(m)) return;
       hipLaunchKernelGGL(k_bicg_s, dim3(ge), dim3(kBlock), 0, s, n, V0, V3, V4, scal, flags);
       if (pre) amg_apply(m, V4, V7, flags, alpha);
       const double *sh = pre ? V7 : V4;
       hipLaunchKernelGGL(k_spmv_dot_ts, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, sh, V5, V4, part, flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_BICG_OMEGA, gr, n, nf, part, scal, flags);
+      fin(m, FIN_BICG_OMEGA, gr, nf);
       hipLaunchKernelGGL(k_bicg_update, dim3(gr), dim3(kBlock), 0, s, n, dphi, V0, ph, sh, V4, V5, (const double *)V1,
                          scal, part, flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_CONV_BICG_RHO, gr, n, nf, part, scal,
-                         flags);
+      fin(m, FIN_CONV_BICG_RHO, gr, nf);
     });
   } else if (solver == FS_CG) {
     // preconditioned conjugate gradient; r=V0 z=V1 p=V2 q=V3
@@ -1792,20 +1873,20 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     const double spmv_bytes = 8.0 * n + (nb.d16 ? 4.0 * ((w + 1) / 2) : 4.0 * w) * n + 8.0 * m->nnz + 16.0 * n;
     hipLaunchKernelGGL(k_resid_vec, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, V0, nullptr,
                        part);
-    iters = run_batches(m, itmax, nf * 8 + solver, [&]() {
+    run_iterations(m, itmax, [&]() {
       const double *z = V0;
       if (pre) {
         amg_apply(m, V0, V1, flags, alpha);
         z = V1;
       }
       hipLaunchKernelGGL(k_dot2, dim3(gr), dim3(kBlock), 0, s, n, V0, z, nullptr, nullptr, part, flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_CG_RHO, gr, n, nf, part, scal, flags);
+      fin(m, FIN_CG_RHO, gr, nf);
       hipLaunchKernelGGL(k_cg_p, dim3(ge), dim3(kBlock), 0, s, n, z, V2, scal, flags);
       timed_launch(m, FS_CLOCK_SPMV, spmv_bytes, k_spmv_dot, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, V2,
                    V3, (const double *)V2, part, (const int *)flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_CG_ALPHA, gr, n, nf, part, scal, flags);
+      fin(m, FIN_CG_ALPHA, gr, nf);
       hipLaunchKernelGGL(k_cg_update, dim3(gr), dim3(kBlock), 0, s, n, dphi, V0, V2, V3, scal, part, flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_CONV, gr, n, nf, part, scal, flags);
+      fin(m, FIN_CONV, gr, nf);
     });
   } else if (solver == FS_GMRES) {
     // restarted GMRES(m), right-preconditioned: basis V (m+1 vectors), z = M^-1 v_j
@@ -1864,7 +1945,6 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
       restart();
       host_flags(m, fl);
     }
-    iters = fl[F_ITER];
   } else if (solver == FS_ILU) {
     // the reference's ILU iteration: exact D-ILU diagonal, then per iteration
     // the residual and the two level-scheduled substitutions
@@ -1872,12 +1952,12 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     if (!sw.ilu.ready) precompute_ilu_sweep(m, sw.diag, sw.ilu);
     ilu_pack(m, anb);
     IluSweep &S = sw.ilu;
-    iters = run_batches(m, itmax, nf * 8 + solver, [&]() {
+    run_iterations(m, itmax, [&]() {
       hipLaunchKernelGGL(k_ilu_resid, dim3(ge), dim3(kBlock), 0, s, n, w, nbr, ac, anb, bc, dphi, S.fwd.order.pos,
                          S.fwd.r, flags);
       ilu_apply(m, dphi, flags);
       hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, flags);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_CONV, gr, n, nf, part, scal, flags);
+      fin(m, FIN_CONV, gr, nf);
     });
   } else {
     set_error("unsupported solver code " + std::to_string(solver));
@@ -1887,23 +1967,31 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   (void)V6;
   (void)V7;
 
-  // true final residual, fit += dphi (:180)
-  int fl[F_NFLAGS];
-  host_flags(m, fl);
-  if (fl[F_BAD]) return refuse(fl[F_BAD]);
-  hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, nullptr);
-  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, s, (int)FIN_TRUE_RES, gr, n, nf, part, scal, flags);
+  // true final residual, fit += dphi (:180).  The sweeps, ILU and PBCG end on
+  // the true residual of the same dphi: formed again it would be the same bits.
+  const bool ends_true = lmg != FS_MG_SOLVER && (solver == FS_SOR || solver == FS_ILU || solver == FS_PBCG) && !warm;
+  if (!ends_true) {
+    hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, nullptr);
+    fin(m, FIN_TRUE_RES, gr, nf);
+  }
   add_inplace(m, fit, dphi);
-  double h_out[S_NSLOTS];
-  FS_HIP(hipMemcpyAsync(h_out, scal, sizeof(h_out), hipMemcpyDeviceToHost, s));
-  FS_HIP(hipStreamSynchronize(s));
+  fin(m, FIN_POST, 0, nf);
+  const unsigned long long last = box_wait_final(m);
+  // for the caller's own streams and copies: everything above is complete
+  if (sync) FS_HIP(hipStreamSynchronize(s));
+  if (box_bad(last)) {
+    if (lmg != FS_MG_OFF) m->ncalls_mg--; // a refused call does not count towards the next aggregation
+    return refuse(box_bad(last));
+  }
+  const double *h_out = m->box->scal;
   if (res4) {
     res4[0] = h_out[S_RES_ABS];
     res4[1] = h_out[S_RES_MAX];
     res4[2] = h_out[S_RES_RMS];
     res4[3] = h_out[S_RES_SCALED];
   }
-  if (lmg != FS_MG_SOLVER) iters = fl[F_ITER];
+  const int iters = box_iterations(last);
+  clock_iterations(m, iters);
   if (st) {
     st->iterations = iters;
     st->levels = (lmg != FS_MG_OFF) ? amg_levels(m) : 1;
@@ -1919,18 +2007,22 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   return converged ? 0 : 1;
 }
 
-__global__ void k_add(int n, double *__restrict__ a, const double *__restrict__ b) {
+// fit += dphi, unless the input was refused
+__global__ void k_add(int n, double *__restrict__ a, const double *__restrict__ b, const int *__restrict__ flags) {
+  if (flags[F_BAD]) return;
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i < n) a[i] = a[i] + b[i];
 }
 
-void launch_fin_conv(fs_mesh *m, int np) {
-  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, m->stream, (int)FIN_CONV, np, m->n, 4,
-                     m->wk.partial, m->wk.scal, m->wk.flags);
+void run_cycles(fs_mesh *m, int np, int itmax, const std::function<void()> &body) {
+  run_iterations(m, itmax, [&]() {
+    body();
+    fin(m, FIN_CONV, np, 4);
+  });
 }
 
 void add_inplace(fs_mesh *m, double *a, const double *b) {
-  hipLaunchKernelGGL(k_add, dim3(grid_for(m->n)), dim3(kBlock), 0, m->stream, m->n, a, b);
+  hipLaunchKernelGGL(k_add, dim3(grid_for(m->n)), dim3(kBlock), 0, m->stream, m->n, a, b, m->wk.flags);
 }
 
 } // namespace fs
