@@ -40,7 +40,7 @@ namespace fs {
 
 namespace {
 
-inline int gfor(int n) { return std::max(1, (n + kBlock - 1) / kBlock); }
+inline int gfor(int n) { return xcd_grid(n); }
 
 // ------------------------------------------------------------ host setup
 struct HostLevel {

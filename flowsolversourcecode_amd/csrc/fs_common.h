@@ -32,7 +32,18 @@ void set_error(const std::string &msg);
   } while (0)
 
 constexpr int kBlock = 256;     // threads per block for streaming kernels
-constexpr int kPartials = 8192; // fixed number of reduction partials (one row per thread up to 2.1 M rows)
+// Most partials of a reduction: one row per thread up to 8.4 M rows.  The
+// partials of a kernel lie gridDim.x apart, k-th sum at part[k gridDim.x + b].
+constexpr int kPartials = 32768;
+
+// Workgroups for n threads of kBlock, a multiple of 8 beyond a few (the extra
+// ones find nothing to do) so that xcd_block() can give each XCD one
+// contiguous range; left as it comes, seven grids of eight stayed in
+// round-robin order, where every L2 fetches every other's neighbours.
+inline int xcd_grid(long long n) {
+  const int g = (int)((n + kBlock - 1) / kBlock);
+  return g < 1 ? 1 : g < 64 ? g : (g + 7) & ~7;
+}
 
 // Device buffer owning a hipMalloc allocation.
 template <class T> struct DevBuf {
@@ -124,7 +135,7 @@ struct fs_mesh {
   fs::DevBuf<int> d_face_code;  // per (cell, slot): face*4 + role
   // work vectors
   fs::DevBuf<double> v[12];
-  fs::DevBuf<double> partial;  // kPartials * 5
+  fs::DevBuf<double> partial;  // 5 sums' partials
   fs::DevBuf<double> scal;     // scalar slots
   fs::DevBuf<int> flags;       // [0] done, [1] iterations
   fs::SolveBox *box = nullptr; // pinned; what the finalise kernels post to the host
@@ -135,7 +146,7 @@ struct fs_mesh {
   struct Scratch {
     double *v[12];
     double *dc;       // D-ILU diagonal
-    double *partial;  // kPartials * 5
+    double *partial;
     double *scal;
     int *flags;
   } wk{};

@@ -37,7 +37,7 @@ namespace {
 
 enum { ROLE_NONE = 0, ROLE_OWNER = 1, ROLE_NEIGH = 2, ROLE_BOUND = 3 };
 
-inline int blocks(int n) { return std::max(1, (n + kBlock - 1) / kBlock); }
+inline int blocks(int n) { return xcd_grid(n); }
 
 struct GradArgs { // up to 4 fields at once
   const double *phi[4];

@@ -9,8 +9,10 @@
 // the neighbour table are the only irregular accesses.
 //
 // Reductions are deterministic: each block reduces with wavefront shuffles in
-// a fixed order into one of kPartials partials (grid-stride loop over a fixed
-// grid), and a one-block kernel combines the partials in index order.  Per
+// a fixed order into its own partial, and a one-block kernel combines the
+// partials in index order.  A thread takes one row: grids that stopped at
+// 8192 workgroups gave some threads of 2.9 M tetrahedra two rows and others
+// one, and k_spmv_dot took 66 us instead of 49.  Per
 // cell, every sum is formed in the reference's slot order, so a sweep,
 // residual or product of one cell is bitwise the reference's.
 //
@@ -66,15 +68,10 @@ __device__ __forceinline__ void post_word(SolveBox *box, unsigned seq, const int
 
 constexpr int kFinBlock = 1024; // threads of the one-workgroup finalise kernels
 
-static inline int grid_for(int n) {
-  int g = (n + kBlock - 1) / kBlock;
-  return g < 1 ? 1 : g;
-}
-static inline int grid_red(int n) {
-  int g = (n + kBlock - 1) / kBlock;
-  if (g > kPartials) g = kPartials;
-  return g < 1 ? 1 : g;
-}
+static inline int grid_for(int n) { return xcd_grid(n); }
+// one row per thread up to kPartials workgroups (the row loops of the reducing
+// kernels stride by the grid beyond)
+static inline int grid_red(int n) { return std::min(kPartials, xcd_grid(n)); }
 
 // The Krylov products stream the FP64 matrix (read twice per iteration, too
 // large to stay cached beside the vectors): non-temporal matrix loads.
@@ -145,10 +142,10 @@ __global__ void k_init_norms(int n, const double *__restrict__ ac, const double 
   bad = block_max<kBlock>(bad);
   if (threadIdx.x == 0) {
     part[blockIdx.x] = s1;
-    part[kPartials + blockIdx.x] = m1;
-    part[2 * kPartials + blockIdx.x] = s2;
-    part[3 * kPartials + blockIdx.x] = m2;
-    part[4 * kPartials + blockIdx.x] = bad;
+    part[gridDim.x + blockIdx.x] = m1;
+    part[2 * gridDim.x + blockIdx.x] = s2;
+    part[3 * gridDim.x + blockIdx.x] = m2;
+    part[4 * gridDim.x + blockIdx.x] = bad;
   }
 }
 
@@ -490,7 +487,7 @@ __global__ void k_dot2(int n, const double *__restrict__ a, const double *__rest
   s1 = block_sum<kBlock>(s1);
   if (threadIdx.x == 0) {
     part[blockIdx.x] = s0;
-    part[kPartials + blockIdx.x] = s1;
+    part[gridDim.x + blockIdx.x] = s1;
   }
 }
 
@@ -551,7 +548,7 @@ __global__ void k_spmv_dot_ts(int n, int w, EllNbr nbr,
   a1 = block_sum<kBlock>(a1);
   if (threadIdx.x == 0) {
     part[blockIdx.x] = a0;
-    part[kPartials + blockIdx.x] = a1;
+    part[gridDim.x + blockIdx.x] = a1;
   }
 }
 
@@ -577,7 +574,7 @@ __global__ void k_bicg_update(int n, double *__restrict__ x, double *__restrict_
   d = block_sum<kBlock>(d);
   if (threadIdx.x == 0) {
     part[blockIdx.x] = a;
-    part[kPartials + blockIdx.x] = d;
+    part[gridDim.x + blockIdx.x] = d;
   }
 }
 
@@ -620,7 +617,7 @@ __global__ void k_gm_spmv(int n, int w, const int *__restrict__ nbr, const doubl
   if (i < n) y[i] = ell_ax(i, n, w, nbr, ac, anb, x);
 }
 
-// part[j*kPartials + block] = (V_j, w); blockIdx.y = j
+// part[j gridDim.x + block] = (V_j, w); blockIdx.y = j
 __global__ void k_gm_dots(int n, const double *__restrict__ V, size_t ldv, const double *__restrict__ wv,
                           double *__restrict__ part, const int *__restrict__ flags) {
   if (flags[F_GATE]) return;
@@ -628,7 +625,7 @@ __global__ void k_gm_dots(int n, const double *__restrict__ V, size_t ldv, const
   double s = 0.0;
   for (int i = xcd_block() * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) s += vj[i] * wv[i];
   s = block_sum<kBlock>(s);
-  if (threadIdx.x == 0) part[(size_t)blockIdx.y * kPartials + blockIdx.x] = s;
+  if (threadIdx.x == 0) part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = s;
 }
 
 __device__ double reduce_partials(const double *part, int np);
@@ -638,7 +635,7 @@ __global__ void k_gm_hfin(int np, int m, int col, const double *__restrict__ par
                           const int *__restrict__ flags) {
   if (flags[F_GATE]) return;
   const int j = blockIdx.x;
-  const double a = reduce_partials(part + (size_t)j * kPartials, np);
+  const double a = reduce_partials(part + (size_t)j * np, np);
   if (threadIdx.x == 0) {
     gm[gm_hpass(m) + j] = a;
     gm[gm_h(m) + (size_t)col * (m + 1) + j] += a;
@@ -761,7 +758,7 @@ __global__ void k_gm_resid(int n, int w, const int *__restrict__ nbr, const doub
   s2 = block_sum<kBlock>(s2);
   if (threadIdx.x == 0) {
     part[blockIdx.x] = s1;
-    part[kPartials + blockIdx.x] = s2;
+    part[gridDim.x + blockIdx.x] = s2;
   }
 }
 
@@ -773,7 +770,7 @@ __global__ void k_gm_restart(int np, int m, const double *__restrict__ part, dou
                              double *__restrict__ scal, int *__restrict__ flags) {
   if (flags[F_DONE]) return;
   const double l1 = reduce_partials(part, np);
-  const double l2 = sqrt(reduce_partials(part + kPartials, np));
+  const double l2 = sqrt(reduce_partials(part + np, np));
   if (threadIdx.x != 0) return;
   scal[S_FRES] = l1;
   const bool done = !(l1 > scal[S_RRF] * scal[S_IRES] && flags[F_ITER] < flags[F_ITMAX]);
@@ -831,34 +828,37 @@ struct Post {
   unsigned seq;
 };
 
-// one workgroup of kFinBlock threads combines up to kPartials partials
-// np <= kPartials = kFinR * kFinBlock: a thread's partials i, i + kFinBlock,
-// ... are loaded together, then folded in index order (the slots past np add
-// +0.0, or take the max with the starting -1.0, which changes nothing)
-constexpr int kFinR = kPartials / kFinBlock;
-static_assert(kFinR * kFinBlock == kPartials, "partials per finalise thread");
+// One workgroup of kFinBlock threads combines the np partials of a sum: a
+// thread's partials i, i + kFinBlock, ... are loaded kFinR at a time, then
+// folded in index order (the slots past np add +0.0, or take the max with the
+// starting -1.0, which changes nothing).
+constexpr int kFinR = 8;
 __device__ double reduce_partials(const double *part, int np) {
-  double v[kFinR];
-#pragma unroll
-  for (int u = 0; u < kFinR; ++u) {
-    const int i = threadIdx.x + u * kFinBlock;
-    v[u] = i < np ? part[i] : 0.0;
-  }
   double s = 0.0;
+  for (int base = threadIdx.x; base < np; base += kFinR * kFinBlock) {
+    double v[kFinR];
 #pragma unroll
-  for (int u = 0; u < kFinR; ++u) s += v[u];
+    for (int u = 0; u < kFinR; ++u) {
+      const int i = base + u * kFinBlock;
+      v[u] = i < np ? part[i] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < kFinR; ++u) s += v[u];
+  }
   return block_sum<kFinBlock>(s);
 }
 __device__ double reduce_partials_max(const double *part, int np) {
-  double v[kFinR];
-#pragma unroll
-  for (int u = 0; u < kFinR; ++u) {
-    const int i = threadIdx.x + u * kFinBlock;
-    v[u] = i < np ? part[i] : -1.0;
-  }
   double s = -1.0;
+  for (int base = threadIdx.x; base < np; base += kFinR * kFinBlock) {
+    double v[kFinR];
 #pragma unroll
-  for (int u = 0; u < kFinR; ++u) s = fmax(s, v[u]);
+    for (int u = 0; u < kFinR; ++u) {
+      const int i = base + u * kFinBlock;
+      v[u] = i < np ? part[i] : -1.0;
+    }
+#pragma unroll
+    for (int u = 0; u < kFinR; ++u) s = fmax(s, v[u]);
+  }
   return block_max<kFinBlock>(s);
 }
 
@@ -885,12 +885,12 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
   const double a = op == FIN_POST ? 0.0 : reduce_partials(part, np);
   double b = 0.0, c = 0.0, d = 0.0, e = 0.0;
   if (op == FIN_INIT_NORMS) {
-    b = reduce_partials_max(part + kPartials, np);
-    c = reduce_partials(part + 2 * kPartials, np);
-    d = reduce_partials_max(part + 3 * kPartials, np);
-    e = reduce_partials_max(part + 4 * kPartials, np);
+    b = reduce_partials_max(part + np, np);
+    c = reduce_partials(part + 2 * np, np);
+    d = reduce_partials_max(part + 3 * np, np);
+    e = reduce_partials_max(part + 4 * np, np);
   } else if (op == FIN_BICG_OMEGA || op == FIN_WARM_SCALE || op == FIN_CONV_BICG_RHO) {
-    b = reduce_partials(part + kPartials, np);
+    b = reduce_partials(part + np, np);
   }
   if (threadIdx.x != 0) return;
   bool counted = false; // an iteration ended
@@ -2063,7 +2063,8 @@ int time_spmv(fs_mesh *m, const double *ac, const double *anb, const double *x, 
 namespace fs {
 constexpr int kNoallocMaxCells = FS_NOALLOC_MAX_CELLS;
 constexpr size_t kNoallocVec = (size_t)kNoallocMaxCells;
-constexpr size_t kNoallocPartial = 5 * (size_t)kPartials;
+constexpr size_t kNoallocPartial = 5 * (size_t)8192;
+static_assert(kNoallocMaxCells / kBlock + 8 <= 8192, "partials of the largest mesh without allocation");
 constexpr size_t kNoallocScal = 64, kNoallocFlags = 64;
 static_assert(S_NSLOTS <= (int)kNoallocScal && F_NFLAGS * sizeof(int) <= kNoallocFlags * sizeof(double),
               "scalar and flag slices");
