@@ -447,25 +447,9 @@ template <class T> __device__ __forceinline__ void scatter_cell(const Scatter<T>
 template <int LPR, class T>
 __device__ __forceinline__ T row_offdiag(int i, int lane, int n, int w, EllNbr nbr,
                                          const T *__restrict__ anb, const T *x) {
+  if (LPR == 1)
+    return ell_fold<kStreamLevel>(i, n, w, nbr, anb, x, T(0), [](T acc, T a, T xk) { return acc + a * xk; });
   T s = T(0);
-  if (LPR == 1) {
-    // one lane per row: the row's slots in batches (loads first, then the
-    // terms in slot order)
-    for (int j0 = 0; j0 < w; j0 += kEllBatch) {
-      int k[kEllBatch];
-      T a[kEllBatch], xv[kEllBatch];
-      ell_batch<kEllBatch, kStreamLevel>(nbr, i, n, w, j0, k);
-#pragma unroll
-      for (int u = 0; u < kEllBatch; ++u) {
-        a[u] = ld_mat<kStreamLevel>(&anb[(size_t)min(j0 + u, w - 1) * n + i]);
-        xv[u] = x[k[u] >= 0 ? k[u] : i];
-      }
-#pragma unroll
-      for (int u = 0; u < kEllBatch; ++u)
-        if (j0 + u < w && k[u] >= 0) s += a[u] * xv[u];
-    }
-    return s;
-  }
   for (int j = lane; j < w; j += LPR) {
     const int k = nbr.i32[(size_t)j * n + i];
     if (k >= 0) s += anb[(size_t)j * n + i] * x[k];
@@ -664,21 +648,9 @@ k_enter_resid(int n, int w, EllNbr nbr, const T *__restrict__ ac, const T *__res
   if (b) b[i] = bi;
   const T xi = omega * bi / ac[i];
   x[i] = xi;
-  T s = T(0);
-  for (int j0 = 0; j0 < w; j0 += kEllBatch) {
-    int k[kEllBatch];
-    T a[kEllBatch], xv[kEllBatch];
-    ell_batch<kEllBatch, kStreamLevel>(nbr, i, n, w, j0, k);
-#pragma unroll
-    for (int u = 0; u < kEllBatch; ++u) {
-      const int kk = k[u] >= 0 ? k[u] : i;
-      a[u] = ld_mat<kStreamLevel>(&anb[(size_t)min(j0 + u, w - 1) * n + i]);
-      xv[u] = omega * (T)rhs[kk] / ac[kk];
-    }
-#pragma unroll
-    for (int u = 0; u < kEllBatch; ++u)
-      if (j0 + u < w && k[u] >= 0) s += a[u] * xv[u];
-  }
+  const T s = ell_fold_get<kStreamLevel>(
+      i, n, w, nbr, anb, [=](int k) { return omega * (T)rhs[k] / ac[k]; }, T(0),
+      [](T acc, T a, T xk) { return acc + a * xk; });
   r[i] = bi - ac[i] * xi - s;
 }
 
@@ -745,7 +717,7 @@ __global__ void k_gsc(int cnt, const int *__restrict__ cells, int n, int w, cons
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= cnt) return;
   const int i = cells[t];
-  const T s = ell_fold<kEllBatch>(i, n, w, nbr, anb, (const T *)x, b[i], [](T acc, T a, T xk) { return acc - a * xk; });
+  const T s = ell_fold(i, n, w, nbr, anb, (const T *)x, b[i], [](T acc, T a, T xk) { return acc - a * xk; });
   x[i] = s / ac[i];
 }
 
@@ -757,7 +729,7 @@ __global__ void k_amg_res(int n, int w, const int *__restrict__ nbr, const doubl
   if (flags[0]) return;
   double s = 0.0;
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    const double v = ell_fold<kEllBatch>(i, n, w, nbr, anb, x, b[i] - ac[i] * x[i],
+    const double v = ell_fold(i, n, w, nbr, anb, x, b[i] - ac[i] * x[i],
                                          [](double acc, double a, double xk) { return acc - a * xk; });
     r[i] = v;
     s += fabs(v);

@@ -100,9 +100,8 @@ __device__ __forceinline__ void ell_batch(const EllNbr &nb, int i, int n, int w,
   }
 }
 
-template <int B, bool NT = false, class T, class Op>
-__device__ __forceinline__ T ell_fold(int i, int n, int w, EllNbr nb, const T *__restrict__ anb, const T *x, T acc,
-                                      Op op) {
+template <int B, bool NT, class T, class Get, class Op>
+__device__ __forceinline__ T ell_fold_by(int i, int n, int w, EllNbr nb, const T *__restrict__ anb, Get get, T acc, Op op) {
   for (int j0 = 0; j0 < w; j0 += B) {
     int k[B];
     T a[B], xv[B];
@@ -110,7 +109,7 @@ __device__ __forceinline__ T ell_fold(int i, int n, int w, EllNbr nb, const T *_
 #pragma unroll
     for (int u = 0; u < B; ++u) {
       a[u] = ld_mat<NT>(&anb[(size_t)min(j0 + u, w - 1) * n + i]);
-      xv[u] = x[k[u] >= 0 ? k[u] : i];
+      xv[u] = get(k[u] >= 0 ? k[u] : i);
     }
 #pragma unroll
     for (int u = 0; u < B; ++u)
@@ -119,8 +118,24 @@ __device__ __forceinline__ T ell_fold(int i, int n, int w, EllNbr nb, const T *_
   return acc;
 }
 
-// batch width for a row of w slots: all of a hexahedron's or tetrahedron's
-// slots at once
-constexpr int kEllBatch = 8;
+// The batch holds all slots of a quadrilateral's or tetrahedron's row (4), of
+// a hexahedron's (6), or 8.  It is not always 8: every slot past w costs a
+// gather that is thrown away, and the gathers bound the rows of an irregular
+// mesh: on 2.9 M tetrahedra, one batch of 8 against one of 4, k_spmv_dot took
+// 49 us against 37.5, k_enter_resid 50.8 against 36.7, the FP32 k_sweep 36.1
+// against 27.5; on 2.1 M hexahedra, 8 against 6, k_spmv_dot 36.7 against 33.0.
+template <bool NT = false, class T, class Get, class Op>
+__device__ __forceinline__ T ell_fold_get(int i, int n, int w, EllNbr nb, const T *__restrict__ anb, Get get, T acc,
+                                          Op op) {
+  if (w <= 4) return ell_fold_by<4, NT>(i, n, w, nb, anb, get, acc, op);
+  if (w <= 6) return ell_fold_by<6, NT>(i, n, w, nb, anb, get, acc, op);
+  return ell_fold_by<8, NT>(i, n, w, nb, anb, get, acc, op);
+}
+
+template <bool NT = false, class T, class Op>
+__device__ __forceinline__ T ell_fold(int i, int n, int w, EllNbr nb, const T *__restrict__ anb, const T *x, T acc,
+                                      Op op) {
+  return ell_fold_get<NT>(i, n, w, nb, anb, [x](int k) { return x[k]; }, acc, op);
+}
 
 } // namespace fs

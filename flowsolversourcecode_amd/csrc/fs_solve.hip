@@ -84,7 +84,7 @@ __device__ __forceinline__ double ell_ax(int i, int n, int w, EllNbr nbr,
                                          const double *__restrict__ anb,
                                          const double *__restrict__ x) {
   const double s = ld_mat<kStreamMatrix>(&ac[i]) * x[i];
-  return ell_fold<kEllBatch, kStreamMatrix>(i, n, w, nbr, anb, x, s,
+  return ell_fold<kStreamMatrix>(i, n, w, nbr, anb, x, s,
                              [](double acc, double a, double xk) { return acc + a * xk; });
 }
 
@@ -96,7 +96,7 @@ __device__ __forceinline__ double ell_res(int i, int n, int w, EllNbr nbr,
                                           const double *__restrict__ b,
                                           const double *__restrict__ x) {
   const double r = b[i] - ld_mat<kStreamMatrix>(&ac[i]) * x[i];
-  return ell_fold<kEllBatch, kStreamMatrix>(i, n, w, nbr, anb, x, r,
+  return ell_fold<kStreamMatrix>(i, n, w, nbr, anb, x, r,
                              [](double acc, double a, double xk) { return acc - a * xk; });
 }
 
@@ -466,7 +466,7 @@ __global__ void k_gs_color(int cnt, const int *__restrict__ cells, int n, int w,
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= cnt) return;
   const int i = cells[t];
-  const double s = ell_fold<kEllBatch>(i, n, w, nbr, anb, (const double *)x, bc[i],
+  const double s = ell_fold(i, n, w, nbr, anb, (const double *)x, bc[i],
                                        [](double acc, double a, double xk) { return acc - a * xk; });
   x[i] = s / ac[i];
 }
@@ -589,7 +589,7 @@ __global__ void k_ilu_resid(int n, int w, const int *__restrict__ nbr, const dou
   if (flags[F_DONE]) return;
   const int i = xcd_block() * kBlock + threadIdx.x;
   if (i >= n) return;
-  r[pos[i]] = ell_fold<kEllBatch>(i, n, w, nbr, anb, dphi, -ac[i] * dphi[i] + bc[i],
+  r[pos[i]] = ell_fold(i, n, w, nbr, anb, dphi, -ac[i] * dphi[i] + bc[i],
                                   [](double acc, double a, double xk) { return acc - a * xk; });
 }
 
