@@ -408,6 +408,14 @@ __global__ void k_to(int n, const double *__restrict__ a, T *__restrict__ b) {
 // sweep from 4.7 to 4.1 TB/s).
 constexpr bool kStreamLevel = false;
 
+// The done flag, as a load that waits for nothing and is waited for with the
+// loads that follow it (a null test around it would wait there); any is any
+// readable address of the kernel.
+__device__ __forceinline__ int done_flag(const int *flags, const void *any) {
+  const int v = *(flags ? flags : (const int *)any);
+  return flags ? v : 0;
+}
+
 // The prolongation of a level's correction into the next finer level: the
 // kernel that forms a coarse cell's value adds alpha times it to the cell's
 // members (x[mem[q]], q in [mptr[p], mptr[p+1])).  Every finer cell belongs to
@@ -424,23 +432,34 @@ template <class T> struct Scatter {
   T alpha;
 };
 
-// members lane, lane + step, ... of cell p, loads of a batch first
-template <class T> __device__ __forceinline__ void scatter_cell(const Scatter<T> &sc, int p, T v, int lane, int step) {
-  const int q1 = sc.mptr[p + 1];
-  const T add = sc.alpha * v;
-  constexpr int B = 4;
-  for (int q = sc.mptr[p] + lane; q < q1; q += B * step) {
-    int id[B];
-    T xv[B];
+// A cell's part of the scatter on LPR lanes: the first 16 members' values are
+// loaded beside the row's own operands, before the cell's value is known.
+template <int LPR, class T> struct ScatterRow {
+  static constexpr int B = LPR < 16 ? 16 / LPR : 1;
+  int q, q1, id[B];
+  T xv[B];
+  // begin: the first member of this lane; end: the members' end
+  __device__ __forceinline__ void members(const Scatter<T> &sc, int begin, int end) {
+    q = begin;
+    q1 = end;
 #pragma unroll
-    for (int u = 0; u < B; ++u) id[u] = sc.mem[min(q + u * step, q1 - 1)];
+    for (int u = 0; u < B; ++u) id[u] = sc.mem[min(q + u * LPR, q1 - 1)];
+  }
+  __device__ __forceinline__ void values(const Scatter<T> &sc) {
 #pragma unroll
     for (int u = 0; u < B; ++u) xv[u] = sc.x[id[u]];
+  }
+  __device__ __forceinline__ void add(const Scatter<T> &sc, T v) {
+    const T a = sc.alpha * v;
 #pragma unroll
     for (int u = 0; u < B; ++u)
-      if (q + u * step < q1) sc.x[id[u]] = xv[u] + add;
+      if (q + u * LPR < q1) sc.x[id[u]] = xv[u] + a;
+    for (int k = q + B * LPR; k < q1; k += LPR) {
+      const int i = sc.mem[k];
+      sc.x[i] = sc.x[i] + a;
+    }
   }
-}
+};
 
 // sum_j anb_ij x_j over the slots of row i, spread over LPR consecutive
 // lanes and combined with shuffles
@@ -491,16 +510,55 @@ k_resid(int n, int w, EllNbr nbr, const T *__restrict__ ac, const T *__restrict_
 
 // ---- coarse levels in row-major CSR (no padding; a row's entries are
 // contiguous, so the LPR lanes of a row read one segment)
-template <int LPR, class T, class V>
-__device__ __forceinline__ T csr_offdiag(int i, int lane, const int *__restrict__ rp, const int *__restrict__ col,
-                                         const V *__restrict__ val, const T *x, bool ok) {
-  T s = T(0);
-  if (ok)
-    for (int q = rp[i] + lane; q < rp[i + 1]; q += LPR) s += val[q] * x[col[q]];
+//
+// The levels between the finest and the dense map are too small to use the
+// chip's bandwidth: a launch on them lasts as long as its chain of dependent
+// loads, about 0.7 us each.  So a row's entries go in batches of kCsrBatch per
+// lane (columns and values, then the gathers: one round for up to
+// kCsrBatch LPR entries), the done flag is read beside the first loads
+// instead of ahead of them, and what a kernel needs after its sum is loaded
+// before it.  On the levels of 2.9 M tetrahedra k_resid_restrict_csr went from
+// 5.7 to 4.4 us, k_sweep_csr from 4.1 to 3.4 (16 lanes) and from 5.8 to 4.8 (8
+// lanes, prolongating), k_dense_apply from 5.1 to 4.6.
+constexpr int kCsrBatch = 4;
+template <int LPR, class T, class V> struct CsrRow {
+  int q, q1, c[kCsrBatch];
+  V a[kCsrBatch];
+  T xv[kCsrBatch];
+  // entries q0 + lane, q0 + lane + LPR, ... of a row's [q0, end)
+  __device__ __forceinline__ void entries(int at, int end, const int *__restrict__ col, const V *__restrict__ val) {
+    q = at;
+    q1 = end;
 #pragma unroll
-  for (int off = LPR / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, LPR);
-  return s;
-}
+    for (int u = 0; u < kCsrBatch; ++u) {
+      const int e = max(min(q + u * LPR, q1 - 1), 0);
+      c[u] = col[e];
+      a[u] = val[e];
+    }
+  }
+  __device__ __forceinline__ void gather(const T *x) {
+#pragma unroll
+    for (int u = 0; u < kCsrBatch; ++u) xv[u] = x[c[u]];
+  }
+  __device__ __forceinline__ T sum(T s) const {
+#pragma unroll
+    for (int u = 0; u < kCsrBatch; ++u)
+      if (q + u * LPR < q1) s += a[u] * xv[u];
+    return s;
+  }
+  // the row's sum on all of its lanes, the first batch being gathered
+  __device__ __forceinline__ T finish(const int *__restrict__ col, const V *__restrict__ val, const T *x) {
+    T s = sum(T(0));
+    while (q + kCsrBatch * LPR < q1) {
+      entries(q + kCsrBatch * LPR, q1, col, val);
+      gather(x);
+      s = sum(s);
+    }
+#pragma unroll
+    for (int off = LPR / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, LPR);
+    return s;
+  }
+};
 
 // SC: the level's last sweep, which also prolongates its result
 template <int LPR, class T, bool SC>
@@ -508,16 +566,26 @@ __global__ void __launch_bounds__(kBlock)
 k_sweep_csr(int n, const int *__restrict__ rp, const int *__restrict__ col, const T *__restrict__ val,
             const T *__restrict__ ac, const T *__restrict__ b, const T *x, T omega, T *xn, Scatter<T> sc,
             const int *__restrict__ flags) {
-  if (flags && flags[0]) return;
+  const int done = done_flag(flags, rp);
   const int t = xcd_block() * kBlock + threadIdx.x;
-  const int i = t / LPR, lane = t % LPR;
-  const bool ok = i < n;
-  const T s = csr_offdiag<LPR, T>(ok ? i : 0, lane, rp, col, val, x, ok);
+  const int i = min(t / LPR, n - 1), lane = t % LPR;
+  const bool ok = t / LPR < n;
+  int q0 = rp[i], q1 = rp[i + 1], m0 = 0, m1 = 0;
+  const T ai = ac[i], bi = b[i], xi = x[i];
+  if (SC) m0 = sc.mptr[i], m1 = sc.mptr[i + 1];
+  in_register(q0);
+  if (done) return;
+  CsrRow<LPR, T, T> row;
+  ScatterRow<LPR, T> to;
+  row.entries(q0 + lane, q1, col, val);
+  if (SC) to.members(sc, m0 + lane, m1);
+  row.gather(x);
+  if (SC) to.values(sc);
+  const T s = row.finish(col, val, x);
   if (!ok) return;
-  const T xi = x[i];
-  const T v = xi + omega * (b[i] - ac[i] * xi - s) / ac[i]; // the same on the row's lanes
+  const T v = xi + omega * (bi - ai * xi - s) / ai; // the same on the row's lanes
   if (lane == 0) xn[i] = v;
-  if (SC) scatter_cell<T>(sc, i, v, lane, LPR);
+  if (SC) to.add(sc, v);
 }
 
 // ---- large coarse levels in sliced ELL: slices of 64 rows (one wavefront),
@@ -589,30 +657,38 @@ k_resid_sell(int nslots, const int *__restrict__ ptr, const int *__restrict__ ro
 // and the groups' sums are combined in a fixed butterfly, so the result is
 // deterministic and a coarse cell waits on ceil(members / MPR) member rows
 // instead of all of them.
+// rows[q] is the range of member q's entries, beside mem[q].
 template <int LPR, int MPR, class T>
 __global__ void __launch_bounds__(kBlock)
-k_resid_restrict_csr(int nc, const int *__restrict__ mptr, const int *__restrict__ mem, const int *__restrict__ rp,
+k_resid_restrict_csr(int nc, const int *__restrict__ mptr, const int *__restrict__ mem, const int2 *__restrict__ rows,
                      const int *__restrict__ col, const T *__restrict__ val, const T *__restrict__ ac,
                      const T *__restrict__ b, const T *__restrict__ x, T *__restrict__ bc, const T *__restrict__ acc,
                      T *__restrict__ xc, T omega, int mode, const int *__restrict__ flags) {
   constexpr int G = LPR * MPR;
   static_assert(64 % G == 0 && kBlock % 64 == 0, "a coarse cell's lanes must share a wavefront");
-  if (flags && flags[0]) return;
+  const int done = done_flag(flags, mptr);
   const int t = xcd_block() * kBlock + threadIdx.x;
-  const int p = t / G, lane = t % LPR, grp = (t % G) / LPR;
-  const bool ok = p < nc;
-  const int q0 = ok ? mptr[p] : 0, q1 = ok ? mptr[p + 1] : 0;
+  const int p = min(t / G, nc - 1), lane = t % LPR, grp = (t % G) / LPR;
+  int q0 = mptr[p], q1 = mptr[p + 1];
+  const T ap = mode == 1 ? acc[p] : T(1);
+  in_register(q0);
+  if (done) return;
   T sum = T(0);
   for (int q = q0 + grp; q < q1; q += MPR) { // the same trip count on the LPR lanes of a group
     const int i = mem[q];
-    const T s = csr_offdiag<LPR, T>(i, lane, rp, col, val, x, true);
-    sum = sum + (b[i] - ac[i] * x[i] - s);
+    const int2 e = rows[q];
+    const T bi = b[i], ai = ac[i], xi = x[i];
+    CsrRow<LPR, T, T> row;
+    row.entries(e.x + lane, e.y, col, val);
+    row.gather(x);
+    const T s = row.finish(col, val, x);
+    sum = sum + (bi - ai * xi - s);
   }
 #pragma unroll
   for (int off = LPR; off < G; off <<= 1) sum += __shfl_xor(sum, off, G);
-  if (ok && lane == 0 && grp == 0) {
+  if (t < nc * G && lane == 0 && grp == 0) {
     bc[p] = sum;
-    if (mode == 1) xc[p] = omega * sum / acc[p];
+    if (mode == 1) xc[p] = omega * sum / ap;
     else if (mode == 2) xc[p] = T(0);
   }
 }
@@ -661,10 +737,12 @@ template <class T>
 __global__ void k_restrict(int nc, const int *__restrict__ mptr, const int *__restrict__ mem,
                            const T *__restrict__ rf, T *__restrict__ bc, const T *__restrict__ acc,
                            T *__restrict__ xc, T omega, int mode, const int *__restrict__ flags) {
-  if (flags && flags[0]) return;
+  const int done = done_flag(flags, mptr);
   const int p = blockIdx.x * kBlock + threadIdx.x;
   if (p >= nc) return;
-  const int q0 = mptr[p], q1 = mptr[p + 1];
+  int q0 = mptr[p], q1 = mptr[p + 1];
+  in_register(q0);
+  if (done) return;
   T s = T(0);
   // members in batches: their indices, then their residuals, then the sum
   // in member order
@@ -912,24 +990,38 @@ k_dense_apply(int n, const T *__restrict__ C, const T *__restrict__ b, T *__rest
   __shared__ T xs[kDenseRows];
   const int i0 = blockIdx.x * kDenseRows, cnt = n * LPC; // 16-byte elements of the strip
   const V *strip = (const V *)(C + (size_t)i0 * n);
-  const int done = flags ? flags[0] : 0; // beside the other loads, tested before the stores
-  double acc[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) acc[k] = 0.0;
-  for (int e0 = threadIdx.x; e0 < cnt; e0 += B * kDenseThreads) {
-    V c[B];
-    T v[B];
+  const int done = done_flag(flags, C); // tested before the stores
+  // the strip's members: this thread's first one is loaded beside the products
+  const int m0 = SC ? sc.mptr[i0] + (int)threadIdx.x : 0, m1 = SC ? sc.mptr[min(i0 + kDenseRows, n)] : 0;
+  int mf = 0, mp = 0;
+  T mx = T(0);
+  V c[B];
+  T v[B];
+  const auto fetch = [&](int e0) {
 #pragma unroll
     for (int u = 0; u < B; ++u) {
       const int e = min(e0 + u * kDenseThreads, cnt - 1);
       c[u] = strip[e];
       v[u] = b[e / LPC];
     }
+  };
+  fetch(threadIdx.x);
+  if (SC) mf = sc.mem[min(m0, m1 - 1)];
+  double acc[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) acc[k] = 0.0;
+  const auto add = [&](int e0) {
 #pragma unroll
     for (int u = 0; u < B; ++u)
       if (e0 + u * kDenseThreads < cnt)
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] += (double)c[u][k] * (double)v[u];
+  };
+  if (SC) mp = parent[mf] - i0, mx = sc.x[mf];
+  add(threadIdx.x);
+  for (int e0 = threadIdx.x + B * kDenseThreads; e0 < cnt; e0 += B * kDenseThreads) {
+    fetch(e0);
+    add(e0);
   }
   if (done) return;
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -952,8 +1044,8 @@ k_dense_apply(int n, const T *__restrict__ C, const T *__restrict__ b, T *__rest
   }
   if constexpr (SC) {
     __syncthreads();
-    const int q1 = sc.mptr[min(i0 + kDenseRows, n)];
-    for (int q = sc.mptr[i0] + threadIdx.x; q < q1; q += kDenseThreads) {
+    if (m0 < m1) sc.x[mf] = mx + sc.alpha * xs[mp];
+    for (int q = m0 + kDenseThreads; q < m1; q += kDenseThreads) {
       const int f = sc.mem[q];
       sc.x[f] = sc.x[f] + sc.alpha * xs[parent[f] - i0];
     }
@@ -1044,6 +1136,7 @@ struct DLevel {
   DevBuf<int> color_cells;
   DevBuf<int> parent;            // 0-based parent in the next level
   DevBuf<int> mptr, mem;         // members of this level's aggregates (coarse)
+  DevBuf<int2> mrow;             // beside mem: the member's entries in the finer level's CSR
   DevBuf<int> gptr;
   DevBuf<int> gsrc;               // 32-bit: fine n + n w stays below 2^31
   int gne = 0;
@@ -1157,6 +1250,7 @@ static void build_hierarchy(fs_mesh *m, const double *ac, const double *anb) {
     ++nl;
   }
   H->lev.resize(nl);
+  std::vector<int> rp_f; // row starts of the finer level's CSR
   for (int l = 0; l < nl; ++l) {
     DLevel &D = H->lev[l];
     HostLevel &h = H->host[l];
@@ -1197,6 +1291,11 @@ static void build_hierarchy(fs_mesh *m, const double *ac, const double *anb) {
       for (int i = 0; i < f.n; ++i) mem[fill[f.parent[i] - 1]++] = i;
       D.mptr.upload(mptr, s);
       D.mem.upload(mem, s);
+      if (l > 1) {
+        std::vector<int2> mrow(f.n);
+        for (int q = 0; q < f.n; ++q) mrow[q] = make_int2(rp_f[mem[q]], rp_f[mem[q] + 1]);
+        D.mrow.upload(mrow, s);
+      }
       std::vector<int> rp(h.n + 1, 0), col, pos((size_t)h.n * h.w, -1);
       for (int i = 0; i < h.n; ++i) {
         for (int j = 0; j < h.w; ++j) {
@@ -1227,6 +1326,7 @@ static void build_hierarchy(fs_mesh *m, const double *ac, const double *anb) {
       D.csr_rp.upload(rp, s);
       D.csr_col.upload(col, s);
       D.csr_pos.upload(pos, s);
+      rp_f = std::move(rp);
       D.val64.alloc(nval);
       D.val32.alloc(nval);
       // padded sliced entries are never written by the Galerkin kernel
@@ -1392,44 +1492,19 @@ static int csr_lpr(const DLevel &D) {
   return a <= 6.0 ? 4 : a <= 16.0 ? 8 : 16;
 }
 
-// member groups per coarse cell in the fused residual-restriction: up to
-// kRestrictGroups, as many as fit one wavefront with LPR lanes each
-constexpr int kRestrictGroups = 8;
-// rows wider than 16 entries are restricted with 8 lanes per member row and
-// 8 member groups rather than 16 lanes and 4 groups
-constexpr bool kRestrictNarrow = true;
-template <int LPR> constexpr int restrict_groups() { return kRestrictGroups < 64 / LPR ? kRestrictGroups : 64 / LPR; }
-
-// residual of coarse level D restricted into C (plus C's first sweep)
+// residual of coarse level D restricted into C (plus C's first sweep): 8 member
+// groups per coarse cell of 4 lanes (rows of up to 6 entries) or 8 lanes each
+// (with 16 lanes, and so 4 groups, wide rows took longer)
 template <class T>
 static void launch_resid_restrict(fs_mesh *m, DLevel &D, DLevel &C, const T *b, const T *x, T om, int mode,
                                   const int *flags) {
-  hipStream_t s = m->stream;
-  const int *rp = D.csr_rp.p, *col = D.csr_col.p;
-  const T *val = LV<T>::val(D), *ac = LV<T>::ac(D);
-  constexpr int M4 = restrict_groups<4>(), M8 = restrict_groups<8>(), M16 = restrict_groups<16>();
-  switch (csr_lpr(D)) {
-  case 4:
-    hipLaunchKernelGGL((k_resid_restrict_csr<4, M4, T>), dim3(gfor(C.n * 4 * M4)), dim3(kBlock), 0, s, C.n,
-                       C.mptr.p, C.mem.p, rp, col, val, ac, b, x, LV<T>::b(C), LV<T>::ac(C), LV<T>::x(C), om, mode,
-                       flags);
-    break;
-  case 8:
-    hipLaunchKernelGGL((k_resid_restrict_csr<8, M8, T>), dim3(gfor(C.n * 8 * M8)), dim3(kBlock), 0, s, C.n,
-                       C.mptr.p, C.mem.p, rp, col, val, ac, b, x, LV<T>::b(C), LV<T>::ac(C), LV<T>::x(C), om, mode,
-                       flags);
-    break;
-  default:
-    if (kRestrictNarrow) {
-      hipLaunchKernelGGL((k_resid_restrict_csr<8, M8, T>), dim3(gfor(C.n * 8 * M8)), dim3(kBlock), 0, s, C.n,
-                         C.mptr.p, C.mem.p, rp, col, val, ac, b, x, LV<T>::b(C), LV<T>::ac(C), LV<T>::x(C), om, mode,
-                         flags);
-      break;
-    }
-    hipLaunchKernelGGL((k_resid_restrict_csr<16, M16, T>), dim3(gfor(C.n * 16 * M16)), dim3(kBlock), 0, s, C.n,
-                       C.mptr.p, C.mem.p, rp, col, val, ac, b, x, LV<T>::b(C), LV<T>::ac(C), LV<T>::x(C), om, mode,
-                       flags);
-  }
+  const auto go = [&](auto kernel, int lanes) {
+    hipLaunchKernelGGL(kernel, dim3(gfor(C.n * lanes)), dim3(kBlock), 0, m->stream, C.n, C.mptr.p, C.mem.p, C.mrow.p,
+                       D.csr_col.p, LV<T>::val(D), LV<T>::ac(D), b, x, LV<T>::b(C), LV<T>::ac(C), LV<T>::x(C), om,
+                       mode, flags);
+  };
+  if (csr_lpr(D) == 4) go(k_resid_restrict_csr<4, 8, T>, 4 * 8);
+  else go(k_resid_restrict_csr<8, 8, T>, 8 * 8);
 }
 
 // one damped-Jacobi sweep on a coarse grid-wide level in CSR, lanes per row by

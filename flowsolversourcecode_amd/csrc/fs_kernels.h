@@ -42,6 +42,10 @@ template <int BS, class T> __device__ __forceinline__ T block_max(T v) {
   return out;
 }
 
+// The value v is in a register here: a load that feeds it was issued, with
+// those before it, ahead of what follows.
+template <class V> __device__ __forceinline__ void in_register(V &v) { asm volatile("" : "+v"(v)); }
+
 // MI355X dispatches consecutive workgroups round-robin over its 8 XCDs, each
 // with a private L2.  Remapping the block index gives every XCD one
 // contiguous range of cells, so the plane neighbours a gather touches are

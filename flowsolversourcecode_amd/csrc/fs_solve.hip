@@ -833,19 +833,32 @@ struct Post {
 // folded in index order (the slots past np add +0.0, or take the max with the
 // starting -1.0, which changes nothing).
 constexpr int kFinR = 8;
-__device__ double reduce_partials(const double *part, int np) {
-  double s = 0.0;
-  for (int base = threadIdx.x; base < np; base += kFinR * kFinBlock) {
-    double v[kFinR];
+struct Partials {
+  double v[kFinR];
+  __device__ __forceinline__ void load(const double *part, int np, int base) {
 #pragma unroll
     for (int u = 0; u < kFinR; ++u) {
       const int i = base + u * kFinBlock;
       v[u] = i < np ? part[i] : 0.0;
     }
-#pragma unroll
-    for (int u = 0; u < kFinR; ++u) s += v[u];
   }
-  return block_sum<kFinBlock>(s);
+  // the sum, the first kFinR kFinBlock partials being loaded
+  __device__ __forceinline__ double sum(const double *part, int np) {
+    double s = 0.0;
+    for (int base = threadIdx.x;;) {
+#pragma unroll
+      for (int u = 0; u < kFinR; ++u) s += v[u];
+      base += kFinR * kFinBlock;
+      if (base >= np) break;
+      load(part, np, base);
+    }
+    return block_sum<kFinBlock>(s);
+  }
+};
+__device__ double reduce_partials(const double *part, int np) {
+  Partials p;
+  p.load(part, np, threadIdx.x);
+  return p.sum(part, np);
 }
 __device__ double reduce_partials_max(const double *part, int np) {
   double s = -1.0;
@@ -862,13 +875,23 @@ __device__ double reduce_partials_max(const double *part, int np) {
   return block_max<kFinBlock>(s);
 }
 
-// rho = (r0, r) and beta of BiCGSTAB.  Breakdown (rho or the last omega
-// zero, or a non-finite beta, as on a singular system whose right-hand side
-// carries round-off outside the range): stop with the current iterate.
-__device__ void bicg_rho(double a, double *__restrict__ scal, int *__restrict__ flags) {
-  if (flags[F_ITER] > 0) {
-    const double beta = (a / scal[S_RHO]) * (scal[S_ALPHA] / scal[S_OMEGA]);
-    if (scal[S_OMEGA] == 0.0 || !isfinite(beta)) {
+// What a solve's scalars held before this kernel
+struct FinState {
+  double rho, alpha, omega, rrf, ires, bknum, bkden;
+  int done, iter, itmax;
+  __device__ FinState(const double *scal, const int *flags)
+      : rho(scal[S_RHO]), alpha(scal[S_ALPHA]), omega(scal[S_OMEGA]), rrf(scal[S_RRF]), ires(scal[S_IRES]),
+        bknum(scal[S_BKNUM]), bkden(scal[S_BKDEN]), done(flags[F_DONE]), iter(flags[F_ITER]), itmax(flags[F_ITMAX]) {}
+};
+
+// rho = (r0, r) and beta of BiCGSTAB after iter iterations.  Breakdown (rho or
+// the last omega zero, or a non-finite beta, as on a singular system whose
+// right-hand side carries round-off outside the range): stop with the current
+// iterate.
+__device__ void bicg_rho(double a, int iter, const FinState &in, double *__restrict__ scal, int *__restrict__ flags) {
+  if (iter > 0) {
+    const double beta = (a / in.rho) * (in.alpha / in.omega);
+    if (in.omega == 0.0 || !isfinite(beta)) {
       flags[F_DONE] = 1;
       return;
     }
@@ -878,19 +901,30 @@ __device__ void bicg_rho(double a, double *__restrict__ scal, int *__restrict__ 
   if (a == 0.0) flags[F_DONE] = 1;
 }
 
+// One workgroup, so it lasts as long as its chain of loads: the solve's
+// scalars and the partials are loaded together, and the done flag is tested
+// after both.
 __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ part,
                       double *__restrict__ scal, int *__restrict__ flags, SolveStart st, Post to) {
   const bool always = op == FIN_INIT_NORMS || op == FIN_TRUE_RES || op == FIN_POST;
-  if (!always && flags[F_DONE]) return;
-  const double a = op == FIN_POST ? 0.0 : reduce_partials(part, np);
+  const FinState in(scal, flags);
+  const bool two = op == FIN_BICG_OMEGA || op == FIN_WARM_SCALE || op == FIN_CONV_BICG_RHO;
+  Partials first, second;
+  if (op != FIN_POST) {
+    first.load(part, np, threadIdx.x);
+    if (two) second.load(part + np, np, threadIdx.x);
+    in_register(first.v[0]);
+  }
+  if (!always && in.done) return;
+  const double a = op == FIN_POST ? 0.0 : first.sum(part, np);
   double b = 0.0, c = 0.0, d = 0.0, e = 0.0;
   if (op == FIN_INIT_NORMS) {
     b = reduce_partials_max(part + np, np);
     c = reduce_partials(part + 2 * np, np);
     d = reduce_partials_max(part + 3 * np, np);
     e = reduce_partials_max(part + 4 * np, np);
-  } else if (op == FIN_BICG_OMEGA || op == FIN_WARM_SCALE || op == FIN_CONV_BICG_RHO) {
-    b = reduce_partials(part + np, np);
+  } else if (two) {
+    b = second.sum(part + np, np);
   }
   if (threadIdx.x != 0) return;
   bool counted = false; // an iteration ended
@@ -916,38 +950,39 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
   }
   case FIN_PBCG_BK: {
     scal[S_BKNUM] = a;
-    if (flags[F_ITER] > 0) scal[S_BK] = a / (scal[S_BKDEN] + 1.0e-10);
+    if (in.iter > 0) scal[S_BK] = a / (in.bkden + 1.0e-10);
     scal[S_BKDEN] = a;
     break;
   }
   case FIN_PBCG_AK:
     scal[S_AKDEN] = a;
-    scal[S_AK] = scal[S_BKNUM] / (a + 1.0e-10);
+    scal[S_AK] = in.bknum / (a + 1.0e-10);
     break;
   case FIN_CONV: {
     counted = true;
     scal[S_FRES] = a;
-    const int it = flags[F_ITER] + 1;
+    const int it = in.iter + 1;
     flags[F_ITER] = it;
     // NaN residuals end the loop as well
-    flags[F_DONE] = !(a > scal[S_RRF] * scal[S_IRES] && it < flags[F_ITMAX]);
+    flags[F_DONE] = !(a > in.rrf * in.ires && it < in.itmax);
     break;
   }
   case FIN_BICG_RHO:
-    bicg_rho(a, scal, flags);
+    bicg_rho(a, in.iter, in, scal, flags);
     break;
   case FIN_CONV_BICG_RHO: {
     counted = true;
     scal[S_FRES] = a;
-    const int it = flags[F_ITER] + 1;
+    const int it = in.iter + 1;
     flags[F_ITER] = it;
-    flags[F_DONE] = !(a > scal[S_RRF] * scal[S_IRES] && it < flags[F_ITMAX]);
-    if (!flags[F_DONE]) bicg_rho(b, scal, flags);
+    const bool more = a > in.rrf * in.ires && it < in.itmax;
+    flags[F_DONE] = !more;
+    if (more) bicg_rho(b, it, in, scal, flags);
     break;
   }
   case FIN_BICG_ALPHA:
     scal[S_RV] = a;
-    scal[S_ALPHA] = (a != 0.0) ? scal[S_RHO] / a : 0.0;
+    scal[S_ALPHA] = (a != 0.0) ? in.rho / a : 0.0;
     break;
   case FIN_BICG_OMEGA:
     scal[S_TS] = a;
@@ -960,8 +995,8 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
   case FIN_POST:
     break;
   case FIN_CG_RHO: {
-    if (flags[F_ITER] > 0) {
-      const double beta = a / scal[S_RHO];
+    if (in.iter > 0) {
+      const double beta = a / in.rho;
       if (!isfinite(beta)) {
         flags[F_DONE] = 1; // breakdown: keep the iterate
         break;
@@ -973,19 +1008,19 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
     break;
   }
   case FIN_WARM:
-    flags[F_REJECT] = !(a <= scal[S_IRES]);
+    flags[F_REJECT] = !(a <= in.ires);
     break;
   case FIN_WARM_SCALE:
     scal[S_GAMMA] = (b > 0.0 && isfinite(a / b)) ? a / b : 0.0;
     break;
-  case FIN_CG_ALPHA:
+  case FIN_CG_ALPHA: {
     scal[S_RV] = a;
-    scal[S_ALPHA] = (a != 0.0) ? scal[S_RHO] / a : 0.0;
-    if (a == 0.0 || !isfinite(scal[S_ALPHA])) {
-      scal[S_ALPHA] = 0.0;
-      flags[F_DONE] = 1;
-    }
+    const double alpha = (a != 0.0) ? in.rho / a : 0.0;
+    const bool fine = a != 0.0 && isfinite(alpha);
+    scal[S_ALPHA] = fine ? alpha : 0.0;
+    if (!fine) flags[F_DONE] = 1;
     break;
+  }
   }
   if (op == FIN_POST) {
     for (int k = 0; k < S_NSLOTS; ++k) to.box->scal[k] = scal[k];
