@@ -471,6 +471,54 @@ __global__ void k_gs_color(int cnt, const int *__restrict__ cells, int n, int w,
   x[i] = s / ac[i];
 }
 
+// The system in colour order: row t is that of cell cells[t], a colour's rows
+// one after the other (ELL as before, the neighbours cell numbers).  In cell
+// order a colour's rows are every third or fourth one of an irregular mesh, so
+// each colour's launch fetched the lines of the whole matrix.
+struct GsRows {
+  const int *pos = nullptr, *nbr = nullptr;          // position of a cell; neighbours
+  double *ac = nullptr, *anb = nullptr, *bc = nullptr;
+};
+
+__global__ void k_gs_rows(int n, int w, const double *__restrict__ ac, const double *__restrict__ anb,
+                          const double *__restrict__ bc, GsRows g) {
+  const int i = xcd_block() * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const int t = g.pos[i];
+  g.ac[t] = ac[i];
+  g.bc[t] = bc[i];
+  for (int j0 = 0; j0 < w; j0 += 4) {
+    double a[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a[u] = anb[(size_t)min(j0 + u, w - 1) * n + i];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (j0 + u < w) g.anb[(size_t)(j0 + u) * n + t] = a[u];
+  }
+}
+
+__global__ void k_gs_order(int n, int w, const int *__restrict__ cells, const int *__restrict__ nbr,
+                           int *__restrict__ pos, int *__restrict__ out) {
+  const int t = xcd_block() * kBlock + threadIdx.x;
+  if (t >= n) return;
+  const int i = cells[t];
+  pos[i] = t;
+  for (int j = 0; j < w; ++j) out[(size_t)j * n + t] = nbr[(size_t)j * n + i];
+}
+
+// k_gs_color over rows t0 ... t0 + cnt - 1 of the colour order: the same
+// values in the same order.
+__global__ void k_gs_rows_color(int t0, int cnt, const int *__restrict__ cells, int n, int w, GsRows g,
+                                double *__restrict__ x, const int *__restrict__ flags) {
+  if (flags && flags[F_DONE]) return;
+  const int q = xcd_block() * kBlock + threadIdx.x;
+  if (q >= cnt) return;
+  const int t = t0 + q;
+  const double s = ell_fold(t, n, w, EllNbr(g.nbr), (const double *)g.anb, (const double *)x, g.bc[t],
+                            [](double acc, double a, double xk) { return acc - a * xk; });
+  x[cells[t]] = s / g.ac[t];
+}
+
 // ---- generic vector kernels for the Krylov solvers
 
 // partial dots: out0 = sum a*b, and if c: out1 = sum c*d
@@ -1276,6 +1324,9 @@ struct SolveWork {
   DevBuf<int> tlin, tsrc;
   std::vector<int> color_ptr;
   DevBuf<int> color_cells;
+  DevBuf<int> gs_ints;    // the rows in colour order (GsRows), for the meshes gs_by_rows() names
+  DevBuf<double> gs_vals;
+  GsRows gs;
   DevBuf<double> dc;
 };
 
@@ -1354,6 +1405,17 @@ static void precompute_ilu_sweep(fs_mesh *m, const IluDiag &diag, IluSweep &S) {
   S.ready = true;
 }
 
+// Whether Gauss-Seidel copies its system into colour order (one pass over the
+// matrix, read and written) and then reads a colour's rows from there: with
+// three colours and more, on rows that overflow the L2s.  A solve of about
+// three iterations in cell order and in colour order, four colours of
+// tetrahedra: 105456 rows 187 and 191 us, 235824 rows 235 and 193, 663552 rows
+// 337 and 271, 2919840 rows 920 and 650.  With the two colours of hexahedra a
+// colour reads its half of the lines twice at worst and the copy pays little:
+// 262144 rows 154 and 158 us, 2048383 rows 450 and 433.
+constexpr size_t kGsRowsSlots = 800000;
+static bool gs_by_rows(int n, int w, int colors) { return colors >= 3 && (size_t)n * w >= kGsRowsSlots; }
+
 int mesh_prepare_solver(fs_mesh *m) {
   auto *sw = new SolveWork();
   m->solve_work = sw;
@@ -1369,6 +1431,17 @@ int mesh_prepare_solver(fs_mesh *m) {
   std::vector<int> cells;
   greedy_colors(m->n, m->w, nbr0.data(), sw->color_ptr, cells);
   sw->color_cells.upload(cells, m->stream);
+  // (a mesh numbered colour by colour is in that order as it is)
+  if (gs_by_rows(m->n, m->w, (int)sw->color_ptr.size() - 1) && !std::is_sorted(cells.begin(), cells.end())) {
+    const size_t n = m->n, w = m->w;
+    sw->gs_ints.alloc((w + 1) * n);
+    sw->gs_vals.alloc((w + 2) * n);
+    int *ip = sw->gs_ints.p;
+    double *vp = sw->gs_vals.p;
+    hipLaunchKernelGGL(k_gs_order, dim3(grid_for(m->n)), dim3(kBlock), 0, m->stream, m->n, m->w, sw->color_cells.p,
+                       m->d_nbr.p, ip, ip + n);
+    sw->gs = GsRows{ip, ip + n, vp, vp + 2 * n, vp + n};
+  }
   sw->dc.alloc(m->n);
   for (auto &v : m->v) v.alloc(m->n);
   m->partial.alloc(5 * kPartials);
@@ -1851,19 +1924,24 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     // forward pass after the first at colour 1 (the residual check between
     // iterations leaves x alone).
     bool first = true;
+    const bool rows = sw.gs.pos;
+    if (rows) hipLaunchKernelGGL(k_gs_rows, dim3(ge), dim3(kBlock), 0, s, n, w, ac, anb, bc, sw.gs);
+    const auto color = [&](int c) {
+      const int b = sw.color_ptr[c], e = sw.color_ptr[c + 1];
+      if (rows)
+        hipLaunchKernelGGL(k_gs_rows_color, dim3(grid_for(e - b)), dim3(kBlock), 0, s, b, e - b, sw.color_cells.p, n, w,
+                           sw.gs, dphi, flags);
+      else
+        hipLaunchKernelGGL(k_gs_color, dim3(grid_for(e - b)), dim3(kBlock), 0, s, e - b, sw.color_cells.p + b, n, w, nb,
+                           ac, anb, bc, dphi, flags);
+    };
     run_iterations(m, itmax, [&]() {
       const int nc = (int)sw.color_ptr.size() - 1;
       for (int c = first ? 0 : 1; c < nc; ++c) {
         if (solve_done(m)) return; // the rest would return at once
-        const int b = sw.color_ptr[c], e = sw.color_ptr[c + 1];
-        hipLaunchKernelGGL(k_gs_color, dim3(grid_for(e - b)), dim3(kBlock), 0, s, e - b,
-                           sw.color_cells.p + b, n, w, nb, ac, anb, bc, dphi, flags);
+        color(c);
       }
-      for (int c = nc - 2; c >= 0; --c) {
-        const int b = sw.color_ptr[c], e = sw.color_ptr[c + 1];
-        hipLaunchKernelGGL(k_gs_color, dim3(grid_for(e - b)), dim3(kBlock), 0, s, e - b,
-                           sw.color_cells.p + b, n, w, nb, ac, anb, bc, dphi, flags);
-      }
+      for (int c = nc - 2; c >= 0; --c) color(c);
       first = false;
       hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, flags);
       fin(m, FIN_CONV, gr, nf);
