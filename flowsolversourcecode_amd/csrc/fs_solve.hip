@@ -302,7 +302,7 @@ __global__ void k_pbcg_p(int n, const double *__restrict__ r, const double *__re
 }
 
 // z = A*p, zz = A^T*pp, akden partials = sum z*pp (PBCGMethod.for:195-205).
-__global__ void k_pbcg_ap(int n, int w, int wt, const int *__restrict__ nbr,
+__global__ void k_pbcg_ap(int n, int w, int wt, EllNbr nbr,
                           const int *__restrict__ tlin, const int *__restrict__ tsrc,
                           const double *__restrict__ ac, const double *__restrict__ anb,
                           const double *__restrict__ p, const double *__restrict__ pp,
@@ -320,18 +320,28 @@ __global__ void k_pbcg_ap(int n, int w, int wt, const int *__restrict__ nbr,
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// dphi += ak*p, r -= ak*z, rr -= ak*zz (PBCGMethod.for:207-213).
+// dphi += ak*p, r -= ak*z, rr -= ak*zz (PBCGMethod.for:207-213), and with dc
+// the next iteration's bknum partials (those of k_pbcg_bknum): its launch and
+// its finaliser's, two of eight in an iteration, go (101050 hexahedra, 40 iterations: 1.55 -> 1.40
+// ms a solve).
 __global__ void k_pbcg_axpy(int n, double *__restrict__ dphi, double *__restrict__ r,
                             double *__restrict__ rr, const double *__restrict__ p,
                             const double *__restrict__ z, const double *__restrict__ zz,
+                            const double *__restrict__ dc, double *__restrict__ part,
                             const double *__restrict__ scal, const int *__restrict__ flags) {
   if (flags[F_DONE]) return;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
   const double ak = scal[S_AK];
-  dphi[i] = dphi[i] + ak * p[i];
-  r[i] = r[i] - ak * z[i];
-  rr[i] = rr[i] - ak * zz[i];
+  double s = 0.0;
+  for (int i = xcd_block() * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    dphi[i] = dphi[i] + ak * p[i];
+    const double ri = r[i] - ak * z[i], rri = rr[i] - ak * zz[i];
+    r[i] = ri;
+    rr[i] = rri;
+    if (dc) s += ri * dc[i] * rri;
+  }
+  if (!dc) return;
+  s = block_sum<kBlock>(s);
+  if (threadIdx.x == 0) part[gridDim.x + blockIdx.x] = s; // beside the residual's partials
 }
 
 // ---- level schedules of the natural-order triangular recurrences (the
@@ -877,6 +887,7 @@ enum FinOp {
   FIN_CG_ALPHA,       // alpha = rz/(p,q)
   FIN_WARM,           // reject an initial guess whose L1 residual exceeds ires
   FIN_WARM_SCALE,     // gamma = (A x0, b)/(A x0, A x0)
+  FIN_CONV_PBCG_BK,   // FIN_CONV, then (unless done) FIN_PBCG_BK of the next iteration
   FIN_CONV_BICG_RHO,  // FIN_CONV, then (unless done) FIN_BICG_RHO of the next iteration
   FIN_POST            // post the scalars and the final word
 };
@@ -972,7 +983,8 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
                       double *__restrict__ scal, int *__restrict__ flags, SolveStart st, Post to) {
   const bool always = op == FIN_INIT_NORMS || op == FIN_TRUE_RES || op == FIN_POST;
   const FinState in(scal, flags);
-  const bool two = op == FIN_BICG_OMEGA || op == FIN_WARM_SCALE || op == FIN_CONV_BICG_RHO;
+  const bool two = op == FIN_BICG_OMEGA || op == FIN_WARM_SCALE || op == FIN_CONV_BICG_RHO ||
+                   op == FIN_CONV_PBCG_BK;
   Partials first, second;
   if (op != FIN_POST) {
     first.load(part, np, threadIdx.x);
@@ -1029,6 +1041,20 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
     flags[F_ITER] = it;
     // NaN residuals end the loop as well
     flags[F_DONE] = !(a > in.rrf * in.ires && it < in.itmax);
+    break;
+  }
+  case FIN_CONV_PBCG_BK: {
+    counted = true;
+    scal[S_FRES] = a;
+    const int it = in.iter + 1;
+    flags[F_ITER] = it;
+    const bool more = a > in.rrf * in.ires && it < in.itmax;
+    flags[F_DONE] = !more;
+    if (more) {
+      scal[S_BKNUM] = b;
+      scal[S_BK] = b / (in.bkden + 1.0e-10);
+      scal[S_BKDEN] = b;
+    }
     break;
   }
   case FIN_BICG_RHO:
@@ -2051,20 +2077,24 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     const double alpha = m->mg_alpha > 0.0 ? m->mg_alpha : 1.7;
     if (pre) amg_prepare(m, ac, anb, alpha);
     const double *dc = pre ? nullptr : m->wk.dc;
+    const auto bknum = [&]() {
+      hipLaunchKernelGGL(k_pbcg_bknum, dim3(gr), dim3(kBlock), 0, s, n, V0, V1, dc, V6, part, flags);
+      fin(m, FIN_PBCG_BK, gr, nf);
+    };
+    if (!pre) bknum(); // every later one comes with the update
     run_iterations(m, itmax, [&]() {
       if (pre) {
         amg_apply(m, V0, V6, flags, alpha);
         amg_apply(m, V1, V7, flags, alpha);
+        bknum();
       }
-      hipLaunchKernelGGL(k_pbcg_bknum, dim3(gr), dim3(kBlock), 0, s, n, V0, V1, dc, V6, part, flags);
-      fin(m, FIN_PBCG_BK, gr, nf);
       hipLaunchKernelGGL(k_pbcg_p, dim3(ge), dim3(kBlock), 0, s, n, V0, V1, dc, V6, V7, V2, V3, scal, flags);
-      hipLaunchKernelGGL(k_pbcg_ap, dim3(gr), dim3(kBlock), 0, s, n, w, sw.wt, nbr, sw.tlin.p,
+      hipLaunchKernelGGL(k_pbcg_ap, dim3(gr), dim3(kBlock), 0, s, n, w, sw.wt, nb, sw.tlin.p,
                          sw.tsrc.p, ac, anb, V2, V3, V4, V5, part, flags);
       fin(m, FIN_PBCG_AK, gr, nf);
-      hipLaunchKernelGGL(k_pbcg_axpy, dim3(ge), dim3(kBlock), 0, s, n, dphi, V0, V1, V2, V4, V5, scal, flags);
+      hipLaunchKernelGGL(k_pbcg_axpy, dim3(gr), dim3(kBlock), 0, s, n, dphi, V0, V1, V2, V4, V5, dc, part, scal, flags);
       hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, flags);
-      fin(m, FIN_CONV, gr, nf);
+      fin(m, pre ? FIN_CONV : FIN_CONV_PBCG_BK, gr, nf);
     });
   } else if (one) {
     gs_one(m, sw.color_ptr, sw.color_cells.p, ac, anb, bc, dphi, fit);
