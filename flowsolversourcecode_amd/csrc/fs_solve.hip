@@ -109,17 +109,37 @@ __device__ __forceinline__ double ell_res(int i, int n, int w, EllNbr nbr,
 // then the contributions of source rows in increasing row order.  tlin/tsrc
 // list, per target cell, the linear anb index and source row of each
 // transposed entry, pre-sorted by (row, slot).
-__device__ __forceinline__ double ell_atx(int i, int n, int wt, const int *__restrict__ tlin,
-                                          const int *__restrict__ tsrc,
-                                          const double *__restrict__ ac,
-                                          const double *__restrict__ anb,
-                                          const double *__restrict__ x) {
-  double s = ac[i] * x[i];
-  for (int j = 0; j < wt; ++j) {
-    const int l = tlin[(size_t)j * n + i];
-    if (l >= 0) s = s + anb[l] * x[tsrc[(size_t)j * n + i]];
+// The sources go in batches like the slots of ell_fold: indices, then values
+// and gathers, then the terms in order (one at a time, 40 products of 101050
+// rows took 60 us more).
+template <int B>
+__device__ __forceinline__ double ell_atx_by(int i, int n, int wt, const int *__restrict__ tlin,
+                                             const int *__restrict__ tsrc, const double *__restrict__ anb,
+                                             const double *__restrict__ x, double s) {
+  for (int j0 = 0; j0 < wt; j0 += B) {
+    int l[B], k[B];
+    double a[B], xv[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const size_t q = (size_t)min(j0 + u, wt - 1) * n + i;
+      l[u] = tlin[q], k[u] = tsrc[q];
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      a[u] = anb[max(l[u], 0)];
+      xv[u] = x[l[u] >= 0 ? k[u] : i];
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (j0 + u < wt && l[u] >= 0) s = s + a[u] * xv[u];
   }
   return s;
+}
+__device__ __forceinline__ double ell_atx(int i, int n, int wt, const int *__restrict__ tlin,
+                                          const int *__restrict__ tsrc, const double *__restrict__ ac,
+                                          const double *__restrict__ anb, const double *__restrict__ x) {
+  const double s = ac[i] * x[i];
+  return wt <= 4 ? ell_atx_by<4>(i, n, wt, tlin, tsrc, anb, x, s) : ell_atx_by<6>(i, n, wt, tlin, tsrc, anb, x, s);
 }
 
 // ---------------------------------------------------------------- kernels
