@@ -19,7 +19,7 @@
 // Convergence never waits for the host: a one-block kernel updates the device
 // flags (done, iteration count), and every iteration kernel returns
 // immediately once done is set.  The same kernel posts the iteration count
-// and done to pinned host memory, and the host launches iterations only one
+// and done to pinned host memory, and the host launches iterations at most two
 // ahead of the last one posted.
 #include <hip/hip_runtime.h>
 
@@ -60,13 +60,15 @@ constexpr unsigned long long kBoxDone = 1, kBoxFinal = 2;
 __device__ __forceinline__ void post_word(SolveBox *box, unsigned seq, const int *flags, unsigned long long final_bit) {
   const unsigned long long w = ((unsigned long long)seq << 32) | ((unsigned long long)(flags[F_ITER] & 0xfffffff) << 4) |
                                ((unsigned long long)flags[F_BAD] << 2) | final_bit | (flags[F_DONE] ? kBoxDone : 0);
-  __hip_atomic_store(&box->word, w, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  // the final post publishes the scalars beside it; the others are the word alone
+  if (final_bit) __hip_atomic_store(&box->word, w, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  else __hip_atomic_store(&box->word, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // F_INNER: the GMRES cycle in progress has finished its Arnoldi steps;
 // F_GATE = F_DONE | F_INNER, the flag the cycle's kernels (and the V-cycle
 // they call) test
 
-constexpr int kFinBlock = 1024; // threads of the one-workgroup finalise kernels
+constexpr int kFinBlock = 1024; // threads of the one-workgroup finalise kernels (256 where fin() says so)
 
 static inline int grid_for(int n) { return xcd_grid(n); }
 // one row per thread up to kPartials workgroups (the row loops of the reducing
@@ -722,7 +724,7 @@ __global__ void k_gm_dots(int n, const double *__restrict__ V, size_t ldv, const
   if (threadIdx.x == 0) part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = s;
 }
 
-__device__ double reduce_partials(const double *part, int np);
+template <int BS = kFinBlock> __device__ double reduce_partials(const double *part, int np);
 
 // hpass[j] = (V_j, w) from the partials; H[j][col] += hpass[j]; blockIdx.x = j
 __global__ void k_gm_hfin(int np, int m, int col, const double *__restrict__ part, double *__restrict__ gm,
@@ -923,51 +925,51 @@ struct Post {
   unsigned seq;
 };
 
-// One workgroup of kFinBlock threads combines the np partials of a sum: a
-// thread's partials i, i + kFinBlock, ... are loaded kFinR at a time, then
+// One workgroup of BS threads combines the np partials of a sum: a thread's
+// partials i, i + BS, ... are loaded kFinR at a time, then
 // folded in index order (the slots past np add +0.0, or take the max with the
 // starting -1.0, which changes nothing).
 constexpr int kFinR = 8;
-struct Partials {
+template <int BS> struct Partials {
   double v[kFinR];
   __device__ __forceinline__ void load(const double *part, int np, int base) {
 #pragma unroll
     for (int u = 0; u < kFinR; ++u) {
-      const int i = base + u * kFinBlock;
+      const int i = base + u * BS;
       v[u] = i < np ? part[i] : 0.0;
     }
   }
-  // the sum, the first kFinR kFinBlock partials being loaded
+  // the sum, the first kFinR BS partials being loaded
   __device__ __forceinline__ double sum(const double *part, int np) {
     double s = 0.0;
     for (int base = threadIdx.x;;) {
 #pragma unroll
       for (int u = 0; u < kFinR; ++u) s += v[u];
-      base += kFinR * kFinBlock;
+      base += kFinR * BS;
       if (base >= np) break;
       load(part, np, base);
     }
-    return block_sum<kFinBlock>(s);
+    return block_sum<BS>(s);
   }
 };
-__device__ double reduce_partials(const double *part, int np) {
-  Partials p;
+template <int BS> __device__ double reduce_partials(const double *part, int np) {
+  Partials<BS> p;
   p.load(part, np, threadIdx.x);
   return p.sum(part, np);
 }
-__device__ double reduce_partials_max(const double *part, int np) {
+template <int BS> __device__ double reduce_partials_max(const double *part, int np) {
   double s = -1.0;
-  for (int base = threadIdx.x; base < np; base += kFinR * kFinBlock) {
+  for (int base = threadIdx.x; base < np; base += kFinR * BS) {
     double v[kFinR];
 #pragma unroll
     for (int u = 0; u < kFinR; ++u) {
-      const int i = base + u * kFinBlock;
+      const int i = base + u * BS;
       v[u] = i < np ? part[i] : -1.0;
     }
 #pragma unroll
     for (int u = 0; u < kFinR; ++u) s = fmax(s, v[u]);
   }
-  return block_max<kFinBlock>(s);
+  return block_max<BS>(s);
 }
 
 // What a solve's scalars held before this kernel
@@ -999,13 +1001,14 @@ __device__ void bicg_rho(double a, int iter, const FinState &in, double *__restr
 // One workgroup, so it lasts as long as its chain of loads: the solve's
 // scalars and the partials are loaded together, and the done flag is tested
 // after both.
-__global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ part,
+template <int BS>
+__global__ void __launch_bounds__(BS) k_fin(int op, int np, int n, int nf, const double *__restrict__ part,
                       double *__restrict__ scal, int *__restrict__ flags, SolveStart st, Post to) {
   const bool always = op == FIN_INIT_NORMS || op == FIN_TRUE_RES || op == FIN_POST;
   const FinState in(scal, flags);
   const bool two = op == FIN_BICG_OMEGA || op == FIN_WARM_SCALE || op == FIN_CONV_BICG_RHO ||
                    op == FIN_CONV_PBCG_BK;
-  Partials first, second;
+  Partials<BS> first, second;
   if (op != FIN_POST) {
     first.load(part, np, threadIdx.x);
     if (two) second.load(part + np, np, threadIdx.x);
@@ -1015,10 +1018,10 @@ __global__ void k_fin(int op, int np, int n, int nf, const double *__restrict__ 
   const double a = op == FIN_POST ? 0.0 : first.sum(part, np);
   double b = 0.0, c = 0.0, d = 0.0, e = 0.0;
   if (op == FIN_INIT_NORMS) {
-    b = reduce_partials_max(part + np, np);
-    c = reduce_partials(part + 2 * np, np);
-    d = reduce_partials_max(part + 3 * np, np);
-    e = reduce_partials_max(part + 4 * np, np);
+    b = reduce_partials_max<BS>(part + np, np);
+    c = reduce_partials<BS>(part + 2 * np, np);
+    d = reduce_partials_max<BS>(part + 3 * np, np);
+    e = reduce_partials_max<BS>(part + 4 * np, np);
   } else if (two) {
     b = second.sum(part + np, np);
   }
@@ -1811,8 +1814,11 @@ static void ilu_apply(fs_mesh *m, double *dphi, const int *flags) {
 }
 
 static void fin(fs_mesh *m, FinOp op, int np, int nf, SolveStart st = SolveStart{}) {
-  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, m->stream, (int)op, np, m->n, nf, m->wk.partial, m->wk.scal,
-                     m->wk.flags, st, Post{m->box, m->seq});
+  // few partials: a workgroup of 256 starts and reduces sooner (396 partials, with
+  // the plain posts: 4.1 us a launch in workgroups of 1024, 2.7 in 256)
+  const bool few = np <= 256 * kFinR;
+  hipLaunchKernelGGL(few ? k_fin<256> : k_fin<kFinBlock>, dim3(1), dim3(few ? 256 : kFinBlock), 0, m->stream, (int)op, np,
+                     m->n, nf, m->wk.partial, m->wk.scal, m->wk.flags, st, Post{m->box, m->seq});
 }
 
 static void host_flags(fs_mesh *m, int *fl) {
