@@ -1656,7 +1656,8 @@ static void launch_sweep(fs_mesh *m, DLevel &D, int level, const T *b, const T *
     launch_sweep_fine<T, T>(m, D, b, x, om, xn, flags);
   else if (D.sell)
     hipLaunchKernelGGL((D.sell16 ? k_sweep_sell<T, true> : k_sweep_sell<T, false>), dim3(gfor(D.sell_slots)),
-                       dim3(kBlock), 0, m->stream, D.sell_slots, D.sell_ptr.p, D.sell_row.p, D.sell_col.p, LV<T>::val(D), LV<T>::ac(D), b, x, om, xn, flags);
+                       dim3(kBlock), 0, m->stream, D.sell_slots, D.sell_ptr.p, D.sell_row.p, D.sell_col.p,
+                       LV<T>::val(D), LV<T>::ac(D), b, x, om, xn, flags);
   else
     launch_sweep_csr<T, false>(m, D, b, x, om, xn, Scatter<T>{}, flags);
 }
@@ -1667,7 +1668,8 @@ static void launch_resid(fs_mesh *m, DLevel &D, const T *b, const T *x, T *r, co
   const T *ac = LV<T>::ac(D), *anb = LV<T>::anb(D);
   if (D.sell) {
     hipLaunchKernelGGL((D.sell16 ? k_resid_sell<T, true> : k_resid_sell<T, false>), dim3(gfor(D.sell_slots)),
-                       dim3(kBlock), 0, s, D.sell_slots, D.sell_ptr.p, D.sell_row.p, D.sell_col.p, LV<T>::val(D), ac, b, x, r, flags);
+                       dim3(kBlock), 0, s, D.sell_slots, D.sell_ptr.p, D.sell_row.p, D.sell_col.p, LV<T>::val(D), ac,
+                       b, x, r, flags);
     return;
   }
   const EllNbr nb(D.nbr, D.nbr16);
