@@ -74,11 +74,14 @@ static inline int grid_for(int n) { return xcd_grid(n); }
 // one row per thread up to kPartials workgroups (the row loops of the reducing
 // kernels stride by the grid beyond)
 static inline int grid_red(int n) { return std::min(kPartials, xcd_grid(n)); }
-// kernels that only sum take kSumRows rows per thread, their loads first: the
-// reduction of a workgroup costs as much as its loads otherwise (2.9 M rows, one
-// row against four: k_dot 15.4 and 9.0 us, k_init_norms 36 and 17)
-constexpr int kSumRows = 4;
-static inline int grid_sum(int n) { return grid_red((n + kSumRows - 1) / kSumRows); }
+// Kernels that only sum take four rows per thread, their loads first, from a
+// million rows on: the reduction of a workgroup costs as much as its loads
+// otherwise (2.9 M rows, one row against four: k_dot 15.4 and 9.0 us,
+// k_init_norms 36 and 17).  Below, a launch is latency and the sums keep the
+// grouping of one row per thread.
+constexpr int kSumRows = 4, kSumRowsFrom = 1000000;
+static inline int sum_rows(int n) { return n >= kSumRowsFrom ? kSumRows : 1; }
+static inline int grid_sum(int n) { return grid_red((n + sum_rows(n) - 1) / sum_rows(n)); }
 
 // The Krylov products stream the FP64 matrix (read twice per iteration, too
 // large to stay cached beside the vectors): non-temporal matrix loads.
@@ -150,18 +153,19 @@ __device__ __forceinline__ double ell_atx(int i, int n, int wt, const int *__res
 // 19-67) with dphi = 0: r_i = bc_i.  Partials: sum|r|, max|r|, sum r^2,
 // max|ac*fit|, and the input check: the largest of 0 (row fine), 1 (ac <= 0)
 // and 2 (ac or bc not finite).
+template <int ROWS>
 __global__ void k_init_norms(int n, const double *__restrict__ ac, const double *__restrict__ bc,
                              const double *__restrict__ fit, double *__restrict__ part) {
   double s1 = 0.0, m1 = -1.0, s2 = 0.0, m2 = -1.0, bad = 0.0;
-  for (int i0 = xcd_block() * kBlock * kSumRows + threadIdx.x; i0 < n; i0 += gridDim.x * kBlock * kSumRows) {
-    double a[kSumRows], b[kSumRows], f[kSumRows];
+  for (int i0 = xcd_block() * kBlock * ROWS + threadIdx.x; i0 < n; i0 += gridDim.x * kBlock * ROWS) {
+    double a[ROWS], b[ROWS], f[ROWS];
 #pragma unroll
-    for (int u = 0; u < kSumRows; ++u) {
+    for (int u = 0; u < ROWS; ++u) {
       const int i = min(i0 + u * kBlock, n - 1);
       a[u] = ac[i], b[u] = bc[i], f[u] = fit[i];
     }
 #pragma unroll
-    for (int u = 0; u < kSumRows; ++u) {
+    for (int u = 0; u < ROWS; ++u) {
       if (i0 + u * kBlock >= n) break;
       const double r = fabs(b[u]);
       s1 += r;
@@ -568,19 +572,20 @@ __global__ void k_gs_rows_color(int t0, int cnt, const int *__restrict__ cells, 
 // ---- generic vector kernels for the Krylov solvers
 
 // partial sums of a*b
+template <int ROWS>
 __global__ void k_dot(int n, const double *__restrict__ a, const double *__restrict__ b, double *__restrict__ part,
                       const int *__restrict__ flags) {
   if (flags && flags[F_DONE]) return;
   double s = 0.0;
-  for (int i0 = xcd_block() * kBlock * kSumRows + threadIdx.x; i0 < n; i0 += gridDim.x * kBlock * kSumRows) {
-    double av[kSumRows], bv[kSumRows];
+  for (int i0 = xcd_block() * kBlock * ROWS + threadIdx.x; i0 < n; i0 += gridDim.x * kBlock * ROWS) {
+    double av[ROWS], bv[ROWS];
 #pragma unroll
-    for (int u = 0; u < kSumRows; ++u) {
+    for (int u = 0; u < ROWS; ++u) {
       const int i = min(i0 + u * kBlock, n - 1);
       av[u] = a[i], bv[u] = b[i];
     }
 #pragma unroll
-    for (int u = 0; u < kSumRows; ++u)
+    for (int u = 0; u < ROWS; ++u)
       if (i0 + u * kBlock < n) s += av[u] * bv[u];
   }
   s = block_sum<kBlock>(s);
@@ -2058,7 +2063,7 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   SolveStart start{rrf, lmg == FS_MG_SOLVER ? m->mg_maxcycles : itmax, itmax, 0};
   start.needpos = (lmg != FS_MG_OFF || solver == FS_SOR || solver == FS_ILU || solver == FS_PBCG) ? 1 : 0;
   ++m->seq;
-  hipLaunchKernelGGL(k_init_norms, dim3(gs), dim3(kBlock), 0, s, n, ac, bc, fit, part);
+  hipLaunchKernelGGL(sum_rows(n) == 1 ? k_init_norms<1> : k_init_norms<kSumRows>, dim3(gs), dim3(kBlock), 0, s, n, ac, bc, fit, part);
   fin(m, FIN_INIT_NORMS, gs, nf, start);
   const bool one = solver == FS_SOR && !warm && lmg != FS_MG_SOLVER && gs_in_one(n, w, (int)sw.color_ptr.size() - 1);
   if (!warm && !one) hipLaunchKernelGGL(k_zero_start, dim3(ge), dim3(kBlock), 0, s, n, dphi, (const int *)flags);
@@ -2166,7 +2171,7 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     hipLaunchKernelGGL(k_resid_vec, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, V0, V1, part);
     hipLaunchKernelGGL(k_zero, dim3(ge), dim3(kBlock), 0, s, n, V3);
     // rho of the first iteration; every later rho comes with the update
-    hipLaunchKernelGGL(k_dot, dim3(gs), dim3(kBlock), 0, s, n, V1, V0, part, flags);
+    hipLaunchKernelGGL(sum_rows(n) == 1 ? k_dot<1> : k_dot<kSumRows>, dim3(gs), dim3(kBlock), 0, s, n, V1, V0, part, flags);
     fin(m, FIN_BICG_RHO, gs, nf);
     run_iterations(m, itmax, [&]() {
       hipLaunchKernelGGL(k_bicg_p, dim3(ge), dim3(kBlock), 0, s, n, V0, V3, V2, scal, flags);
@@ -2200,7 +2205,7 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
         amg_apply(m, V0, V1, flags, alpha);
         z = V1;
       }
-      hipLaunchKernelGGL(k_dot, dim3(gs), dim3(kBlock), 0, s, n, V0, z, part, flags);
+      hipLaunchKernelGGL(sum_rows(n) == 1 ? k_dot<1> : k_dot<kSumRows>, dim3(gs), dim3(kBlock), 0, s, n, V0, z, part, flags);
       fin(m, FIN_CG_RHO, gs, nf);
       hipLaunchKernelGGL(k_cg_p, dim3(ge), dim3(kBlock), 0, s, n, z, V2, scal, flags);
       timed_launch(m, FS_CLOCK_SPMV, spmv_bytes, k_spmv_dot, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, V2,
