@@ -99,26 +99,19 @@ __global__ void k_stats(int N, const int *__restrict__ ids, const T *__restrict_
   }
 }
 
-// sum over the 64 lanes of a wavefront in a fixed order, valid in lane 0
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  return v;
-}
-
-// scal[s] = {s_b, s_a, mean vol, mean x, mean xp}; one wavefront per sample,
-// nb <= 64 partials, one a lane
-__global__ void k_stats_fin(int N, int nb, const double *__restrict__ part, double *__restrict__ scal) {
-  static_assert(kStatBlocks <= 64, "one partial a lane");
-  const int s = blockIdx.x, k = threadIdx.x;
-  double a[kStats];
-#pragma unroll
-  for (int q = 0; q < kStats; ++q) a[q] = k < nb ? part[((size_t)s * nb + k) * kStats + q] : 0.0;
-#pragma unroll
-  for (int q = 0; q < kStats; ++q) a[q] = wave_sum(a[q]);
-  if (k != 0) return;
-  scal[s * kStats + 0] = sqrt(a[0] / N) + 1e-300;
-  for (int q = 1; q < kStats; ++q) scal[s * kStats + q] = a[q] / N;
+// scal[s] = {s_b, s_a, mean vol, mean x, mean xp}; one wavefront per sample:
+// the partials are loaded together and each quantity is summed in block order
+// by a thread of its own
+__global__ void __launch_bounds__(64)
+k_stats_fin(int N, int nb, const double *__restrict__ part, double *__restrict__ scal) {
+  __shared__ double v[kStatBlocks * kStats];
+  const int s = blockIdx.x, q = threadIdx.x;
+  for (int k = threadIdx.x; k < nb * kStats; k += 64) v[k] = part[(size_t)s * nb * kStats + k];
+  __syncthreads();
+  if (q >= kStats) return;
+  double a = 0.0;
+  for (int k = 0; k < nb; ++k) a += v[k * kStats + q];
+  scal[s * kStats + q] = q == 0 ? sqrt(a / N) + 1e-300 : a / N;
 }
 
 // X0, edge weights E[j][c] and the normalised target of the batch cells
@@ -276,11 +269,18 @@ __global__ void k_decode(int N, int Bn, const unsigned short *__restrict__ H, co
   (void)Bn;
 }
 
-// ymean[s] from the partials, one a lane
-__global__ void k_mean_fin(int N, int nb, const double *__restrict__ part, double *__restrict__ ymean) {
-  const int s = blockIdx.x, k = threadIdx.x;
-  const double a = wave_sum(k < nb ? part[(size_t)s * nb + k] : 0.0);
-  if (k == 0) ymean[s] = a / N;
+// ymean[s] from the partials, loaded together and summed in block order
+__global__ void __launch_bounds__(64)
+k_mean_fin(int N, int nb, const double *__restrict__ part, double *__restrict__ ymean) {
+  static_assert(kStatBlocks <= 64, "one partial a lane");
+  __shared__ double v[64];
+  const int s = blockIdx.x;
+  v[threadIdx.x] = (int)threadIdx.x < nb ? part[(size_t)s * nb + threadIdx.x] : 0.0;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double a = 0.0;
+  for (int k = 0; k < nb; ++k) a += v[k];
+  ymean[s] = a / N;
 }
 
 // yc = y - mean; loss partials and dy = 2 (yc - t)/total (training), or the
@@ -502,13 +502,9 @@ k_dense_bwd_w(int Bn, int chunk, const unsigned short *__restrict__ H, const uns
         for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv[nt], acc[mt][nt], 0, 0, 0);
       }
     }
-    // column sums: lane o, a quarter of the stage's cells per wave
+    // column sums: lane o, every fourth cell per wave
 #pragma unroll
-    for (int k = 0; k < kStage / 32; ++k) {
-      const u16x8 z = *reinterpret_cast<const u16x8 *>(zs + lane * kStageStride + wave * (kStage / 4) + k * 8);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) bs += bf2f(z[q]);
-    }
+    for (int k = 0; k < kStage / 4; ++k) bs += bf2f(zs[lane * kStageStride + 4 * k + wave]);
   }
   bred[wave][lane] = bs;
   __syncthreads();
@@ -570,30 +566,40 @@ __global__ void k_enc_bwd(int Bn, int chunk, const float *__restrict__ X0, const
       out[((size_t)blockIdx.x * (kF + 1) + f) * kH + o] = red[0][f][o] + red[1][f][o] + red[2][f][o] + red[3][f][o];
 }
 
-// dst[k] = sum over the nb blocks' partials part[b][k], k < K.  A block sums 32
-// columns with 8 row groups (rows g, g + 8, ... in order, 8 loads in flight),
-// the groups combined in order: 4-8 us for 256 x 8256 values (one thread a
-// column over all rows: 60 us, and as much for each bias).
-__global__ void k_reduce(int nb, int K, const float *__restrict__ part, float *__restrict__ dst) {
-  constexpr int C = 32, G = kBlock / C, B = 8;
+// dst[k] = sum over the nb blocks' partials part[b][k] in block order, k < K.  A
+// block sums 32 columns: its threads load kReduceRows rows of them together
+// into LDS, where one thread a column adds them up one after the other.
+constexpr int kReduceRows = 256;
+__global__ void __launch_bounds__(kBlock)
+k_reduce(int nb, int K, const float *__restrict__ part, float *__restrict__ dst) {
+  constexpr int C = 32, G = kBlock / C;
+  __shared__ float v[kReduceRows][C];
   const int kk = threadIdx.x % C, g = threadIdx.x / C, k = blockIdx.x * C + kk;
   float s = 0.f;
-  for (int b0 = g; b0 < nb; b0 += G * B) {
-    float v[B];
+  for (int b0 = 0; b0 < nb; b0 += kReduceRows) {
+    const int rows = min(kReduceRows, nb - b0);
+    if (k < K) {
+      float r[kReduceRows / G];
 #pragma unroll
-    for (int u = 0; u < B; ++u) v[u] = k < K && b0 + u * G < nb ? part[(size_t)(b0 + u * G) * K + k] : 0.f;
+      for (int u = 0; u < kReduceRows / G; ++u) r[u] = part[(size_t)(b0 + min(g + u * G, rows - 1)) * K + k];
 #pragma unroll
-    for (int u = 0; u < B; ++u) s += v[u];
+      for (int u = 0; u < kReduceRows / G; ++u) v[g + u * G][kk] = r[u];
+    }
+    __syncthreads();
+    if (g == 0 && k < K) {
+      int b = 0;
+      for (; b + 16 <= rows; b += 16) {
+        float t[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) t[u] = v[b + u][kk];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s += t[u];
+      }
+      for (; b < rows; ++b) s += v[b][kk];
+    }
+    __syncthreads();
   }
-  __shared__ float red[G][C];
-  red[g][kk] = s;
-  __syncthreads();
-  if (g == 0 && k < K) {
-    float t = 0.f;
-#pragma unroll
-    for (int u = 0; u < G; ++u) t += red[u][kk];
-    dst[k] = t;
-  }
+  if (g == 0 && k < K) dst[k] = s;
 }
 
 __global__ void k_adam(int n, float *__restrict__ th, const float *__restrict__ g, float *__restrict__ m,
