@@ -37,7 +37,7 @@ constexpr int kTile = 16;      // cells of a matrix-core tile
 constexpr int kTiles = 2;      // tiles a wavefront of the dense kernels works through
 constexpr int kRowsFwd = 4 * kTiles * kTile; // cells per block of the dense kernels
 constexpr int kStage = 64;     // cells the weight-gradient kernel stages at a time
-constexpr int kGradBlocks = 512; // most blocks (partial gradients) of the gradient kernels
+constexpr int kChunk = 256;    // cells per block (and partial gradient) of the gradient kernels
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
@@ -46,10 +46,11 @@ typedef unsigned char u8x4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 inline int cdiv(long long a, int b) { return (int)((a + b - 1) / b); }
-// cells per block of the gradient kernels: 256 fill the chip at 65536 cells;
-// above kGradBlocks blocks the partial gradients (33 KB each) would outgrow
-// the activations, so the blocks take more cells instead
-inline int grad_chunk(long long Bn) { return std::max(256, cdiv(cdiv(Bn, kGradBlocks), kStage) * kStage); }
+// blocks of the gradient kernels for a batch of Bn cells.  Their workspace is
+// sized for the largest batch so far, so this must not fall as Bn grows: the
+// chunk is the same for every batch (blocks of more cells above 131072 cells
+// saved 1-2 % of a step: 557 and 571 us at 135168, 3.52 and 3.56 ms at 1048576).
+inline int grad_blocks(long long Bn) { return cdiv(Bn, kChunk); }
 
 // float -> bfloat16 bits, round to nearest even (NaN kept quiet)
 __device__ __forceinline__ unsigned short f2bf(float f) {
@@ -339,10 +340,10 @@ __global__ void k_dec_bwd(int Bn, const float *__restrict__ DY, const float *__r
 // Decoder gradient: per-block sums out[blk][o] = sum of dy[c] H[c][o] over the
 // block's cells, out[blk][64] = sum of dy[c].  Block: 256 threads = 4 cell
 // lanes x 64 columns, the loads of 8 cells in flight.
-__global__ void k_dec_grad(int Bn, int chunk, const float *__restrict__ DY, const unsigned short *__restrict__ H,
+__global__ void k_dec_grad(int Bn, const float *__restrict__ DY, const unsigned short *__restrict__ H,
                            float *__restrict__ out) {
   const int o = threadIdx.x & 63, r = threadIdx.x >> 6;
-  const int c0 = blockIdx.x * chunk, c1 = min(Bn, c0 + chunk);
+  const int c0 = blockIdx.x * kChunk, c1 = min(Bn, c0 + kChunk);
   float s = 0.f, sa = 0.f;
   constexpr int B = 8;
   for (int cb = c0 + r; cb < c1; cb += 4 * B) {
@@ -437,18 +438,18 @@ __global__ void k_agg_t(int N, int W, int Bn, const int *__restrict__ nbr0, cons
 // a time in LDS, each thread transposing one 8 cells x 8 features tile in
 // registers (16-byte loads and LDS stores; the next stage's loads are in
 // flight behind the products).  Wave w owns input features 32w..32w+31 (2 x 4
-// output tiles).  65536 cells: 9.4 us (2-byte staging of 32 cells: 53.6 us,
+// output tiles).  65536 cells: 9.5 us (2-byte staging of 32 cells: 53.6 us,
 // and another 20 us for the column sums).
 constexpr int kStageStride = kStage + 8; // bf16 elements per staged row: 16-byte rows, spread over the banks
 constexpr int kGradW = kIn * kH + kH;    // values of a layer's gradient (W, b)
 
 __global__ void __launch_bounds__(256)
-k_dense_bwd_w(int Bn, int chunk, const unsigned short *__restrict__ H, const unsigned short *__restrict__ M,
+k_dense_bwd_w(int Bn, const unsigned short *__restrict__ H, const unsigned short *__restrict__ M,
               const unsigned short *__restrict__ DZ, float *__restrict__ out) {
   __shared__ __attribute__((aligned(16))) unsigned short st[(kIn + kH) * kStageStride];
   __shared__ float bred[4][kH];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, kg = lane >> 4;
-  const int c0 = blockIdx.x * chunk, c1 = min(Bn, c0 + chunk);
+  const int c0 = blockIdx.x * kChunk, c1 = min(Bn, c0 + kChunk);
   // the thread's tile: cells 8 cg.., feature group fg of [H | M | dz]
   const int cg = threadIdx.x & 7, fg = threadIdx.x >> 3;
   const bool loads = fg < (kIn + kH) / 8;
@@ -527,10 +528,10 @@ k_dense_bwd_w(int Bn, int chunk, const unsigned short *__restrict__ H, const uns
 
 // encoder gradient partials: out[blk][f][o] = sum X0[c][f] dz0[c][o] (f < 8),
 // out[blk][8][o] = sum dz0[c][o], dz0 = (H0 > 0) ? dH : 0
-__global__ void k_enc_bwd(int Bn, int chunk, const float *__restrict__ X0, const unsigned short *__restrict__ H0,
+__global__ void k_enc_bwd(int Bn, const float *__restrict__ X0, const unsigned short *__restrict__ H0,
                           const float *__restrict__ dH, float *__restrict__ out) {
   const int o = threadIdx.x & 63, r = threadIdx.x >> 6;
-  const int c0 = blockIdx.x * chunk, c1 = min(Bn, c0 + chunk);
+  const int c0 = blockIdx.x * kChunk, c1 = min(Bn, c0 + kChunk);
   static_assert(kF == 8, "features in two 16-byte loads");
   float s[kF + 1];
 #pragma unroll
@@ -568,7 +569,8 @@ __global__ void k_enc_bwd(int Bn, int chunk, const float *__restrict__ X0, const
 
 // dst[k] = sum over the nb blocks' partials part[b][k] in block order, k < K.  A
 // block sums 32 columns: its threads load kReduceRows rows of them together
-// into LDS, where one thread a column adds them up one after the other.
+// into LDS, where one thread a column adds them up one after the other: 3.6-6.5
+// us for 256 blocks (one thread a column over all rows: 60 us).
 constexpr int kReduceRows = 256;
 __global__ void __launch_bounds__(kBlock)
 k_reduce(int nb, int K, const float *__restrict__ part, float *__restrict__ dst) {
@@ -682,7 +684,7 @@ static void mpnn_grow(fs_mpnn *n, int B) {
   for (auto &h : n->Hs) h.alloc(Bn * kH);
   for (auto &m : n->Ms) m.alloc(Bn * kH);
   for (auto &m : n->masks) m.alloc(Bn * kH);
-  n->gpart.alloc((size_t)cdiv(Bn, grad_chunk(Bn)) * kGradW);
+  n->gpart.alloc((size_t)grad_blocks(Bn) * kGradW);
   n->bn_cap = Bn;
 }
 
@@ -733,20 +735,21 @@ static void mpnn_loss_grad(fs_mpnn *n, const int *ids, int B, bool want_grad) {
   hipLaunchKernelGGL(k_loss, dim3(nb, B), dim3(kBlock), 0, s, N, n->ymean.p, n->scal.p, n->Y.p, n->Tg.p, n->DY.p,
                      1.0 / Bn, n->part.p, (double *)nullptr);
   if (!want_grad) return;
-  const int L = n->L, chunk = grad_chunk(Bn), nbc = cdiv(Bn, chunk);
+  const int L = n->L, nbc = grad_blocks(Bn);
+  if ((size_t)nbc * kGradW > n->gpart.n) throw std::runtime_error("gradient workspace too small for the batch");
   float *g = n->grad.p;
   auto reduce = [&](int K, float *dst) {
     hipLaunchKernelGGL(k_reduce, dim3(cdiv(K, 32)), dim3(kBlock), 0, s, nbc, K, n->gpart.p, dst);
   };
   // decoder (wd and bd are the last parameters)
-  hipLaunchKernelGGL(k_dec_grad, dim3(nbc), dim3(256), 0, s, Bn, chunk, n->DY.p, n->Hs[L].p, n->gpart.p);
+  hipLaunchKernelGGL(k_dec_grad, dim3(nbc), dim3(256), 0, s, Bn, n->DY.p, n->Hs[L].p, n->gpart.p);
   reduce(kH + 1, g + mpnn_offset_W(L));
   const unsigned quads = cdiv((long long)Bn * (kH / 4), kBlock);
   hipLaunchKernelGGL(k_dec_bwd, dim3(quads), dim3(kBlock), 0, s, Bn, n->DY.p, n->wdq.p, n->dH.p, n->masks[L - 1].p,
                      n->DZ.p);
   float *dH = n->dH.p, *dH2 = n->dH2.p;
   for (int l = L - 1; l >= 0; --l) {
-    hipLaunchKernelGGL(k_dense_bwd_w, dim3(nbc), dim3(256), 0, s, Bn, chunk, n->Hs[l].p, n->Ms[l].p, n->DZ.p,
+    hipLaunchKernelGGL(k_dense_bwd_w, dim3(nbc), dim3(256), 0, s, Bn, n->Hs[l].p, n->Ms[l].p, n->DZ.p,
                        n->gpart.p);
     reduce(kGradW, g + mpnn_offset_W(l));
     hipLaunchKernelGGL(k_dense_bwd_x, dim3(cdiv(Bn, kRowsFwd)), dim3(256), 0, s, Bn, n->DZ.p,
@@ -755,7 +758,7 @@ static void mpnn_loss_grad(fs_mpnn *n, const int *ids, int B, bool want_grad) {
                        dH2, l > 0 ? n->masks[l - 1].p : nullptr, n->DZ.p);
     std::swap(dH, dH2);
   }
-  hipLaunchKernelGGL(k_enc_bwd, dim3(nbc), dim3(256), 0, s, Bn, chunk, n->X0.p, n->Hs[0].p, dH, n->gpart.p);
+  hipLaunchKernelGGL(k_enc_bwd, dim3(nbc), dim3(256), 0, s, Bn, n->X0.p, n->Hs[0].p, dH, n->gpart.p);
   reduce((kF + 1) * kH, g);
 }
 

@@ -21,6 +21,7 @@ CASES = {
     "tile": ((5, 7, 3), 1, [1]),           # 105 cells: less than one block of the gradient kernels
     "blocks": ((13, 11, 9), 2, [2, 0, 1]),  # 3861 cells: 16 blocks, the last of 21 cells
     "many": ((64, 64, 1), 1, [0, 1, 2] * 7),  # 86016 cells: 336 blocks
+    "large": ((64, 64, 1), 1, [0, 1, 2] * 11),  # 135168 cells: 528 blocks
 }
 SAMPLES = 3
 

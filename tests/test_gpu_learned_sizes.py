@@ -1,7 +1,7 @@
 """The network's loss and gradient at sizes off the kernels' tiles.
 
 The dense kernels work 16 cells a tile and 128 a block, the weight gradients
-64 cells a stage and 256 a block (more when the batch passes 131072 cells):
+64 cells a stage and 256 a block:
 cell counts below one tile, one past a stage, a block, and a batch of many
 blocks, against the CPU statement of the network.  Tolerances as in
 test_gpu_learned.py: loss 1e-3, each gradient tensor 2e-2 (relative L2).  A
@@ -59,10 +59,22 @@ def test_gradient_off_the_tiles(shape, ids):
         o += k
 
 
-@pytest.mark.parametrize("copies", [2, 51, 105])  # 105 x 1287 cells: blocks of more than 256 cells
+@pytest.mark.parametrize("copies", [2, 51, 105])
 def test_copies_have_the_samples_gradient(copies):
     net, theta = network((13, 11, 9), 1)
     loss, g = net.loss_grad([0])
     lc, gc = net.loss_grad([0] * copies)
     assert abs(loss - lc) <= 1e-6 * loss
     assert np.linalg.norm(g[:-1] - gc[:-1]) <= 1e-3 * np.linalg.norm(g[:-1])
+
+
+@pytest.mark.parametrize("first, then, grad", [(105, 101, True), (110, 102, False), (160, 4, True)])
+def test_smaller_batch_after_a_larger_one(first, then, grad):
+    """A network keeps its largest batch's workspaces: what a smaller batch
+    gives there is, bit for bit, what it gives on a fresh network."""
+    net, theta = network((13, 11, 9), 1)
+    net.loss_grad([0] * first, grad=grad)
+    loss, g = net.loss_grad([0] * then)
+    fresh, _ = network((13, 11, 9), 1)
+    lf, gf = fresh.loss_grad([0] * then)
+    assert loss == lf and np.array_equal(g, gf)
