@@ -1182,7 +1182,11 @@ k_gs_one(int n, int w, GsColors col, const int *__restrict__ cells, const int *_
     }
     return;
   }
-  int cell[R], color[R], k2[R][W / 2]; // neighbours as two 16-bit cells, the cell itself: none
+  // neighbours as two 16-bit cells; filled slots as bits W r + j of `filled`
+  // (a cell may couple to itself: one cell between two periodic patches)
+  static_assert(R * W <= 32 && R * kGsOneThreads <= 65536, "packed slots");
+  int cell[R], color[R], k2[R][W / 2];
+  unsigned filled = 0;
   double a[R][W], d[R], b[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -1204,8 +1208,10 @@ k_gs_one(int n, int w, GsColors col, const int *__restrict__ cells, const int *_
       k[j] = nbr[q], a[r][j] = anb[q];
     }
 #pragma unroll
-    for (int j = 0; j < W; ++j)
-      if (j >= w || k[j] < 0) k[j] = i;
+    for (int j = 0; j < W; ++j) {
+      if (j < w && k[j] >= 0) filled |= 1u << (W * r + j);
+      else k[j] = i;
+    }
 #pragma unroll
     for (int j = 0; j < W; j += 2) k2[r][j / 2] = k[j] | (k[j + 1] << 16);
   }
@@ -1215,10 +1221,8 @@ k_gs_one(int n, int w, GsColors col, const int *__restrict__ cells, const int *_
 #pragma unroll
     for (int j = 0; j < W; ++j) xk[j] = x[j & 1 ? (unsigned)k2[r][j / 2] >> 16 : k2[r][j / 2] & 0xffff];
 #pragma unroll
-    for (int j = 0; j < W; ++j) {
-      const int k = j & 1 ? (unsigned)k2[r][j / 2] >> 16 : k2[r][j / 2] & 0xffff;
-      if (k != cell[r]) v = v - a[r][j] * xk[j];
-    }
+    for (int j = 0; j < W; ++j)
+      if (filled >> (W * r + j) & 1u) v = v - a[r][j] * xk[j];
     return v;
   };
   const auto sweep = [&](int c) {

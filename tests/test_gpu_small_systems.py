@@ -1,6 +1,7 @@
 """Gauss-Seidel solves that run in one workgroup (up to 4096 rows of up to six
 slots) against the same sweeps in numpy, bit for bit, on both sides of every
-size at which the kernel changes; and the ways a solve can end.
+size at which the kernel changes; cells that couple to themselves; and the
+ways a solve can end.
 """
 import numpy as np
 import pytest
@@ -30,6 +31,35 @@ def test_sweeps_are_numpys(n, w):
     assert np.array_equal(f, fit + x)
     # a sum of n terms in another order; rows solved last have only round-off
     r = bc - ac * x - sum(np.where(nbr[j] > 0, anb[j] * x[np.maximum(nbr[j], 1) - 1], 0.0) for j in range(w))
+    np.testing.assert_allclose(st["final_l1"], np.abs(r).sum(), rtol=1e-9, atol=1e-14 * np.abs(bc).sum())
+
+
+@pytest.mark.parametrize("n", [5, 1024, 1025, 4096, 4097])
+@pytest.mark.parametrize("w", [4, 6])
+def test_a_cells_coupling_to_itself(n, w):
+    """A periodic direction one cell thick makes a cell its own neighbour: the
+    term takes the value the cell had before its update, and the residual
+    holds it, however many rows there are."""
+    nbr, nnbr, ac, anb, bc = graph(n, n, w - 1, n + w)
+    rng = np.random.default_rng(n)
+    own = rng.random(n) < 0.5
+    nbr = np.vstack([np.where(own, np.arange(1, n + 1), 0)[None, :].astype(nbr.dtype), nbr])
+    anb = np.vstack([np.where(own, rng.uniform(0.3, 0.6, n), 0.0)[None, :] * ac, anb])
+    nnbr = nnbr + 1
+    color = colors(np.where(nbr == np.arange(1, n + 1), 0, nbr))
+    m = fs.Mesh(nbr, nnbr)
+    fit = np.linspace(-1.0, 1.0, n)
+    rc, f, dphi, res4, st = m.solve_equation("velx", fit, 1e-30, 3, "sor", 0, ac, anb, bc)
+    lists = [np.nonzero(color == c)[0] for c in range(color.max() + 1)]
+    # a colour is not swept twice in a row (at the turn, and at the first colour
+    # between iterations), which only a cell's coupling to itself could show
+    y = np.zeros(n)
+    for it in range(st["iterations"]):
+        for c in list(range(1 if it else 0, len(lists))) + list(range(len(lists) - 2, -1, -1)):
+            sweep(nbr, ac, anb, bc, y, lists[c])
+    assert np.array_equal(dphi, y), np.abs(dphi - y).max()
+    assert np.array_equal(f, fit + y)
+    r = bc - ac * y - sum(np.where(nbr[j] > 0, anb[j] * y[np.maximum(nbr[j], 1) - 1], 0.0) for j in range(w))
     np.testing.assert_allclose(st["final_l1"], np.abs(r).sum(), rtol=1e-9, atol=1e-14 * np.abs(bc).sum())
 
 
