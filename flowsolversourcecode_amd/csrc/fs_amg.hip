@@ -913,18 +913,23 @@ __global__ void k_add2(int n, double *__restrict__ x, const double *__restrict__
 // once per operator as a dense matrix and applied as a matrix-vector product.
 // Column j is the cycle's answer to the j-th unit vector: k_dense_level forms
 // all columns of a level from the level's sparse operator and the dense map of
-// the level below it.  A product is bound by one round of loads (1190 cells in
-// FP32: 5.7 MB, spread over the chip) and takes 5 us
-// (1939 cells 7 us), where one workgroup
-// that walked the levels in LDS took 13-25 us per visit, 8 to 30 visits per
-// Krylov iteration; forming the maps takes 60-150 us per operator.
+// the level below it.  Maps are FP64 for every hierarchy: they hold the inverse
+// of the coarsest operator, which on a nearly singular system is one large
+// constant and, below its FP32 rounding, the part that corrects.  A product is
+// bound by one round of loads (1190 cells: 11 MB, spread over the chip) and takes
+// 5.0 us (828 cells 3.9, 1939 cells 9.0; with FP32 maps 4.7, 4.6, 6.5), where one
+// workgroup that walked the levels in LDS took 13-25 us per visit, 8 to 30 visits
+// per Krylov iteration; forming the maps takes 60-210 us per operator.  2.1 M
+// hexahedra take 531 us a BiCGSTAB iteration (519 with FP32 maps), 2.9 M
+// tetrahedra 549 us a CG iteration (545).
 constexpr int kDirectMax = 64;               // coarsest levels up to this size are solved directly
-constexpr size_t kDenseBytes = 16u << 20;    // largest map: 2048 cells in FP32, 1448 in FP64 (the L2s hold 32 MB)
 constexpr int kDenseThreads = 512;
 constexpr int kDenseRows = 8;                // rows of a product's workgroup
-
-inline int dense_max(size_t tsz) { return tsz == 4 ? 2048 : 1448; }
-static_assert((size_t)2048 * 2048 * 4 <= kDenseBytes && (size_t)1448 * 1448 * 8 <= kDenseBytes, "dense map size");
+// cells of the largest map.  FP64 hierarchies: 16 MB, half of what the L2s hold;
+// FP32 ones up to 34 MB, where the map is even with the level's own launches
+// around the map below (1939 cells under 2.1 M hexahedra: 531 us an iteration
+// and 528).
+inline int dense_max(bool fp32) { return fp32 ? 2048 : 1448; }
 
 // A map is stored in strips of kDenseRows rows, each strip column by column,
 // so that a strip is one contiguous run of memory: entry (i, j) of an n x n map.
@@ -934,30 +939,29 @@ __host__ __device__ __forceinline__ size_t dense_at(int i, int j, int n) {
 // values of a map of n cells (the last strip is padded)
 inline size_t dense_size(int n) { return (size_t)((n + kDenseRows - 1) / kDenseRows) * kDenseRows * n; }
 
-// 16 bytes of T: the columns a workgroup of k_dense_level forms together, the
-// rows a lane of k_dense_apply loads at once
-template <class T> struct Vec16 {
-  static constexpr int K = 16 / sizeof(T);
-  typedef T V __attribute__((ext_vector_type(16 / sizeof(T))));
-};
+typedef double doublex2 __attribute__((ext_vector_type(2)));
+constexpr int kDenseColumns = 2;             // columns a workgroup of k_dense_level forms together
 
-// The map of a level, K columns per workgroup: `pre` damped-Jacobi sweeps from
+// The map of a level, K = 2 columns per workgroup: `pre` damped-Jacobi sweeps from
 // zero on the unit vectors, the restricted residual through the map Cc of the
 // next level (nc cells), alpha times the result prolongated, `post` sweeps.
 // Cc null: the sweeps alone (a coarsest level too large for the direct solve).
 // The vectors live in LDS, K to a 16-byte element, and the level's rows come
-// from L2 once per pass for all K (the pass is bound by those reads: one
-// FP64 column a workgroup took 314 us for 1939 cells, 4 FP32 columns 100).  After one
+// from L2 once per pass for all K, in the hierarchy's precision (the pass is
+// bound by those reads: 1939 cells 148 us; one column a workgroup from FP64 rows
+// took 314, four columns, whose LDS leaves one workgroup a CU, no less).  After one
 // sweep from zero the residual reaches only the aggregates next to the unit's
 // cell, so the coarse map is applied to the nonzero entries alone.
-template <class T, class TC>
+template <class A>
 __global__ void __launch_bounds__(kDenseThreads)
-k_dense_level(int n, int w, const int *__restrict__ nbr, const T *__restrict__ anb,
-              const T *__restrict__ ac, const int *__restrict__ parent, int nc, const int *__restrict__ mptr,
-              const int *__restrict__ mem, const TC *__restrict__ Cc, int pre, int post, T omega, T alpha,
-              T *__restrict__ C) {
-  constexpr int K = Vec16<T>::K;
-  typedef typename Vec16<T>::V V;
+k_dense_level(int n, int w, const int *__restrict__ nbr, const A *__restrict__ anb,
+              const A *__restrict__ ac, const int *__restrict__ parent, int nc, const int *__restrict__ mptr,
+              const int *__restrict__ mem, const double *__restrict__ Cc, int pre, int post, double omega,
+              double alpha, double *__restrict__ C) {
+  constexpr int K = kDenseColumns;
+  typedef double T;
+  typedef doublex2 V;
+  static_assert(sizeof(V) == K * sizeof(T), "columns of a vector element");
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   V *x = (V *)lds, *y = x + n, *rc = y + n;
   int *list = (int *)(rc + nc);
@@ -1031,19 +1035,9 @@ k_dense_level(int n, int w, const int *__restrict__ nbr, const T *__restrict__ a
     __syncthreads();
     const int cnt = s_cnt;
     for (int p = threadIdx.x; p < nc; p += kDenseThreads) {
-      TC s[K];
-#pragma unroll
-      for (int k = 0; k < K; ++k) s[k] = TC(0);
-      for (int q = 0; q < cnt; ++q) {
-        const TC c = Cc[dense_at(p, list[q], nc)];
-        const V r = rc[list[q]];
-#pragma unroll
-        for (int k = 0; k < K; ++k) s[k] += c * (TC)r[k];
-      }
-      V o;
-#pragma unroll
-      for (int k = 0; k < K; ++k) o[k] = (T)s[k];
-      y[p] = o; // the residuals are summed: y is free
+      V s = T(0);
+      for (int q = 0; q < cnt; ++q) s = s + Cc[dense_at(p, list[q], nc)] * rc[list[q]];
+      y[p] = s; // the residuals are summed: y is free
     }
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += kDenseThreads) x[i] = x[i] + alpha * y[parent[i]];
@@ -1066,10 +1060,10 @@ k_dense_level(int n, int w, const int *__restrict__ nbr, const T *__restrict__ a
 // fixed order.
 template <class T, bool ACC, bool SC>
 __global__ void __launch_bounds__(kDenseThreads)
-k_dense_apply(int n, const T *__restrict__ C, const T *__restrict__ b, T *__restrict__ x,
+k_dense_apply(int n, const double *__restrict__ C, const T *__restrict__ b, T *__restrict__ x,
               const int *__restrict__ parent, Scatter<T> sc, const int *__restrict__ flags) {
-  constexpr int K = Vec16<T>::K, LPC = kDenseRows / K, W = kDenseThreads / 64, B = 8; // lanes per column
-  typedef typename Vec16<T>::V V;
+  constexpr int K = 2, LPC = kDenseRows / K, W = kDenseThreads / 64, B = 8; // lanes per column
+  typedef doublex2 V;
   __shared__ double part[W][kDenseRows];
   __shared__ T xs[kDenseRows];
   const int i0 = blockIdx.x * kDenseRows, cnt = n * LPC; // 16-byte elements of the strip
@@ -1099,7 +1093,7 @@ k_dense_apply(int n, const T *__restrict__ C, const T *__restrict__ b, T *__rest
     for (int u = 0; u < B; ++u)
       if (e0 + u * kDenseThreads < cnt)
 #pragma unroll
-        for (int k = 0; k < K; ++k) acc[k] += (double)c[u][k] * (double)v[u];
+        for (int k = 0; k < K; ++k) acc[k] += c[u][k] * (double)v[u];
   };
   if (SC) mp = parent[mf] - i0, mx = sc.x[mf];
   add(threadIdx.x);
@@ -1230,10 +1224,7 @@ struct DLevel {
   DevBuf<int> csr_rp, csr_col, csr_pos;
   DevBuf<double> val64;
   DevBuf<float> val32;
-  // small levels: the dense map of the cycle from this level down, in the
-  // hierarchy's precision (the direct solve of a coarsest level always FP64)
-  DevBuf<double> dense64;
-  DevBuf<float> dense32;
+  DevBuf<double> dense; // small levels: the map of the cycle from this level down
   // large levels: sliced ELL instead (val64/val32 then hold the sliced
   // layout and csr_pos points into it)
   bool sell = false, sell16 = false; // sell16: sell_col as 16-bit offsets (k_sweep_sell)
@@ -1289,7 +1280,7 @@ static void build_sell(int n, bool even, const std::vector<int> &rp, const std::
 
 // The levels whose cycle is held as a dense map (k_dense_level), for one
 // precision of the hierarchy.  ts: the first level of at most mg_tail_cells
-// cells (and whose map fits kDenseBytes), the bottom of the cycle pattern;
+// cells (and at most dense_max()), the bottom of the cycle pattern;
 // levels when there is none.  dl: the level the map is applied on, ts or the
 // level above it when that one's map fits as well.
 struct DenseTail {
@@ -1470,7 +1461,7 @@ static int coarsest_sweeps(const fs_mesh *m) { return std::max(m->mg_coarse_swee
 // The dense maps of the small levels, from the coarsest up to the one applied.
 static void build_dense(fs_mesh *m, Hierarchy &H, double alpha) {
   hipStream_t s = m->stream;
-  const int nl = (int)H.lev.size(), most = dense_max(H.fp32 ? 4 : 8);
+  const int nl = (int)H.lev.size(), most = dense_max(H.fp32);
   DenseTail &dt = H.tail;
   dt.ts = nl;
   for (int l = 1; l < nl; ++l)
@@ -1484,42 +1475,30 @@ static void build_dense(fs_mesh *m, Hierarchy &H, double alpha) {
     const DLevel &U = H.lev[dt.ts - 1];
     if (U.n <= most && !U.sell && !use_gs(m, U)) dt.dl = dt.ts - 1;
   }
-  const bool f32 = H.fp32;
   for (int l = nl - 1; l >= dt.dl; --l) {
     DLevel &D = H.lev[l];
-    const size_t size = dense_size(D.n);
-    const bool last = l == nl - 1, direct = last && D.n <= kDirectMax;
-    if (direct || !f32) D.dense64.alloc(size);
-    if (f32 && (!direct || l == dt.dl)) D.dense32.alloc(size);
-    if (direct) {
+    D.dense.alloc(dense_size(D.n));
+    const bool last = l == nl - 1;
+    if (last && D.n <= kDirectMax) {
       hipLaunchKernelGGL(k_coarse_inverse, dim3(1), dim3(kInvThreads), 0, s, D.n, D.w, D.nbr, D.ac64, D.anb64,
-                         D.dense64.p);
-      if (f32 && l == dt.dl)
-        hipLaunchKernelGGL(k_to<float>, dim3(gfor((int)size)), dim3(kBlock), 0, s, (int)size,
-                           (const double *)D.dense64.p, D.dense32.p);
+                         D.dense.p);
       continue;
     }
     DLevel *U = last ? nullptr : &H.lev[l + 1];
-    const bool below64 = !f32 || (!last && l + 1 == nl - 1 && U->n <= kDirectMax); // the type of the map below
     const int nc = last ? 0 : U->n, pre = last ? coarsest_sweeps(m) : coarse_pre(m), post = last ? 0 : coarse_post(m);
-    const size_t lds = 16 * (2 * (size_t)D.n + nc) + sizeof(int) * (size_t)nc;
-    auto level = [&](auto kernel, const auto *anb, const auto *ac, const auto *Cc, auto *C) {
+    const size_t lds = sizeof(doublex2) * (2 * (size_t)D.n + nc) + sizeof(int) * (size_t)nc;
+    const auto form = [&](auto kernel, const auto *anb, const auto *ac) {
       // the largest maps ask for more than the default dynamic LDS window
-      typedef std::decay_t<decltype(*C)> T;
       if (lds > 64 * 1024)
         FS_HIP_THROW(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-      constexpr int K = Vec16<T>::K;
-      hipLaunchKernelGGL(kernel, dim3((D.n + K - 1) / K), dim3(kDenseThreads), (unsigned)lds, s, D.n, D.w, D.nbr,
-                         anb, ac, D.parent.p, nc, last ? nullptr : U->mptr.p, last ? nullptr : U->mem.p,
-                         Cc, pre, post, (T)m->mg_omega, (T)alpha, C);
+      hipLaunchKernelGGL(kernel, dim3((D.n + kDenseColumns - 1) / kDenseColumns), dim3(kDenseThreads), (unsigned)lds, s,
+                         D.n, D.w, D.nbr, anb, ac, D.parent.p, nc, last ? nullptr : U->mptr.p,
+                         last ? nullptr : U->mem.p, last ? nullptr : (const double *)U->dense.p, pre, post,
+                         m->mg_omega, alpha, D.dense.p);
       FS_HIP_THROW(hipGetLastError()); // a refused launch (LDS request) must not pass silently
     };
-    const double *c64 = last ? nullptr : U->dense64.p;
-    const float *c32 = last ? nullptr : U->dense32.p;
-    if (!f32) level(k_dense_level<double, double>, D.anb64, D.ac64, c64, D.dense64.p);
-    else if (below64)
-      level(k_dense_level<float, double>, (const float *)D.anb32.p, (const float *)D.ac32.p, c64, D.dense32.p);
-    else level(k_dense_level<float, float>, (const float *)D.anb32.p, (const float *)D.ac32.p, c32, D.dense32.p);
+    if (H.fp32) form(k_dense_level<float>, (const float *)D.anb32.p, (const float *)D.ac32.p);
+    else form(k_dense_level<double>, (const double *)D.anb64, (const double *)D.ac64);
   }
 }
 
@@ -1562,7 +1541,6 @@ template <class T> struct LV {
   static const T *ac(DLevel &d);
   static const T *anb(DLevel &d);
   static const T *val(DLevel &d);
-  static const T *dense(DLevel &d);
 };
 template <> struct LV<double> {
   static double *x(DLevel &d) { return d.x64.p; }
@@ -1572,7 +1550,6 @@ template <> struct LV<double> {
   static const double *ac(DLevel &d) { return d.ac64; }
   static const double *anb(DLevel &d) { return d.anb64; }
   static const double *val(DLevel &d) { return d.val64.p; }
-  static const double *dense(DLevel &d) { return d.dense64.p; }
 };
 template <> struct LV<float> {
   static float *x(DLevel &d) { return d.x32.p; }
@@ -1582,7 +1559,6 @@ template <> struct LV<float> {
   static const float *ac(DLevel &d) { return d.ac32.p; }
   static const float *anb(DLevel &d) { return d.anb32.p; }
   static const float *val(DLevel &d) { return d.val32.p; }
-  static const float *dense(DLevel &d) { return d.dense32.p; }
 };
 
 // lanes per row of a coarse level's CSR kernels by its mean row length
@@ -1843,7 +1819,7 @@ static void vcycle(fs_mesh *m, const double *rhs, double *out, double alpha, con
     const Scatter<T> sc{D.mptr.p, D.mem.p, up ? res[dl - 1] : nullptr, al};
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3((D.n + kDenseRows - 1) / kDenseRows), dim3(kDenseThreads), 0, s, D.n,
-                         LV<T>::dense(D), b, LV<T>::x(D), F.parent.p, sc, flags);
+                         (const double *)D.dense.p, b, LV<T>::x(D), F.parent.p, sc, flags);
     };
     if (acc) {
       if (up) go(k_dense_apply<T, true, true>);

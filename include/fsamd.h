@@ -77,10 +77,10 @@ enum fs_option {
                                  is known to have ended, 2 = one ahead, more =
                                  two ahead [8]                                 */
   FS_OPT_MG_TAIL_CELLS = 12,  /* from the first level with at most this many
-                                 cells down (at most 2048 cells in FP32, 1448
-                                 in FP64) the cycle is formed as one dense map
-                                 and counts as one level; 0 = no such level
-                                 [1024]                                        */
+                                 cells down (at most 2048 cells with MG_FP32,
+                                 1448 without) the cycle is formed as one dense
+                                 map in FP64 and counts as one level; 0 = no
+                                 such level [1024]                             */
   FS_OPT_MG_COARSE_SWEEPS = 13,/* smoothing sweeps on a coarsest level too large
                                  for the direct FP64 solve (> 64 cells) [16]   */
   FS_OPT_MG_ALPHA = 14,       /* over-correction of the prolongated coarse

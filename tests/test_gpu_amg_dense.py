@@ -111,7 +111,7 @@ def run(system, opts):
 
 
 # cells: one or two small levels; the level above the tail small enough for a
-# dense map of its own (dl = ts - 1) or not; odd sizes off the 16-row tiles
+# dense map of its own (dl = ts - 1) or not; odd sizes off the strips of 8 rows
 @pytest.mark.parametrize("shape", [(5, 4, 3), (13, 11, 9), (32, 24, 20), (41, 37, 1)])
 @pytest.mark.parametrize("opts", [
     {}, {"mg_fp32": 1}, {"mg_presweep": 1, "mg_postsweep": 1}, {"mg_presweep": 1, "mg_postsweep": 2, "mg_fp32": 1},
@@ -132,6 +132,27 @@ def test_one_cycle_is_numpys(shape, opts, shift):
     want = full_cycle(levels, len(levels) - 1 if ts is None else ts, system[4], opts, cs if ts is None else -cs)
     scale = np.abs(want).max()
     np.testing.assert_allclose(dphi, want, rtol=0, atol=(1e-4 if opts.get("mg_fp32") else 1e-11) * scale)
+
+
+@pytest.mark.parametrize("shape", [(5, 4, 3), (13, 11, 9), (32, 24, 20), (41, 37, 1)])
+@pytest.mark.parametrize("fp32", [0, 1])
+def test_coarsest_solve_is_fp64(shape, fp32):
+    """A nearly singular operator (row sums 4e-9 of the diagonal: above the line
+    at which the coarsest is taken as singular).  Its coarsest inverse is a
+    constant of size 1e5 to 1e6 in every entry, which a source without mean
+    cancels, plus the part that corrects; held in FP32 the constant's rounding
+    (6e-8 of it) would be 1 to 10 % of that part.  Constants apart, an FP32
+    cycle is the FP64 one to FP32's own rounding."""
+    nbr, nnbr, ac, anb, bc = systems.pressure_like(*shape, 7, shift=3e-8)
+    bc = bc - bc.mean()
+    opts = {"mg_fp32": fp32}
+    dphi, levels = run((nbr, nnbr, ac, anb, bc), opts)
+    ts = next(l for l in range(1, len(levels)) if levels[l].n <= 1024)
+    want = full_cycle(levels, ts, bc, opts, -16)
+    d, w = dphi - dphi.mean(), want - want.mean()
+    # FP64: 1e-16 times the constant's 1e6 and the condition of the rest; FP32:
+    # the module's bound for its sweeps
+    assert np.abs(d - w).max() <= (1e-4 if fp32 else 1e-8) * np.abs(w).max()
 
 
 def full_cycle(levels, ts, bc, opts, cs):
