@@ -38,7 +38,7 @@ void kernel_clock_release(fs_mesh *m);
 int mesh_prepare_solver(fs_mesh *m);
 void mesh_release_solver(fs_mesh *m);
 void greedy_colors(int n, int w, const int *nbr0, std::vector<int> &ptr, std::vector<int> &cells);
-void add_inplace(fs_mesh *m, double *a, const double *b);
+void add_inplace(fs_mesh *m, double *a, double *b);
 // Runs body and the convergence update from the np L1 partials it leaves
 // (iteration count, done) until done, at most itmax times.
 void run_cycles(fs_mesh *m, int np, int itmax, const std::function<void()> &body);

@@ -10,7 +10,8 @@
 //
 // Reductions are deterministic: each block reduces with wavefront shuffles in
 // a fixed order into its own partial, and a one-block kernel combines the
-// partials in index order.  A thread takes one row: grids that stopped at
+// partials in index order.  A thread takes one row (four of a large system in
+// the kernels that only sum): grids that stopped at
 // 8192 workgroups gave some threads of 2.9 M tetrahedra two rows and others
 // one, and k_spmv_dot took 66 us instead of 49.  Per
 // cell, every sum is formed in the reference's slot order, so a sweep,
@@ -44,7 +45,8 @@ enum Slot {
   S_RES_RMS, S_RES_SCALED, S_ACPHI, S_GAMMA, S_NSLOTS
 };
 enum Flag {
-  F_DONE = 0, F_ITER = 1, F_ITMAX = 2, F_REJECT = 3, F_INNER = 4, F_GATE = 5,
+  F_DONE = 0, F_ITER = 1, F_ITMAX = 2, F_INNER = 4, F_GATE = 5,
+  F_REJECT = 3,  // the initial guess, at the end the iterate, is dropped for zero
   F_BAD = 6,     // the input was refused: 2 = a non-finite ac or bc, 1 = a diagonal <= 0
                  // for a solver that divides by it
   F_NEEDPOS = 7, // set by the host when the solver divides by the diagonal
@@ -76,9 +78,10 @@ static inline int grid_for(int n) { return xcd_grid(n); }
 static inline int grid_red(int n) { return std::min(kPartials, xcd_grid(n)); }
 // Kernels that only sum take four rows per thread, their loads first, from a
 // million rows on: the reduction of a workgroup costs as much as its loads
-// otherwise (2.9 M rows, one row against four: k_dot 15.4 and 9.0 us,
-// k_init_norms 36 and 17).  Below, a launch is latency and the sums keep the
-// grouping of one row per thread.
+// otherwise.  k_dot, one row against four, 125000 rows 2.80 and 3.08 us, 343000
+// 3.40 and 3.44, 512000 3.84 and 3.80, 729000 4.52 and 4.32, 2.9 M 15.4 and 9.0;
+// k_init_norms at 2.9 M 36 and 17.  The line lies past the tie, where a solve
+// shows the gain (673000 cells of flow 0.5 % in noise of 0.9, 2.9 M rows 4 %).
 constexpr int kSumRows = 4, kSumRowsFrom = 1000000;
 static inline int sum_rows(int n) { return n >= kSumRowsFrom ? kSumRows : 1; }
 static inline int grid_sum(int n) { return grid_red((n + sum_rows(n) - 1) / sum_rows(n)); }
@@ -909,7 +912,7 @@ enum FinOp {
   FIN_BICG_RHO,       // rho, beta
   FIN_BICG_ALPHA,     // alpha = rho/(r0,v)
   FIN_BICG_OMEGA,     // omega = (t,s)/(t,t)
-  FIN_TRUE_RES,       // fres only
+  FIN_TRUE_RES,       // fres, and whether the iterate is dropped
   FIN_CG_RHO,         // rz = (r,z), beta
   FIN_CG_ALPHA,       // alpha = rz/(p,q)
   FIN_WARM,           // reject an initial guess whose L1 residual exceeds ires
@@ -924,7 +927,17 @@ struct SolveStart {
   double rrf;
   int itmax, itmax0; // of the loop; itmax0 < 1: done before it starts
   int needpos;       // the solver divides by the diagonal
+  int drop;          // a diverged iterate is dropped at the end (FIN_TRUE_RES)
 };
+// A Krylov iterate whose true residual ends this many times above |bc|_1, that
+// of the zero start, has diverged and is dropped.  A converged flow asks for
+// that all the time: its singular p' system has round-off for a source, part of
+// it outside the range, so the stop rule cannot be met and BiCGSTAB, CG and
+// GMRES run to itmax, in every other solve to a residual above the first one,
+// now and then 1e13 times.  Taken as a correction such an iterate threw a flow
+// converged to 1e-15 back by up to 0.4, on an occasion that any change in the
+// order of a sum moves.
+constexpr double kDiverged = 100.0;
 struct Post {
   SolveBox *box;
   unsigned seq;
@@ -1107,9 +1120,12 @@ __global__ void __launch_bounds__(BS) k_fin(int op, int np, int n, int nf, const
     scal[S_TT] = b;
     scal[S_OMEGA] = (b != 0.0) ? a / b : 0.0;
     break;
-  case FIN_TRUE_RES:
-    scal[S_FRES] = a;
+  case FIN_TRUE_RES: {
+    const bool drop = st.drop && a > kDiverged * in.ires;
+    flags[F_REJECT] = drop;
+    scal[S_FRES] = drop ? in.ires : a;
     break;
+  }
   case FIN_POST:
     break;
   case FIN_CG_RHO: {
@@ -2064,7 +2080,7 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   }
   // Gauss-Seidel, D-ILU (also PBCG's preconditioner) and every multigrid
   // smoother divide by the diagonal
-  SolveStart start{rrf, lmg == FS_MG_SOLVER ? m->mg_maxcycles : itmax, itmax, 0};
+  SolveStart start{rrf, lmg == FS_MG_SOLVER ? m->mg_maxcycles : itmax, itmax, 0, 0};
   start.needpos = (lmg != FS_MG_OFF || solver == FS_SOR || solver == FS_ILU || solver == FS_PBCG) ? 1 : 0;
   ++m->seq;
   hipLaunchKernelGGL(sum_rows(n) == 1 ? k_init_norms<1> : k_init_norms<kSumRows>, dim3(gs), dim3(kBlock), 0, s, n, ac, bc, fit, part);
@@ -2302,7 +2318,8 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   const bool ends_true = lmg != FS_MG_SOLVER && (solver == FS_SOR || solver == FS_ILU || solver == FS_PBCG) && !warm;
   if (!ends_true) {
     hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, nullptr);
-    fin(m, FIN_TRUE_RES, gr, nf);
+    start.drop = lmg != FS_MG_SOLVER && (solver == FS_BICGS || solver == FS_CG || solver == FS_GMRES);
+    fin(m, FIN_TRUE_RES, gr, nf, start);
   }
   if (!one) {
     add_inplace(m, fit, dphi);
@@ -2339,11 +2356,13 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   return converged ? 0 : 1;
 }
 
-// fit += dphi, unless the input was refused
-__global__ void k_add(int n, double *__restrict__ a, const double *__restrict__ b, const int *__restrict__ flags) {
+// fit += dphi, unless the input was refused; a dropped dphi becomes zero
+__global__ void k_add(int n, double *__restrict__ a, double *__restrict__ b, const int *__restrict__ flags) {
   if (flags[F_BAD]) return;
   const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) a[i] = a[i] + b[i];
+  if (i >= n) return;
+  if (flags[F_REJECT]) b[i] = 0.0;
+  else a[i] = a[i] + b[i];
 }
 
 void run_cycles(fs_mesh *m, int np, int itmax, const std::function<void()> &body) {
@@ -2353,7 +2372,7 @@ void run_cycles(fs_mesh *m, int np, int itmax, const std::function<void()> &body
   });
 }
 
-void add_inplace(fs_mesh *m, double *a, const double *b) {
+void add_inplace(fs_mesh *m, double *a, double *b) {
   hipLaunchKernelGGL(k_add, dim3(grid_for(m->n)), dim3(kBlock), 0, m->stream, m->n, a, b, m->wk.flags);
 }
 

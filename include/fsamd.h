@@ -149,7 +149,11 @@ int fs_set_option(fs_mesh *mesh, int key, double value);
  * nf is the GetNFfromVariable code (AssignNFvaluesToVariables.for:4; 4 = p').
  * On return fit += dphi, dphi holds the correction, res4 = ResorAbs, ResorMax,
  * ResorRMS, ResorScaled of the initial residual (CalculateResidualsRoutine.for
- * :19-67).  Host arrays; copies in and out over PCIe. */
+ * :19-67).  Host arrays; copies in and out over PCIe.
+ * BICGS, CG and GMRES (no counterparts of the reference's own solvers) return
+ * dphi = 0 and 1 where they diverged: where the true residual ends more than
+ * 100 times above |bc|_1, as on a singular system whose source lies outside
+ * the range. */
 int fs_solve_equation(fs_mesh *mesh, int nf, double *fit, double rrf,
                       int itmax, int solver, int lmultigrid, const double *ac,
                       const double *anb, const double *bc, double *dphi,

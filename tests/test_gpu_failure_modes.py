@@ -150,3 +150,26 @@ def test_converged_guess_meets_the_stop_rule_at_once(solver, lmg):
     # the residual norms and the stop rule are those of the zero start
     np.testing.assert_allclose(st2["initial_l1"], np.abs(bc).sum(), rtol=1e-13)
     assert st2["final_l1"] <= 1e-8 * st2["initial_l1"]
+
+
+@pytest.mark.parametrize("solver,lmg", [("bicgs", 0), ("bicgs", 2), ("cg", 0), ("cg", 2), ("gmres", 0), ("gmres", 2)])
+def test_a_diverged_krylov_iterate_is_dropped(solver, lmg):
+    """A singular system whose source lies outside the range has no solution:
+    the Krylov solvers run to itmax and may end far above the residual they
+    started with.  What they return is never more than 100 times worse than
+    zero, and what they report is the residual of what they return."""
+    nbr, nnbr, ac, anb, _ = systems.pressure_like(8, 7, 6, 7, shift=0.0)
+    A = systems.sparse(nbr, nnbr, ac, anb)
+    m = fs.Mesh(nbr, nnbr)
+    fit0 = np.linspace(0.0, 1.0, len(ac))
+    dropped = 0
+    for seed in range(30):
+        bc = 1e-15 * np.random.default_rng(seed).standard_normal(len(ac))
+        rc, fit, dphi, res4, st = m.solve_equation("pressc", fit0, 1e-8, 300, solver, lmg, ac, anb, bc)
+        r1 = np.abs(bc - A @ dphi).sum()
+        assert rc == 1 and r1 <= 101 * np.abs(bc).sum(), (seed, r1 / np.abs(bc).sum())
+        # (what dphi leaves is a difference of terms as large as |A| |dphi|)
+        np.testing.assert_allclose(st["final_l1"], r1, rtol=1e-9, atol=1e-15 * (abs(A) @ np.abs(dphi)).sum())
+        assert np.array_equal(fit, fit0 + dphi)
+        dropped += not dphi.any()
+    print(solver, lmg, "dropped", dropped)

@@ -50,6 +50,23 @@ def test_converged_fields_match_the_reference_run(name, iters, fp32):
         assert np.abs(a - b).max() <= 1e-6 * max(np.abs(b).max(), 1e-12), (k, np.abs(a - b).max())
 
 
+def test_a_converged_flow_stays_converged():
+    """From 400 iterations on every further one leaves the fields within 1e-9
+    of the reference's: their p' systems hold round-off alone, and a Krylov
+    iterate that diverges on one is no correction."""
+    g = golden("simple_hex_converged.npz")
+    pm, bu, bv, bw, _ = msg.build_mesh(msg.SIMPLE["hex_converged"][0])
+    dc = fs.Case(pm, bu, bv, bw, rho=1.0, mu=0.01)
+    dc.configure(urf_u=0.7, urf_p=0.3, msolver="sor", mrrf=0.1, mitmax=10, psolver="bicgs", prrf=1e-8, pitmax=300,
+                 plmg=fs.MG_PRECOND)
+    dc.iterate(400)
+    for it in range(401, 601):
+        dc.iterate(1)
+        for k in ("u", "v", "w", "p"):
+            d = np.abs(dc.get(k) - g[k]).max()
+            assert d <= 1e-9 * np.abs(g[k]).max(), (it, k, d)
+
+
 def test_simplec_phases_bitwise():
     """SIMPLEC's D2 = V/(a_P + sum anb) on the device, and the p' system it
     shapes, bitwise the oracle's (which is bitwise the reference's)."""
