@@ -2316,16 +2316,24 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   // true final residual, fit += dphi (:180).  The sweeps, ILU and PBCG end on
   // the true residual of the same dphi: formed again it would be the same bits.
   const bool ends_true = lmg != FS_MG_SOLVER && (solver == FS_SOR || solver == FS_ILU || solver == FS_PBCG) && !warm;
-  if (!ends_true) {
+  start.drop = lmg != FS_MG_SOLVER && (solver == FS_BICGS || solver == FS_CG || solver == FS_GMRES);
+  const auto true_residual = [&]() {
     hipLaunchKernelGGL(k_resid_l1, dim3(gr), dim3(kBlock), 0, s, n, w, nb, ac, anb, bc, dphi, part, nullptr);
-    start.drop = lmg != FS_MG_SOLVER && (solver == FS_BICGS || solver == FS_CG || solver == FS_GMRES);
     fin(m, FIN_TRUE_RES, gr, nf, start);
-  }
+  };
+  if (!ends_true) true_residual();
   if (!one) {
     add_inplace(m, fit, dphi);
     fin(m, FIN_POST, 0, nf);
   }
-  const unsigned long long last = box_wait_final(m);
+  unsigned long long last = box_wait_final(m);
+  if (ends_true && box_iterations(last) == 0 && !box_bad(last)) {
+    // nothing was iterated, so nothing has looked at anb yet
+    ++m->seq;
+    true_residual();
+    fin(m, FIN_POST, 0, nf);
+    last = box_wait_final(m);
+  }
   // for the caller's own streams and copies: everything above is complete
   if (sync) FS_HIP(hipStreamSynchronize(s));
   if (box_bad(last)) {

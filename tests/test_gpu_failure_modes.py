@@ -173,3 +173,23 @@ def test_a_diverged_krylov_iterate_is_dropped(solver, lmg):
         assert np.array_equal(fit, fit0 + dphi)
         dropped += not dphi.any()
     print(solver, lmg, "dropped", dropped)
+
+
+@pytest.mark.parametrize("solver,lmg", [("sor", 0), ("ilu", 0), ("pbcg", 0), ("bicgs", 0), ("cg", 2), ("sor", 1)])
+@pytest.mark.parametrize("shape", [(9, 8, 7), (20, 16, 15)])
+def test_nan_off_the_diagonal_without_an_iteration(solver, lmg, shape):
+    """A source of zero, or no iterations allowed, ends a solve before its
+    first iteration; a NaN coefficient is an error there too."""
+    nbr, nnbr, ac, anb, bc = systems.pressure_like(*shape, 9, shift=0.1)
+    m = fs.Mesh(nbr, nnbr)
+    fit = np.zeros(len(ac))
+    for b, itmax in ((np.zeros_like(bc), 20), (bc, 0)):
+        rc, f, dphi, res4, st = m.solve_equation("pressc", fit, 1e-6, itmax, solver, lmg, ac, anb, b)
+        assert st["iterations"] == 0 and not dphi.any() and st["final_l1"] == st["initial_l1"]
+        assert rc == (1 if b.any() else 0)
+    bad = anb.copy()
+    bad[np.nonzero(nbr[:, 11])[0][0], 11] = np.nan
+    for b, itmax in ((np.zeros_like(bc), 20), (bc, 0)):
+        with pytest.raises(fs.FsError) as e:
+            m.solve_equation("pressc", fit, 1e-6, itmax, solver, lmg, ac, bad, b)
+        assert "(-4)" in str(e.value)
