@@ -692,7 +692,7 @@ def main():
         return {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBPS, "traffic": None, "kernel": kernel,
                 "bytes_per_launch": c["bytes"], "bytes_per_cell": per_cell, "avg_ms": c["avg_ms"],
-                "launches": c["launches"], "idle_launches": c["untimed"], "sampled_every": args.clock_stride,
+                "launches": c["launches"], "untimed_launches": c["untimed"], "sampled_every": args.clock_stride,
                 "share_of_step": c["launches"] * c["avg_ms"] * 1e-3 / el}
 
     roof_spmv = roof(clk["spmv"], "k_spmv_dot (FP64 ELL y=A*x with (r0,y) partials, BiCGSTAB loop)",

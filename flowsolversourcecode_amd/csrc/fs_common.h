@@ -98,20 +98,24 @@ struct SolveBox {
 };
 
 // Per-launch HIP-event timing of one kernel site of the solve loops: events
-// are recorded by the dispatch itself (hipExtLaunchKernelGGL), tagged with
-// the Krylov iteration that launched them, so launches after convergence
-// (which return at once) can be told from the ones that did the work.
+// are recorded by the dispatch itself (hipExtLaunchKernelGGL).  How many
+// iterations past the last one were launched (they return at once) is a matter
+// of the host's timing, so a solve ends by setting the counts back to where
+// they stood before those: what is counted did its work, and is the same
+// every time.
 struct KernelClock {
-  int sites = 0, cap = 0, used = 0;  // sites: bit (1 << site) per armed site
-  int dropped[4] = {0, 0, 0, 0};
-  int stride = 1;                    // time every stride-th launch of a site
-  long long seen[4] = {0, 0, 0, 0};  // launches of each site since the start
-  int cur_iter = -1;       // Krylov iteration being launched, -1 outside a loop
-  int solve_first = 0;     // first record of the solve in progress
+  struct Counts {
+    int used = 0;                      // records
+    int dropped[4] = {0, 0, 0, 0};     // launches beyond the capacity
+    long long seen[4] = {0, 0, 0, 0};  // launches of each site since the start
+  };
+  int sites = 0, cap = 0;  // sites: bit (1 << site) per armed site
+  int stride = 1;          // time every stride-th launch of a site
+  Counts c;
+  std::vector<Counts> before;  // the counts before each iteration of the solve in progress
   std::vector<hipEvent_t> ev;  // 2 per record
-  std::vector<int> iter, site;
+  std::vector<int> site;
   std::vector<double> bytes;
-  std::vector<char> live;
 };
 
 } // namespace fs

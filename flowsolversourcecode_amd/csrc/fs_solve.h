@@ -15,17 +15,15 @@ template <class K, class... A>
 void timed_launch(fs_mesh *m, int site, double bytes, K kernel, dim3 grid, dim3 block, unsigned lds,
                   hipStream_t s, A... args) {
   KernelClock &c = m->kclock;
-  if (site != 0 && (c.sites >> site & 1) && c.seen[site & 3]++ % c.stride == 0) {
-    if (c.used < c.cap) {
-      const int u = c.used++;
-      c.iter[u] = c.cur_iter;
+  if (site != 0 && (c.sites >> site & 1) && c.c.seen[site & 3]++ % c.stride == 0) {
+    if (c.c.used < c.cap) {
+      const int u = c.c.used++;
       c.site[u] = site;
       c.bytes[u] = bytes;
-      c.live[u] = 1;
       hipExtLaunchKernelGGL(kernel, grid, block, lds, s, c.ev[2 * u], c.ev[2 * u + 1], 0u, args...);
       return;
     }
-    c.dropped[site & 3]++;
+    c.c.dropped[site & 3]++;
   }
   hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);
 }

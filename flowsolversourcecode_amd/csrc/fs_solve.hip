@@ -1707,14 +1707,9 @@ int kernel_clock_start(fs_mesh *m, int site_mask, int capacity) {
   }
   c.sites = site_mask;
   c.cap = capacity;
-  c.used = 0;
-  for (int &d : c.dropped) d = 0;
-  for (long long &k : c.seen) k = 0;
-  c.solve_first = 0;
-  c.iter.assign(capacity, -1);
+  c.c = KernelClock::Counts{};
   c.site.assign(capacity, 0);
   c.bytes.assign(capacity, 0.0);
-  c.live.assign(capacity, 0);
   return 0;
 }
 
@@ -1725,14 +1720,10 @@ int kernel_clock_read(fs_mesh *m, int site, double *out) {
     return -1;
   }
   FS_HIP(hipStreamSynchronize(m->stream));
-  long long k = 0, idle = 0;
+  long long k = 0;
   double ms = 0.0, by = 0.0;
-  for (int u = 0; u < c.used; ++u) {
+  for (int u = 0; u < c.c.used; ++u) {
     if (c.site[u] != site) continue;
-    if (!c.live[u]) {
-      ++idle;
-      continue;
-    }
     float t = 0.f;
     FS_HIP(hipEventElapsedTime(&t, c.ev[2 * u], c.ev[2 * u + 1]));
     ms += t;
@@ -1742,17 +1733,14 @@ int kernel_clock_read(fs_mesh *m, int site, double *out) {
   out[0] = (double)k;
   out[1] = k ? ms / k : 0.0;
   out[2] = k ? by / k : 0.0;
-  out[3] = (double)(c.dropped[site & 3] + idle);
+  out[3] = (double)c.c.dropped[site & 3];
   return 0;
 }
 
 int kernel_clock_clear(fs_mesh *m) {
   KernelClock &c = m->kclock;
   FS_HIP(hipStreamSynchronize(m->stream));
-  c.used = 0;
-  for (int &d : c.dropped) d = 0;
-  for (long long &k : c.seen) k = 0;
-  c.solve_first = 0;
+  c.c = KernelClock::Counts{};
   return 0;
 }
 
@@ -1762,7 +1750,7 @@ int kernel_clock_stride(fs_mesh *m, int stride) {
     return -1;
   }
   m->kclock.stride = stride;
-  for (long long &k : m->kclock.seen) k = 0;
+  for (long long &k : m->kclock.c.seen) k = 0;
   return 0;
 }
 
@@ -1897,23 +1885,21 @@ unsigned long long box_wait_final(fs_mesh *m) {
 // synchronisation of about 20 us a batch and up to check_every idle iterations.
 template <class F> static void run_iterations(fs_mesh *m, int itmax, F body) {
   const int ahead = std::min(2, m->check_every - 1);
-  m->kclock.solve_first = m->kclock.used;
   for (int k = 0; k < itmax; ++k) {
     const unsigned long long w = box_wait(m, [&](unsigned long long v) {
       return (v & kBoxDone) || (v ? box_iterations(v) : -1) + ahead >= k;
     });
     if (w & kBoxDone) break;
-    m->kclock.cur_iter = k;
+    if (m->kclock.sites) m->kclock.before.push_back(m->kclock.c);
     body();
   }
-  m->kclock.cur_iter = -1;
 }
 
-// the clock's launches of iterations past the converged one returned at once
+// the launches of iterations past the converged one returned at once
 static void clock_iterations(fs_mesh *m, int iters) {
   KernelClock &c = m->kclock;
-  for (int u = c.solve_first; u < c.used; ++u)
-    if (c.iter[u] >= iters) c.live[u] = 0;
+  if (iters < (int)c.before.size()) c.c = c.before[iters];
+  c.before.clear();
 }
 
 // x0 *= (A x0, b)/(A x0, A x0): the scaling of an initial guess with the
@@ -2083,6 +2069,7 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   SolveStart start{rrf, lmg == FS_MG_SOLVER ? m->mg_maxcycles : itmax, itmax, 0, 0};
   start.needpos = (lmg != FS_MG_OFF || solver == FS_SOR || solver == FS_ILU || solver == FS_PBCG) ? 1 : 0;
   ++m->seq;
+  m->kclock.before.clear();
   hipLaunchKernelGGL(sum_rows(n) == 1 ? k_init_norms<1> : k_init_norms<kSumRows>, dim3(gs), dim3(kBlock), 0, s, n, ac, bc, fit, part);
   fin(m, FIN_INIT_NORMS, gs, nf, start);
   const bool one = solver == FS_SOR && !warm && lmg != FS_MG_SOLVER && gs_in_one(n, w, (int)sw.color_ptr.size() - 1);
@@ -2260,7 +2247,6 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     restart();
     int fl[F_NFLAGS];
     host_flags(m, fl);
-    m->kclock.solve_first = m->kclock.used;
     while (!fl[F_DONE]) {
       for (int j = 0; j < gmm; ++j) {
         const double *vj = V + (size_t)j * ldv;
@@ -2334,6 +2320,8 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     fin(m, FIN_POST, 0, nf);
     last = box_wait_final(m);
   }
+  const int iters = box_iterations(last);
+  clock_iterations(m, iters);
   // for the caller's own streams and copies: everything above is complete
   if (sync) FS_HIP(hipStreamSynchronize(s));
   if (box_bad(last)) {
@@ -2347,8 +2335,6 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     res4[2] = h_out[S_RES_RMS];
     res4[3] = h_out[S_RES_SCALED];
   }
-  const int iters = box_iterations(last);
-  clock_iterations(m, iters);
   if (st) {
     st->iterations = iters;
     st->levels = (lmg != FS_MG_OFF) ? amg_levels(m) : 1;

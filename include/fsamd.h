@@ -249,9 +249,9 @@ int fs_time_device_copy(long long bytes, int reps, double *avg_ms);
  * any timed region) and arms the sites of site_mask (bit 1 << FS_CLOCK_*; 0
  * disarms).  fs_kernel_clock_read synchronises the stream and returns for one
  * site out[0] launches that did work (launches of Krylov iterations after
- * convergence, which return at once, are left out), out[1] their mean
- * duration in ms, out[2] their mean algorithmic bytes, out[3] launches of the
- * site not timed (idle or beyond the capacity).  fs_kernel_clock_clear
+ * convergence, which return at once, are left out, also of the stride), out[1]
+ * their mean duration in ms, out[2] their mean algorithmic bytes, out[3]
+ * launches of the site beyond the capacity.  fs_kernel_clock_clear
  * empties the records; the sites stay armed.  fs_kernel_clock_stride times
  * only every stride-th launch of each site (default 1: every launch), which
  * keeps the events' own cost out of the throughput of the timed region. */
