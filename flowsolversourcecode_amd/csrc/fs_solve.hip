@@ -2070,6 +2070,7 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   start.needpos = (lmg != FS_MG_OFF || solver == FS_SOR || solver == FS_ILU || solver == FS_PBCG) ? 1 : 0;
   ++m->seq;
   m->kclock.before.clear();
+  const int ncalls_mg = m->ncalls_mg;
   hipLaunchKernelGGL(sum_rows(n) == 1 ? k_init_norms<1> : k_init_norms<kSumRows>, dim3(gs), dim3(kBlock), 0, s, n, ac, bc, fit, part);
   fin(m, FIN_INIT_NORMS, gs, nf, start);
   const bool one = solver == FS_SOR && !warm && lmg != FS_MG_SOLVER && gs_in_one(n, w, (int)sw.color_ptr.size() - 1);
@@ -2325,7 +2326,7 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
   // for the caller's own streams and copies: everything above is complete
   if (sync) FS_HIP(hipStreamSynchronize(s));
   if (box_bad(last)) {
-    if (lmg != FS_MG_OFF) m->ncalls_mg--; // a refused call does not count towards the next aggregation
+    m->ncalls_mg = ncalls_mg; // a refused call does not count towards the next aggregation
     return refuse(box_bad(last));
   }
   const double *h_out = m->box->scal;

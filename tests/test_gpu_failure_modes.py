@@ -152,6 +152,34 @@ def test_converged_guess_meets_the_stop_rule_at_once(solver, lmg):
     assert st2["final_l1"] <= 1e-8 * st2["initial_l1"]
 
 
+@pytest.mark.parametrize("refused", ["sor", "ilu", "bicgs", "cg"])
+def test_refused_calls_do_not_count_towards_aggregation(refused):
+    """The hierarchy is aggregated anew every mg_reagglomerate-th call with multigrid;
+    a refused call is none, whether or not its solver would have used it."""
+    n = (12, 10, 8)
+    nbr, nnbr, ac, anb, bc = systems.pressure_like(*n, 9, shift=0.1)
+    strong = {}
+    for name, slots in (("x", (0, 1)), ("y", (2, 3))):
+        a = anb.copy()
+        a[list(slots)] *= 50.0
+        strong[name] = (0.1 - a.sum(0), a)
+    m = fs.Mesh(nbr, nnbr)
+    m.set_option("mg_reagglomerate", 2)
+    z = np.zeros(len(ac))
+
+    def parents(name):
+        m.solve_equation("pressc", z, 1e-6, 50, "bicgs", 2, *strong[name], bc)
+        return m.amg_level(0)["parent"].copy()
+
+    first = parents("x")
+    bad = ac.copy()
+    bad[7] = 0.0
+    with pytest.raises(fs.FsError):
+        m.solve_equation("pressc", z, 1e-6, 50, refused, 2, bad, anb, bc)
+    assert np.array_equal(parents("y"), first)      # the second call: the first one's aggregates
+    assert not np.array_equal(parents("y"), first)  # the third: new ones
+
+
 @pytest.mark.parametrize("solver,lmg", [("bicgs", 0), ("bicgs", 2), ("cg", 0), ("cg", 2), ("gmres", 0), ("gmres", 2)])
 def test_a_diverged_krylov_iterate_is_dropped(solver, lmg):
     """A singular system whose source lies outside the range has no solution:
