@@ -1547,7 +1547,8 @@ struct SolveWork {
   DevBuf<int> tlin, tsrc;
   std::vector<int> color_ptr;
   DevBuf<int> color_cells;
-  DevBuf<int> gs_ints;    // the rows in colour order (GsRows), for the meshes gs_by_rows() names
+  bool gs_rows = false;   // Gauss-Seidel reads its rows in colour order (gs_by_rows()):
+  DevBuf<int> gs_ints;    // the buffers of GsRows
   DevBuf<double> gs_vals;
   GsRows gs;
   DevBuf<double> dc;
@@ -1639,6 +1640,18 @@ static void precompute_ilu_sweep(fs_mesh *m, const IluDiag &diag, IluSweep &S) {
 constexpr size_t kGsRowsSlots = 800000;
 static bool gs_by_rows(int n, int w, int colors) { return colors >= 3 && (size_t)n * w >= kGsRowsSlots; }
 
+// The buffers of a system in colour order, and its neighbours.
+static void prepare_gs_rows(fs_mesh *m, SolveWork &sw) {
+  const size_t n = m->n, w = m->w;
+  sw.gs_ints.alloc((w + 1) * n);
+  sw.gs_vals.alloc((w + 2) * n);
+  int *ip = sw.gs_ints.p;
+  double *vp = sw.gs_vals.p;
+  hipLaunchKernelGGL(k_gs_order, dim3(grid_for(m->n)), dim3(kBlock), 0, m->stream, m->n, m->w, sw.color_cells.p,
+                     m->d_nbr.p, ip, ip + n);
+  sw.gs = GsRows{ip, ip + n, vp, vp + 2 * n, vp + n};
+}
+
 int mesh_prepare_solver(fs_mesh *m) {
   auto *sw = new SolveWork();
   m->solve_work = sw;
@@ -1655,16 +1668,11 @@ int mesh_prepare_solver(fs_mesh *m) {
   greedy_colors(m->n, m->w, nbr0.data(), sw->color_ptr, cells);
   sw->color_cells.upload(cells, m->stream);
   // (a mesh numbered colour by colour is in that order as it is)
-  if (gs_by_rows(m->n, m->w, (int)sw->color_ptr.size() - 1) && !std::is_sorted(cells.begin(), cells.end())) {
-    const size_t n = m->n, w = m->w;
-    sw->gs_ints.alloc((w + 1) * n);
-    sw->gs_vals.alloc((w + 2) * n);
-    int *ip = sw->gs_ints.p;
-    double *vp = sw->gs_vals.p;
-    hipLaunchKernelGGL(k_gs_order, dim3(grid_for(m->n)), dim3(kBlock), 0, m->stream, m->n, m->w, sw->color_cells.p,
-                       m->d_nbr.p, ip, ip + n);
-    sw->gs = GsRows{ip, ip + n, vp, vp + 2 * n, vp + n};
-  }
+  sw->gs_rows = gs_by_rows(m->n, m->w, (int)sw->color_ptr.size() - 1) && !std::is_sorted(cells.begin(), cells.end());
+  // the solve without allocation may ask for the rows; a larger mesh gets them
+  // with its first Gauss-Seidel solve (a flow's pressure mesh never: 68 bytes a
+  // tetrahedron)
+  if (sw->gs_rows && m->n <= FS_NOALLOC_MAX_CELLS) prepare_gs_rows(m, *sw);
   sw->dc.alloc(m->n);
   for (auto &v : m->v) v.alloc(m->n);
   m->partial.alloc(5 * kPartials);
@@ -2145,7 +2153,8 @@ int solve_device(fs_mesh *m, int nf, double *fit, double rrf, int itmax, int sol
     // forward pass after the first at colour 1 (the residual check between
     // iterations leaves x alone).
     bool first = true;
-    const bool rows = sw.gs.pos;
+    const bool rows = sw.gs_rows;
+    if (rows && !sw.gs.pos) prepare_gs_rows(m, sw);
     if (rows) hipLaunchKernelGGL(k_gs_rows, dim3(ge), dim3(kBlock), 0, s, n, w, ac, anb, bc, sw.gs);
     const auto color = [&](int c) {
       const int b = sw.color_ptr[c], e = sw.color_ptr[c + 1];

@@ -50,3 +50,28 @@ def test_sweeps_are_numpys(n, edges, w):
         for c in list(range(nc)) + list(range(nc - 2, -1, -1)):
             sweep(nbr, ac, anb, bc, x, lists[c])
     assert np.array_equal(dphi, x), np.abs(dphi - x).max()
+
+
+def test_a_large_meshs_rows_come_with_its_first_sweep():
+    """Above FS_NOALLOC_MAX_CELLS the buffers in colour order (68 bytes a cell of
+    four slots) are not taken before a Gauss-Seidel solve asks for them."""
+    import torch
+    n, w = 600000, 4
+    i = np.arange(n)
+    nbr = np.zeros((w, n), np.int32)
+    for s, d in enumerate((-2, -1, 1, 2)):  # three colours, taking turns
+        nbr[s] = np.where((i + d >= 0) & (i + d < n), i + d + 1, 0)
+    rng = np.random.default_rng(5)
+    anb = np.where(nbr > 0, -rng.uniform(0.2, 1.0, (w, n)), 0.0)
+    ac, bc, z = 0.3 - anb.sum(0), rng.standard_normal(n), np.zeros(n)
+    m = fs.Mesh(nbr, np.full(n, w, np.int32))
+    m.solve_equation("velx", z, 1e-30, 1, "bicgs", 0, ac, anb, bc)
+    before = torch.cuda.mem_get_info()[0]
+    rc, f, dphi, res4, st = m.solve_equation("velx", z, 1e-30, 2, "sor", 0, ac, anb, bc)
+    taken = before - torch.cuda.mem_get_info()[0]
+    assert taken >= 68 * n - (4 << 20), taken  # memory is counted in pages of 2 MB
+    x = np.zeros(n)
+    for _ in range(2):
+        for c in (0, 1, 2, 1, 0):
+            sweep(nbr, ac, anb, bc, x, np.arange(c, n, 3))
+    assert np.array_equal(dphi, x), np.abs(dphi - x).max()
