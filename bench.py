@@ -296,7 +296,7 @@ def cell_heights(pm):
 
 
 def channel_case(args, fs, pm, types, pairs, tr, fp32, alpha, pre=2, post=2, omega=0.8, wd=None, agg=0,
-                 psolver="bicgs", fuse=1, maxlevels=10, cycle=0, csweeps=None):
+                 psolver="bicgs", maxlevels=10, cycle=0, csweeps=None):
     """The headline's case: SIMPLE with second-order upwind (TVD sou) and the
     min/max limiter on the velocity gradients, momentum and k, omega by
     multicolour Gauss-Seidel (rrF 0.1, <= 10 sweeps), p' BiCGSTAB + AMG to
@@ -315,8 +315,7 @@ def channel_case(args, fs, pm, types, pairs, tr, fp32, alpha, pre=2, post=2, ome
     c.set_convection("tvd", "sou")
     c.set_gradient_limiters(momentum=1)
     for key, v in (("mg_fp32", fp32), ("mg_alpha", alpha), ("mg_presweep", pre), ("mg_postsweep", post),
-                   ("mg_omega", omega), ("mg_aggregation", agg), ("mg_fuse_prolong", fuse),
-                   ("mg_maxlevels", maxlevels), ("mg_cycle", cycle)):
+                   ("mg_omega", omega), ("mg_aggregation", agg), ("mg_maxlevels", maxlevels), ("mg_cycle", cycle)):
         c.set_option(key, v)
     if csweeps is not None:
         c.set_option("mg_coarse_presweep", csweeps[0])
@@ -398,7 +397,7 @@ def channel_main(args):
     pm, types, pairs, tr = channel_mesh(dims, meshgen)
     print(f"# mesh {dims} x 6: {time.perf_counter() - t0:.1f} s", file=sys.stderr, flush=True)
     tuned = dict(alpha=args.ch_alpha, pre=args.ch_pre, post=args.ch_post, omega=args.ch_omega,
-                 agg=args.mg_aggregation, psolver=args.ch_psolver, fuse=args.ch_fuse_prolong,
+                 agg=args.mg_aggregation, psolver=args.ch_psolver,
                  maxlevels=args.ch_maxlevels, cycle=args.ch_cycle, csweeps=args.ch_coarse_sweeps)
     t0 = time.perf_counter()
     case, wd, passes = channel_case(args, fs, pm, types, pairs, tr, 1 if args.precision == "fp32amg" else 0,
@@ -534,8 +533,7 @@ def channel_main(args):
                        args.ch_warm_previous, f"projection on the last {args.ch_warm_previous} p' fields, scaled"),
                    "vcycle": {"cycle": "VFW"[args.ch_cycle], "coarse_sweeps": args.ch_coarse_sweeps,
                               "presweeps": args.ch_pre, "postsweeps": args.ch_post, "alpha": args.ch_alpha,
-                              "omega": args.ch_omega, "fused_prolongation": bool(args.ch_fuse_prolong),
-                              "max_levels": args.ch_maxlevels,
+                              "omega": args.ch_omega, "max_levels": args.ch_maxlevels,
                               "aggregation": ["reference greedy", "pairwise, 1 pass",
                                               "pairwise, 2 passes"][args.mg_aggregation]}},
         "pc_solve_ms": 1e3 * st["pc_seconds"] / args.steps,
@@ -582,14 +580,14 @@ def main():
     # alpha 1.2 48 and 1.4 43; from alpha 1.6 the cycle stops being a usable
     # CG preconditioner (solves hit itmax), so 1.3 keeps a margin.  Among V
     # cycles CG beats BiCGSTAB (81 against 91 ms) and every tuned or pairwise
-    # variant measured; damping 0.9 and the unfused prolongation each take a
-    # further 5-6 %
+    # variant measured; damping 0.9 takes a further 5-6 %
     ap.add_argument("--ch-psolver", default="cg", choices=["cg", "bicgs", "gmres", "pbcg"])
     ap.add_argument("--ch-alpha", type=float, default=1.3)
     ap.add_argument("--ch-pre", type=int, default=1)
     ap.add_argument("--ch-post", type=int, default=1)
     ap.add_argument("--ch-omega", type=float, default=0.9)
-    ap.add_argument("--ch-fuse-prolong", type=int, default=0, choices=[0, 1])
+    ap.add_argument("--ch-fuse-prolong", type=int, default=0, choices=[0, 1],
+                    help="accepted, without effect: the prolongation is fused wherever its level is in CSR")
     # each p' solve of the headline starts from the previous iteration's p'
     # (scaled to its best multiple, dropped when worse than zero): 10.05
     # against 9.13 it/s from zero on the 7.86M-tet channel

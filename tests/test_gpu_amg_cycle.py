@@ -1,7 +1,7 @@
 """Device AMG cycle variants against what the mathematics fixes.
 
 The V-cycle's form (damped Jacobi or multicolour Gauss-Seidel smoothing,
-fused restriction/prolongation kernels, the one-workgroup LDS tail, the FP64
+fused restriction/prolongation kernels, the dense map of the small levels, the FP64
 direct solve of the coarsest level, over-correction) changes the iterates but
 not the solution: every variant must drive the true L1 residual of the system
 below 1e-8 of its initial value, and on a non-singular system reach the sparse
@@ -52,7 +52,7 @@ VARIANTS = [
     {"mg_sell_rows": 1, "mg_tail_cells": 0, "mg_fp32": 1},
     {"mg_sell_rows": 1, "mg_coarse_presweep": 0, "mg_coarse_postsweep": 2},
     {"mg_sell_rows": 0},                        # CSR on every coarse level
-    {"mg_fuse_prolong": 0},                     # prolongation as a pass of its own
+    {"mg_fuse_prolong": 0},                     # accepted, without effect
     {"mg_fuse_prolong": 0, "mg_fp32": 1, "mg_sell_rows": 1},
     {"mg_cycle": 1},                            # F cycle
     {"mg_cycle": 2, "mg_fp32": 1},              # W cycle
